@@ -6,36 +6,38 @@
 // products in fp32.  Rows are independent, so a row's result does not depend on
 // how many rows its expert has.
 //
-// Work split: a workgroup of 8 waves (two a SIMD) owns 256 weight rows of one expert
-// (down: 16 row blocks; gate||up: 8 gate blocks and the 8 up blocks of the same
-// output columns, so SwiGLU is fused) and every token of the expert's segment, in
-// chunks of up to 16 * TTS tokens.  Each wave owns 2 row blocks (gate||up: a gate
-// block and its up block).  K is walked in steps of one group pair (128 k): the wave
-// dequantizes its 2 row blocks' pair into bf16 MFMA B fragments once (one fma and
-// half a convert per weight) and uses them against every token tile of the chunk,
-// whose activations the workgroup stages in LDS (gathered through pair_row for
-// gate||up).  The next step's packed weights and activations are loaded while the
-// current step computes.  Two waves a SIMD let one wave's dequantization (vector ALU)
-// run while the other's MFMAs keep the matrix core busy.  fp32 accumulators: TTS x 2
-// tiles of 16 x 16 per wave.
+// Work split: a workgroup of WAVES waves (4 or 8) owns 32 WAVES weight rows of one expert (gate||up:
+// gate blocks and the up blocks of the same output columns, so SwiGLU is fused) and every token of
+// the expert's segment, in chunks of up to 16 * TTS tokens.  Each wave owns 2 row blocks (gate||up: a
+// gate block and its up block).  K is walked in steps of one group pair (128 k): the wave
+// dequantizes its 2 row blocks' pair into bf16 MFMA B fragments once and uses them against every
+// token tile of the chunk, whose activations the workgroup stages in LDS (gathered through pair_row
+// for gate||up).  The next steps' packed weights and activations are loaded while the current step
+// computes.  fp32 accumulators: TTS x 2 tiles of 16 x 16 per wave.
+//
+// What bounds it, and the shapes (SegShape).  Long segments are bound by issue: the dequantization
+// (vector ALU, the same for any chunk length) and the MFMAs, which two waves a SIMD overlap; 10 tiles a
+// chunk spread the dequantization over 160 tokens.  A short segment (a 512-row prompt chunk leaves 32
+// pairs an expert) is bound by the latency of its K steps -- barrier, activations, weights -- and wastes
+// what it computes past its last token: it takes a chunk of few tiles in workgroups of 4 waves and at
+// most 51 KB of LDS, three or four of them a CU, whose steps, prologues and epilogues overlap.
+// Deeper rings do not help: loads complete in order, so a wait for a step's activations also waits for
+// every weight load issued before them.  128 experts, top-8, 2048 x 768, us (gate||up + down; 10 tiles
+// at every size before -> now): 64 rows 130 + 66 -> 49 + 33, 256 rows 124 + 68 -> 60 + 34, 512 rows
+// 128 + 70 -> 75 + 42, 1,024 rows 138 + 75 -> 101 + 60, 2,108 rows 153 + 93 -> 144 + 88.
+#include <cmath>
+
 #include "qtile.hpp"
 
 namespace {
 
-constexpr int kSegWaves = 8;
 constexpr int kSegRB = 2;                 // row blocks per wave
-constexpr int kSegThreads = 64 * kSegWaves;
-constexpr int kSegRows = 16 * kSegRB * kSegWaves;  // weight rows per workgroup
-constexpr int kSegTT = 10;                // token tiles per chunk of an expert segment (160 tokens)
-// (a dense batch, one matrix with its token chunks spread over workgroups, sizes its chunks to the
-// CUs: jit_qmm_seg)
+constexpr int seg_rows(int waves) { return 16 * kSegRB * waves; }  // weight rows per workgroup
+constexpr int kSegRows = seg_rows(8);     // rows a dense matrix or a down stack is a multiple of
 #ifndef JIT_SEG_AHEAD
 #define JIT_SEG_AHEAD 1
 #endif
 constexpr int kSegAhead = JIT_SEG_AHEAD;  // token tiles whose fragment reads run ahead of the MFMAs
-#ifndef JIT_SEG_IGLP
-#define JIT_SEG_IGLP 0
-#endif
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // (HIP's uint4 is a union-based struct)
 
@@ -68,45 +70,53 @@ __device__ __forceinline__ bool seg_block(const SegArgs &a, int &g, int &cb) {
 
 inline dim3 seg_grid(int nx, int groups) { return dim3(nx * 8 * ((groups + 7) / 8)); }
 
-// 8 packed-order nibbles of a word -> 8 bf16 weights bf16(s * q + b) in natural k order.
-// The masked words pass through an empty asm so that each byte converts with one
-// v_cvt_f32_ubyteN (the compiler would otherwise extract every nibble separately), and the
-// weights are rounded in pairs (one v_cvt_pk_bf16_f32 each; s q + b is finite).
-__device__ __forceinline__ Frag8 dequant_word(uint32_t w, float s, float b) {
-  uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
-  asm volatile("" : "+v"(lo), "+v"(hi));
-  // packed order: nibble positions 0..7 hold q0 q2 q4 q6 q1 q3 q5 q7, so the bytes of
-  // lo are (q0, q4, q1, q5) and those of hi (q2, q6, q3, q7)
-  const float q0 = (float)(lo & 0xffu), q4 = (float)((lo >> 8) & 0xffu);
-  const float q1 = (float)((lo >> 16) & 0xffu), q5 = (float)(lo >> 24);
-  const float q2 = (float)(hi & 0xffu), q6 = (float)((hi >> 8) & 0xffu);
-  const float q3 = (float)((hi >> 16) & 0xffu), q7 = (float)(hi >> 24);
+// 8 packed-order nibbles of a word -> 8 bf16 weights bf16(s * q + b) in natural k order, 19 vector
+// instructions: a shift and a mask leave two nibbles in the low bits of a register's halves, where as
+// f16 denormals they are q 2^-24; v_fma_mix_f32 takes such a half as an operand, so s2 = 2^24 s (exact
+// for |s| < 2^104) times it plus b is the fp32 fma(s, q, b) in one instruction, where a byte conversion
+// and an fma were two (gate||up of 2,108 rows 147 -> 144 us, of 512 rows 78 -> 75 us; the same bits).
+// The weights are rounded in pairs (one v_cvt_pk_bf16_f32 each; s q + b is finite).
+__device__ __forceinline__ Frag8 dequant_word(uint32_t w, float s2, float b) {
   Frag8 f;
-  f.u[0] = pack_bf16x2_rne(fmaf(s, q0, b), fmaf(s, q1, b));
-  f.u[1] = pack_bf16x2_rne(fmaf(s, q2, b), fmaf(s, q3, b));
-  f.u[2] = pack_bf16x2_rne(fmaf(s, q4, b), fmaf(s, q5, b));
-  f.u[3] = pack_bf16x2_rne(fmaf(s, q6, b), fmaf(s, q7, b));
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const uint32_t u = (w >> (4 * j)) & 0x000F000Fu;  // (q[2j], q[2j + 1])
+    float lo, hi;
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(u), "v"(s2), "v"(b));
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(hi) : "v"(u), "v"(s2), "v"(b));
+    f.u[j] = pack_bf16x2_rne(lo, hi);
+  }
   return f;
 }
 
 // LDS of a workgroup:
-//   two activation stages: one K step's activations, 16 TTS token rows of 128 k (256 B, no
+//   activation stages: one K step's activations, 16 TTS token rows of 128 k (256 B, no
 //     padding).  Row r's 16 B piece c sits in slot c ^ (r % 16), so the 16 rows one fragment
 //     read touches (same piece, rows 16 t .. 16 t + 15) fall in 16 different slots: the reads
 //     are free of bank conflicts without the padding the direct global->LDS loads (1 KB = 4
 //     whole rows per wave instruction) could not insert;
-//   three weight stages: per wave its 2 row blocks' nibble tiles of one K step (2 x 1 KB) and
-//     their scale tiles (2 x 128 B, then copies of them: the instruction writes 1 KB);
-//   the chunk's activation row indices.
-// (per chunk of TTS token tiles: the expert segments take kSegTT, dense batches 5, 8 or 10, jit_qmm_seg)
-constexpr int seg_stage_bytes(int tts) { return 16 * tts * 256; }
+//   weight stages: per wave its 2 row blocks' nibble tiles of one K step (2 x 1 KB) and their scale
+//     tiles (2 x 128 B).
 constexpr int kSegWLoads = kSegRB + 1;  // direct loads of a wave's weights per K step
-constexpr int kSegWWave = kSegWLoads * 1024;
-constexpr int kSegWStageBytes = kSegWaves * kSegWWave;
-constexpr int seg_w_off(int tts) { return 2 * seg_stage_bytes(tts); }
-constexpr int seg_row_off(int tts) { return seg_w_off(tts) + 3 * kSegWStageBytes; }
-constexpr int seg_lds_bytes(int tts) { return seg_row_off(tts) + 16 * tts * (int)sizeof(int); }
-static_assert(seg_lds_bytes(kSegTT) <= 160 * 1024, "gfx950 gives a workgroup at most 160 KB of LDS");
+constexpr int kSegWWave = kSegRB * (qtile::kNibbleBytes + qtile::kScaleBytes);
+
+// A shape of the kernel: TTS token tiles a chunk, WAVES waves a workgroup, activations requested DX
+// K steps ahead and weights DW steps ahead.
+template <int TTS_, int WAVES_, int DX_, int DW_, int OCC_ = 2>
+struct SegShape {
+  static constexpr int TTS = TTS_, WAVES = WAVES_, DX = DX_, DW = DW_, OCC = OCC_;
+  static constexpr int kThreads = 64 * WAVES, kRows = seg_rows(WAVES), kTokens = 16 * TTS;
+  static constexpr int kXLoads = 4 * TTS / WAVES;  // a wave's activation loads per K step
+  static constexpr int kXStage = kTokens * 256, kWStage = WAVES * kSegWWave;
+  static constexpr int kWOff = (DX + 1) * kXStage;
+  static constexpr int kLds = kWOff + DW * kWStage;
+  // the most loads one of the kernel's waits can leave in flight
+  static constexpr int kMaxWait = (DX > DW ? DX : DW) * (kXLoads + kSegWLoads);
+  static_assert(WAVES == 4 || WAVES == 8, "a wave stages 4 rows of a token tile: 4 waves a tile");
+  static_assert(4 * TTS % WAVES == 0, "the halves of 8 waves stage alternate token tiles");
+  static_assert(DX <= DW && kMaxWait < 64, "the waits' steady counts; vmcnt is 6 bits");
+  static_assert(kLds <= 160 * 1024, "gfx950 gives a workgroup at most 160 KB of LDS");
+};
 
 // s_waitcnt vmcnt(N), nothing else.  Direct loads are counted by hand: the compiler does not see
 // the ones issued by inline assembly.
@@ -114,6 +124,21 @@ template <int N>
 __device__ __forceinline__ void seg_wait_vm() {
   static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// s_waitcnt vmcnt(n) for a count known at run time (uniform), n in [LO, HI): the instruction's count
+// is an immediate, so the value is found by bisection over scalar branches.
+template <int LO, int HI>
+__device__ __forceinline__ void seg_wait_vm_n(int n) {
+  if constexpr (HI - LO == 1) {
+    seg_wait_vm<LO>();
+  } else {
+    constexpr int MID = (LO + HI) / 2;
+    if (n >= MID)
+      seg_wait_vm_n<MID, HI>(n);
+    else
+      seg_wait_vm_n<LO, MID>(n);
+  }
 }
 
 // A workgroup barrier that waits for nothing else: every wave has already waited for its own
@@ -124,30 +149,33 @@ __device__ __forceinline__ void seg_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// (the dword form: 256 B a wave)
+__device__ __forceinline__ void seg_load_lds4(const void *src, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(dst) : "memory", "m0");
+}
+
 __device__ __forceinline__ void seg_load_lds(const void *src, uint32_t dst) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(dst) : "memory", "m0");
 }
 
 // DENSE: one dense matrix (E = 1, cnt null), one token chunk per group.
 //
-// Pipeline over the K steps p (one group pair each).  Per wave and step, TTS / 2 + 3 direct
-// loads: TTS / 2 of activations (4 rows of each of half the token tiles: waves 0-3 stage the
-// even tiles, 4-7 the odd ones) and 3 of its packed weights.
-//   top of step p: wait for step p's activations (requested at the top of step p - 1), one
-//     barrier; request step p + 1's activations into the other stage and step p + 2's weights;
+// Pipeline over the K steps p (one group pair each).  Per wave and step, 4 TTS / WAVES direct loads of
+// activations (4 rows of a token tile each; with 8 waves, waves 0-3 stage the even tiles and 4-7 the odd
+// ones) and 3 of its packed weights.
+//   top of step p: wait for step p's activations, one barrier; request step p + DX's activations and
+//     step p + DW's weights into the stages that step p - 1 has left;
 //   group 0's token tiles against B fragments dequantized during step p - 1, with the
 //     dequantization of this step's group 1 between their MFMAs;
-//   wait for step p + 1's weights (the wave's own: no barrier), then group 1's token tiles
-//     with the dequantization of step p + 1's group 0 between their MFMAs.
-// Each tile's activation fragments are read kSegAhead tiles ahead of its MFMAs.  Weights are
-// requested one and a half steps before they are dequantized, activations (mostly L2 hits:
-// an expert's column blocks run on one XCD) a step before they are read.
-template <bool SWIGLU, bool DENSE = false, int TTS = kSegTT>
-__global__ __launch_bounds__(kSegThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void seg_kernel(const SegArgs a) {
-  static_assert(TTS % 2 == 0 && TTS >= 2 * kSegRB, "the halves of the waves stage alternate token tiles");
-  constexpr int kTokens = 16 * TTS, kStage = seg_stage_bytes(TTS), kXLoads = TTS / 2;
+//   wait for step p + 1's weights (the wave's own: no barrier) and read them into registers, then group
+//     1's token tiles with the dequantization of step p + 1's group 0 between their MFMAs.
+// Each tile's activation fragments are read kSegAhead tiles ahead of its MFMAs.  (Activations are
+// mostly L2 hits: an expert's column blocks run on one XCD.)
+template <bool SWIGLU, bool DENSE, class S>
+__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::OCC, S::OCC))) void seg_kernel(const SegArgs a) {
+  constexpr int TTS = S::TTS, WAVES = S::WAVES, DX = S::DX, DW = S::DW;
+  constexpr int kTokens = S::kTokens, kStage = S::kXStage, kXLoads = S::kXLoads;
   extern __shared__ __attribute__((aligned(16))) uint8_t seg_lds[];
-  int *xrow = (int *)(seg_lds + seg_row_off(TTS));
   int grp, cb;
   if (!seg_block(a, grp, cb)) return;  // grid padding (uniform over the workgroup)
   const int e = DENSE ? 0 : grp;
@@ -164,66 +192,98 @@ __global__ __launch_bounds__(kSegThreads) __attribute__((amdgpu_waves_per_eu(2, 
   int rbk[kSegRB];
 #pragma unroll
   for (int r = 0; r < kSegRB; r++) {
-    if (SWIGLU)  // gate block 8 cb + wave, and the up block of the same columns
-      rbk[r] = (r ? a.N / 16 : 0) + cb * 8 + wave;
+    if (SWIGLU)  // gate block WAVES cb + wave, and the up block of the same columns
+      rbk[r] = (r ? a.N / 16 : 0) + cb * WAVES + wave;
     else
-      rbk[r] = cb * 16 + kSegRB * wave + r;
+      rbk[r] = kSegRB * (cb * WAVES + wave) + r;
   }
   const uint8_t *wexp = a.w + (long long)e * a.w_estride;
   const long long tile_row = (long long)GP * qtile::kTileBytes;  // bytes of one row block's tiles
   // weight staging: nibble instruction r moves row block r's tile (lane l: its 16 B piece); the
-  // scale instruction's lane l moves piece l % 8 of row block (l / 8) % 2's scale tile
+  // scale instruction's lane l moves word l % 32 of row block l / 32's scale tile
   const uint8_t *wnib = wexp + 16 * l;
-  const int rb_s = (l >> 3) & 1 ? rbk[1] : rbk[0];
-  const uint8_t *wscl = wexp + rb_s * tile_row + (long long)GP * qtile::kNibbleBytes + 16 * (l & 7);
-  const uint32_t wlds = lds0 + seg_w_off(TTS) + wave * kSegWWave;  // + stage * kSegWStageBytes
-  const uint8_t *wmine = seg_lds + seg_w_off(TTS) + wave * kSegWWave;
+  const int rb_s = l >> 5 ? rbk[1] : rbk[0];
+  const uint8_t *wscl = wexp + rb_s * tile_row + (long long)GP * qtile::kNibbleBytes + 4 * (l & 31);
+  const uint32_t wlds = lds0 + S::kWOff + wave * kSegWWave;  // + stage * kWStage
+  const uint8_t *wmine = seg_lds + S::kWOff + wave * kSegWWave;
   auto load_w = [&](int p) {
-    const uint32_t st = wlds + (p % 3) * kSegWStageBytes;
+    const uint32_t st = wlds + (p % DW) * S::kWStage;
 #pragma unroll
     for (int r = 0; r < kSegRB; r++)
       seg_load_lds(wnib + rbk[r] * tile_row + p * qtile::kNibbleBytes, __builtin_amdgcn_readfirstlane(st + r * 1024));
-    seg_load_lds(wscl + p * qtile::kScaleBytes, __builtin_amdgcn_readfirstlane(st + kSegRB * 1024));
+    seg_load_lds4(wscl + p * qtile::kScaleBytes, __builtin_amdgcn_readfirstlane(st + kSegRB * 1024));
   };
-  // B fragment h of group g, row block r, from the staged step p: bf16(s q + b) of the lane's
-  // word h of the group (the nibble tile's 16 B piece holds group 0's two words, then group 1's)
-  auto dequant_word_at = [&](int p, int g, int r, int h, Frag8 (&bw)[kSegRB][2]) {
-    const uint8_t *st = wmine + (p % 3) * kSegWStageBytes;
-    const uint32_t q = *(const uint32_t *)(st + r * 1024 + 16 * l + 8 * g + 4 * h);
-    const uint2 sb = *(const uint2 *)(st + kSegRB * 1024 + r * 128 + 8 * lr);
-    const float sc = g ? bf2f_hi(sb.x) : bf2f(sb.x & 0xffffu);
-    const float bi = g ? bf2f_hi(sb.y) : bf2f(sb.y & 0xffffu);
-    bw[r][h] = dequant_word(q, sc, bi);
+  // the lane's staged weights of step p, read into registers half a step before they are dequantized:
+  // per row block both groups' two words and the row's scale and bias pairs (each group's dequantization
+  // reading its own words would wait on the LDS 16 times a step)
+  uint4 rq[kSegRB];
+  uint2 rs[kSegRB];
+  auto fetch_w = [&](int p) {
+    const uint8_t *st = wmine + (p % DW) * S::kWStage;
+#pragma unroll
+    for (int r = 0; r < kSegRB; r++) {
+      rq[r] = *(const uint4 *)(st + r * 1024 + 16 * l);
+      rs[r] = *(const uint2 *)(st + kSegRB * 1024 + r * 128 + 8 * lr);
+    }
   };
-  auto dequant_rb = [&](int p, int g, int r, Frag8 (&bw)[kSegRB][2]) {
-    dequant_word_at(p, g, r, 0, bw);
-    dequant_word_at(p, g, r, 1, bw);
+  // B fragment h of group g, row block r: bf16(s q + b) of the lane's word h of the group (the nibble
+  // tile's 16 B piece holds group 0's two words, then group 1's)
+  auto dequant_at = [&](int g, int r, int h, Frag8 (&bw)[kSegRB][2]) {
+    const uint32_t q = g ? (h ? rq[r].w : rq[r].z) : (h ? rq[r].y : rq[r].x);
+    const float sc = g ? bf2f_hi(rs[r].x) : bf2f(rs[r].x & 0xffffu);
+    const float bi = g ? bf2f_hi(rs[r].y) : bf2f(rs[r].y & 0xffffu);
+    bw[r][h] = dequant_word(q, sc * 16777216.0f, bi);
   };
   // activation staging: the wave's instruction i moves rows 4 (wave % 4) .. + 3 (1 KB) of token
-  // tile j = 2 i + wave / 4; lane l fetches the piece its slot l % 16 holds in row 16 j + srow
+  // tile j = (WAVES / 4) i + wave / 4; lane l fetches the piece its slot l % 16 holds in row 16 j + srow
   const int srow = 4 * (wave & 3) + (l >> 4), jhalf = wave >> 2;
+  constexpr int kXTile = WAVES / 4;
   const int spiece = (l & 15) ^ srow;
   // fragment reads: lane (lr, lg) reads pieces 8 g + 2 lg and + 1 of row 16 t + lr
   const int frow = lr * 256;
 
   const int cend = DENSE ? min(cnt, (grp + 1) * kTokens) : cnt;
-  for (int c0 = DENSE ? grp * kTokens : 0; c0 < cend; c0 += kTokens) {
+  const int cfirst = DENSE ? grp * kTokens : 0;
+  for (int c0 = cfirst; c0 < cend; c0 += kTokens) {
     const int nt = min(kTokens, cnt - c0);
-    __syncthreads();  // the previous chunk's reads of the stages and of xrow are done
-    for (int j = tid; j < kTokens; j += kSegThreads) {
-      const int pos = off + c0 + min(j, nt - 1);  // rows past the segment re-read its last row
-      xrow[j] = a.row_index ? a.row_index[pos] : pos;
-    }
-    __syncthreads();
-    uint32_t xsrc[kXLoads];  // element offsets of this lane's pieces (x holds < 2^32 elements)
+    if (c0 != cfirst) __syncthreads();  // the previous chunk's reads of the stages are done
+    const int last = GP - 1;
+    // element offsets of this lane's pieces (x holds < 2^32 elements; rows past the segment re-read its
+    // last row)
+    uint32_t xsrc[kXLoads];
+    auto first_w = [&]() {
 #pragma unroll
-    for (int i = 0; i < kXLoads; i++)
-      xsrc[i] = (uint32_t)xrow[16 * (2 * i + jhalf) + srow] * (uint32_t)a.K + 8 * spiece;
+      for (int i = 0; i < DW; i++)
+        if (i <= last) load_w(i);
+    };
+    if constexpr (kXLoads <= 4) {
+      // the first weights go out before the row indices are read (they depend on the expert alone), and
+      // the rows come by scalar loads, whose wait does not wait for the weights
+      first_w();
+#pragma unroll
+      for (int i = 0; i < kXLoads; i++) {
+        int row[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const int pos = off + c0 + min(16 * (kXTile * i + jhalf) + 4 * (wave & 3) + j, nt - 1);
+          row[j] = a.row_index ? ((const __attribute__((address_space(4))) int32_t *)a.row_index)[pos] : pos;
+        }
+        const int rr = lg < 2 ? (lg == 0 ? row[0] : row[1]) : (lg == 2 ? row[2] : row[3]);
+        xsrc[i] = (uint32_t)rr * (uint32_t)a.K + 8 * spiece;
+      }
+    } else {  // (20 or more rows a wave would spill scalar registers)
+#pragma unroll
+      for (int i = 0; i < kXLoads; i++) {
+        const int pos = off + c0 + min(16 * (kXTile * i + jhalf) + srow, nt - 1);
+        xsrc[i] = (uint32_t)(a.row_index ? a.row_index[pos] : pos) * (uint32_t)a.K + 8 * spiece;
+      }
+      first_w();
+    }
     auto load_x = [&](int p) {
-      const uint32_t st = lds0 + (p & 1) * kStage + 4 * (wave & 3) * 256;
+      const uint32_t st = lds0 + (p % (DX + 1)) * kStage + 4 * (wave & 3) * 256;
 #pragma unroll
       for (int i = 0; i < kXLoads; i++)
-        seg_load_lds(a.x + xsrc[i] + 128 * p, __builtin_amdgcn_readfirstlane(st + 16 * (2 * i + jhalf) * 256));
+        seg_load_lds(a.x + xsrc[i] + 128 * p, __builtin_amdgcn_readfirstlane(st + 16 * (kXTile * i + jhalf) * 256));
     };
 
     f32x4 acc[TTS][kSegRB];
@@ -238,7 +298,7 @@ __global__ __launch_bounds__(kSegThreads) __attribute__((amdgpu_waves_per_eu(2, 
     // dequantization from being scheduled between the MFMAs); side(t) is the dequantization of
     // one B fragment (word t % 2 of row block t / 2) interleaved with tile t's MFMAs (t < 8)
     auto tiles = [&](int p, int g, Frag8 (&bw)[kSegRB][2], auto &&side) {
-      const uint8_t *xs = seg_lds + (p & 1) * kStage + frow;
+      const uint8_t *xs = seg_lds + (p % (DX + 1)) * kStage + frow;
       const int pa = 8 * g + 2 * lg;
       const int o0 = 16 * (pa ^ lr), o1 = 16 * ((pa + 1) ^ lr);
       Frag8 xa[kSegAhead + 1][2];
@@ -261,63 +321,70 @@ __global__ __launch_bounds__(kSegThreads) __attribute__((amdgpu_waves_per_eu(2, 
           acc[t][r] = mfma16x16x32(c[1], bw[r][1], acc[t][r]);
         }
         if (t < 2 * kSegRB) side(t);
-#if JIT_SEG_IGLP
-        // one MFMA, then three VALU instructions of the side dequantization, eight times: the
-        // VALU work issues while the matrix core runs instead of between bursts of MFMAs
-        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-        for (int i = 0; i < 2 * kSegRB; i++) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#endif
       }
       // (a chunk of fewer tiles than B fragments runs the rest of them after its tiles)
 #pragma unroll
       for (int t = TTS; t < 2 * kSegRB; t++) side(t);
     };
 
-    // prologue: step 0's activations and weights, step 1's weights; group 0 of step 0
-    load_x(0);
-    load_w(0);
-    if (GP > 1) load_w(1);
-    if (GP > 1)
-      seg_wait_vm<kSegWLoads>();
-    else
-      seg_wait_vm<0>();
+    // Loads are issued as w(0 .. DW - 1), x(0 .. DX - 1), then x(p + DX), w(p + DW) at the top of each
+    // step p, as far as the steps exist.  A wait may leave in flight the loads issued after the awaited
+    // ones; wait_x and wait_w count exactly those (every wave issues the same sequence).
+    auto wait_x = [&](int p) {  // at the top of step p, before its loads: x(p) has landed
+      if (p >= DX && p - 1 + DW <= last) {
+        seg_wait_vm<(DX - 1) * kXLoads + DX * kSegWLoads>();
+        return;
+      }
+      const int nx = min(p - 1 + DX, last) - p;
+      const int nw = min(p - 1 + DW, last) - (p < DX ? DW - 1 : p - DX + DW - 1);
+      seg_wait_vm_n<0, S::kMaxWait + 1>(
+          __builtin_amdgcn_readfirstlane(max(nx, 0) * kXLoads + max(nw, 0) * kSegWLoads));
+    };
+    auto wait_w = [&](int p) {  // in step p, after its loads: w(p + 1) has landed
+      if (p + 1 >= DW && p + DW <= last && p + DX <= last) {
+        seg_wait_vm<(DW - 1) * (kXLoads + kSegWLoads)>();
+        return;
+      }
+      const int nw = min(p + DW, last) - (p + 1);
+      const int nx = min(p + DX, last) - (p + 1 < DW ? -1 : p + 1 - DW + DX);
+      seg_wait_vm_n<0, S::kMaxWait + 1>(
+          __builtin_amdgcn_readfirstlane(max(nx, 0) * kXLoads + max(nw, 0) * kSegWLoads));
+    };
+#pragma unroll
+    for (int i = 0; i < DX; i++)
+      if (i <= last) load_x(i);
+    wait_w(-1);
+    fetch_w(0);
+    wait_x(0);
     seg_barrier();
 #pragma unroll
-    for (int r = 0; r < kSegRB; r++) dequant_rb(0, 0, r, bw0);
+    for (int r = 0; r < kSegRB; r++) {
+      dequant_at(0, r, 0, bw0);
+      dequant_at(0, r, 1, bw0);
+    }
     for (int p = 0; p < GP; p++) {
       if (p > 0) {
-        // step p's activations: the loads issued after them are step p + 1's weights
-        if (p + 1 < GP)
-          seg_wait_vm<kSegWLoads>();
-        else
-          seg_wait_vm<0>();
+        wait_x(p);
         seg_barrier();
       }
-      if (p + 1 < GP) load_x(p + 1);
-      if (p + 2 < GP) load_w(p + 2);
-      tiles(p, 0, bw0, [&](int t) { dequant_word_at(p, 1, t >> 1, t & 1, bw1); });
-      // step p + 1's weights: issued after them, step p + 1's activations (TTS / 2 loads) and
-      // step p + 2's weights, as far as those exist
-      if (p + 2 < GP)
-        seg_wait_vm<kXLoads + kSegWLoads>();
-      else if (p + 1 < GP)
-        seg_wait_vm<kXLoads>();
-      // (after the last step the dequantization below reads a stale stage and is unused)
-      tiles(p, 1, bw1, [&](int t) { dequant_word_at(p + 1, 0, t >> 1, t & 1, bw0); });
+      if (p + DX <= last) load_x(p + DX);
+      if (p + DW <= last) load_w(p + DW);
+      tiles(p, 0, bw0, [&](int t) { dequant_at(1, t >> 1, t & 1, bw1); });
+      if (p < last) wait_w(p);
+      asm volatile("" ::: "memory");
+      fetch_w(p + 1);  // (after the last step a stale stage, unused)
+      tiles(p, 1, bw1, [&](int t) { dequant_at(0, t >> 1, t & 1, bw0); });
     }
 
     // SwiGLU's sigmoid by table (qtile::swiglu_bf16_tab, exhaustively equal to the bf16 steps): every
     // wave is done with the stages, so the table (7.7 KB) takes the start of the LDS, one entry
     // or so a thread instead of ~45 instructions for each of a lane's ~40 outputs
+    // (a short chunk's few outputs cost less by the steps than a table entry or more a thread)
+    constexpr bool kTable = SWIGLU && 4 * TTS > qtile::kSigEntries / S::kThreads + 4;
     const uint16_t *sig_tab = (const uint16_t *)seg_lds;
-    if constexpr (SWIGLU) {
+    if constexpr (kTable) {
       __syncthreads();
-      for (int i = tid; i < qtile::kSigEntries; i += kSegThreads) ((uint16_t *)seg_lds)[i] = qtile::sigmoid_entry(i);
+      for (int i = tid; i < qtile::kSigEntries; i += S::kThreads) ((uint16_t *)seg_lds)[i] = qtile::sigmoid_entry(i);
       __syncthreads();
     }
     // lane l holds C[token 16 t + 4 lg + i][row 16 rbk[r] + lr].  No branch per token: the
@@ -334,8 +401,12 @@ __global__ __launch_bounds__(kSegThreads) __attribute__((amdgpu_waves_per_eu(2, 
         const int tok = 16 * t + 4 * lg + i;
         const uint32_t ro = tok < nt ? (uint32_t)(off + c0 + tok) * (uint32_t)a.N * 2u : 0x80000000u;
         if (SWIGLU) {
-          __builtin_amdgcn_raw_buffer_store_b16((unsigned short)qtile::swiglu_bf16_tab(acc[t][0][i], acc[t][1][i], sig_tab), obuf,
-                                                (int)(ro + 2u * (16 * rbk[0] + lr)), 0, 0);
+          uint32_t hv;
+          if constexpr (kTable)
+            hv = qtile::swiglu_bf16_tab(acc[t][0][i], acc[t][1][i], sig_tab);
+          else
+            hv = qtile::swiglu_bf16(acc[t][0][i], acc[t][1][i]);
+          __builtin_amdgcn_raw_buffer_store_b16((unsigned short)hv, obuf, (int)(ro + 2u * (16 * rbk[0] + lr)), 0, 0);
         } else {
 #pragma unroll
           for (int r = 0; r < kSegRB; r++)
@@ -347,15 +418,77 @@ __global__ __launch_bounds__(kSegThreads) __attribute__((amdgpu_waves_per_eu(2, 
   }
 }
 
-// The kernels take more LDS than the static limit: raise their dynamic limit once.
-template <bool SWIGLU, bool DENSE, int TTS>
-void seg_prepare() {
+// One launch of a shape: `cols` column blocks of its rows for each of a.groups groups (the kernels take
+// more LDS than the static limit: raise their dynamic limit once).
+template <bool SWIGLU, bool DENSE, class S>
+void seg_launch(SegArgs a, int rows, hipStream_t st) {
   static const bool done = [] {
-    (void)hipFuncSetAttribute((const void *)&seg_kernel<SWIGLU, DENSE, TTS>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, seg_lds_bytes(TTS));
+    (void)hipFuncSetAttribute((const void *)&seg_kernel<SWIGLU, DENSE, S>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              S::kLds);
     return true;
   }();
   (void)done;
+  a.nx = rows / S::kRows;
+  if (DENSE) a.groups = (a.T + S::kTokens - 1) / S::kTokens;
+  seg_kernel<SWIGLU, DENSE, S><<<seg_grid(a.nx, a.groups), S::kThreads, S::kLds, st>>>(a);
+}
+
+// The chunk length of expert segments: the smallest that holds the mean segment plus 2.5 of its
+// standard deviations under even routing (sqrt(mean)), so that few experts need a second pass over
+// their weights and few tiles are computed past a segment's end.  A shorter chunk re-reads the weights
+// (512 rows, mean 32: 2 tiles 103 + 54 us gate||up + down, 3 tiles 75 + 42), a longer one computes
+// padding (4 tiles 78 + 43, 6 tiles 95 + 53, 10 tiles 125 + 64).  Every shape gives the same bits.
+template <bool SWIGLU>
+void seg_experts(const SegArgs &a, int rows, int P, hipStream_t st) {
+  const float mean = (float)P / (float)a.groups, need = mean + 2.5f * sqrtf(mean);
+  if (need <= 16.0f)
+    seg_launch<SWIGLU, false, SegShape<1, 4, 2, 2, 4>>(a, rows, st);
+  else if (need <= 32.0f)
+    seg_launch<SWIGLU, false, SegShape<2, 4, 2, 2, 3>>(a, rows, st);
+  else if (need <= 48.0f)
+    seg_launch<SWIGLU, false, SegShape<3, 4, 1, 2, 3>>(a, rows, st);
+  else if (need <= 64.0f)
+    seg_launch<SWIGLU, false, SegShape<4, 4, 1, 2, 3>>(a, rows, st);
+  else if (need <= 96.0f)
+    seg_launch<SWIGLU, false, SegShape<6, 8, 1, 2>>(a, rows, st);
+  else
+    seg_launch<SWIGLU, false, SegShape<10, 8, 1, 2>>(a, rows, st);
+}
+
+// The chunk length of a dense matrix (its token chunks spread over workgroups): the least estimated
+// time of a K step, from the workgroups L that the busiest CU gets (seg_block deals whole groups to 8
+// XCDs).  Up to three workgroups of 4 waves share a CU, 0.38 + L (0.24 + 0.09 tiles) us a step; those of
+// 8 waves follow one another, 0.60 + 0.17 tiles each.  Fitted to N = 5120, K = 2048 and N = 2048,
+// K = 4096 at 192 .. 2,108 rows, where it picks the fastest shape measured: 192 rows 20 + 25 us, 512
+// rows 25 + 26 (36 + 36 before), 1,024 rows 33 + 30, 2,108 rows 56 + 48 (79 + 57 before).
+float seg_dense_step_us(int tts, int waves, int T, int N, int cus) {
+  const int groups = (T + 16 * tts - 1) / (16 * tts), per_xcd = (N / seg_rows(waves)) * ((groups + 7) / 8);
+  const int cu = cus >= 8 ? cus / 8 : 1, L = (per_xcd + cu - 1) / cu;
+  if (waves == 8) return (float)L * (0.60f + 0.17f * (float)tts);
+  auto round_us = [&](int n) { return n ? 0.38f + (float)n * (0.24f + 0.09f * (float)tts) : 0.0f; };
+  return (float)(L / 3) * round_us(3) + round_us(L % 3);
+}
+
+void seg_dense(const SegArgs &a, hipStream_t st) {
+  static constexpr int kTiles[] = {2, 3, 4, 6, 8, 10};
+  const int cus = jit::cu_count();
+  int best = 10;
+  float best_us = INFINITY;
+  for (int t : kTiles) {
+    const float us = seg_dense_step_us(t, t <= 4 ? 4 : 8, a.T, a.N, cus);
+    if (us < best_us) {
+      best_us = us;
+      best = t;
+    }
+  }
+  switch (best) {
+    case 2: return seg_launch<false, true, SegShape<2, 4, 2, 2, 3>>(a, a.N, st);
+    case 3: return seg_launch<false, true, SegShape<3, 4, 1, 2, 3>>(a, a.N, st);
+    case 4: return seg_launch<false, true, SegShape<4, 4, 1, 2, 3>>(a, a.N, st);
+    case 6: return seg_launch<false, true, SegShape<6, 8, 1, 2>>(a, a.N, st);
+    case 8: return seg_launch<false, true, SegShape<8, 8, 1, 2>>(a, a.N, st);
+    default: return seg_launch<false, true, SegShape<10, 8, 1, 2>>(a, a.N, st);
+  }
 }
 
 }  // namespace
@@ -373,10 +506,9 @@ extern "C" int jit_moe_gate_up_swiglu_seg(const uint16_t *x, int K, const int32_
     return jit::fail(JIT_EINVAL, "moe_gate_up_seg: null pointer");
   if ((long long)P * I * 2 >= (1LL << 31))
     return jit::fail(JIT_EUNSUPPORTED, "moe_gate_up_seg: h of %d x %d bf16 exceeds 2 GiB", P, I);
-  SegArgs a{x, pair_row, expert_cnt, expert_off, (const uint8_t *)packed, h, jit_q4_packed_bytes(1, 2 * I, K), K, I, 0,
-            I / 128, E};
-  seg_prepare<true, false, kSegTT>();
-  seg_kernel<true><<<seg_grid(a.nx, E), kSegThreads, seg_lds_bytes(kSegTT), (hipStream_t)stream>>>(a);
+  const SegArgs a{x, pair_row, expert_cnt, expert_off, (const uint8_t *)packed, h, jit_q4_packed_bytes(1, 2 * I, K), K, I,
+                  0, 0, E};
+  seg_experts<true>(a, 2 * I, P, (hipStream_t)stream);
   return jit::check_launch("jit_moe_gate_up_swiglu_seg");
 }
 
@@ -391,10 +523,9 @@ extern "C" int jit_moe_down_seg(const uint16_t *h, int I, const int32_t *expert_
   if (!h || !expert_cnt || !expert_off || !packed || !r) return jit::fail(JIT_EINVAL, "moe_down_seg: null pointer");
   if ((long long)P * D * 2 >= (1LL << 31))
     return jit::fail(JIT_EUNSUPPORTED, "moe_down_seg: r of %d x %d bf16 exceeds 2 GiB", P, D);
-  SegArgs a{h, nullptr, expert_cnt, expert_off, (const uint8_t *)packed, r, jit_q4_packed_bytes(1, D, I), I, D, 0,
-            D / kSegRows, E};
-  seg_prepare<false, false, kSegTT>();
-  seg_kernel<false><<<seg_grid(a.nx, E), kSegThreads, seg_lds_bytes(kSegTT), (hipStream_t)stream>>>(a);
+  const SegArgs a{h, nullptr, expert_cnt, expert_off, (const uint8_t *)packed, r, jit_q4_packed_bytes(1, D, I), I, D, 0, 0,
+                  E};
+  seg_experts<false>(a, D, P, (hipStream_t)stream);
   return jit::check_launch("jit_moe_down_seg");
 }
 
@@ -407,28 +538,7 @@ extern "C" int jit_qmm_seg(const uint16_t *x, int T, int K, const void *packed, 
   if (!x || !packed || !y) return jit::fail(JIT_EINVAL, "qmm_seg: null pointer");
   if ((long long)T * N * 2 >= (1LL << 31))
     return jit::fail(JIT_EUNSUPPORTED, "qmm_seg: y of %d x %d bf16 exceeds 2 GiB", T, N);
-  // The chunk (token tiles per workgroup, even: the two halves of the waves stage alternate
-  // tiles) is the smallest of 4, 6, 8, 10 whose workgroups fill the CUs in one round: chunks of
-  // 10 can leave most CUs idle (config 3's o_proj, N = 2048 over 2,108 tokens: 112 workgroups),
-  // while smaller chunks only add dequantization.  Batches too long for one round take chunks of
-  // 10.
-  const int nx = N / kSegRows, cus = jit::cu_count();
-  auto groups = [&](int tts) { return (T + 16 * tts - 1) / (16 * tts); };
-  const hipStream_t st = (hipStream_t)stream;
-#define JIT_QMM_SEG(TTS)                                                                                       \
-  {                                                                                                            \
-    SegArgs a{x, nullptr, nullptr, nullptr, (const uint8_t *)packed, y, 0, K, N, T, nx, groups(TTS)};          \
-    seg_prepare<false, true, TTS>();                                                                           \
-    seg_kernel<false, true, TTS><<<seg_grid(nx, groups(TTS)), kSegThreads, seg_lds_bytes(TTS), st>>>(a);      \
-  }
-  if (nx * groups(4) <= cus)
-    JIT_QMM_SEG(4)
-  else if (nx * groups(6) <= cus)
-    JIT_QMM_SEG(6)
-  else if (nx * groups(8) <= cus)
-    JIT_QMM_SEG(8)
-  else
-    JIT_QMM_SEG(10)
-#undef JIT_QMM_SEG
+  const SegArgs a{x, nullptr, nullptr, nullptr, (const uint8_t *)packed, y, 0, K, N, T, 0, 0};
+  seg_dense(a, (hipStream_t)stream);
   return jit::check_launch("jit_qmm_seg");
 }

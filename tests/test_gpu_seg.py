@@ -188,3 +188,49 @@ def test_dense_segment_gemm_repeats_bit_for_bit(T, N, K):
     first = ops.qmm(x, q, seg=True)
     for _ in range(12):
         assert torch.equal(ops.qmm(x, q, seg=True), first)
+
+
+@pytest.mark.parametrize("K", [128, 256, 640, 2048])
+@pytest.mark.parametrize("mean", [4, 10, 20, 40, 60, 120])
+def test_segment_gemm_chunk_lengths(mean, K):
+    """Every chunk length of the segment GEMM (its rule goes by the mean pairs per expert: 1, 2, 3, 4,
+    6 and 10 token tiles here) at its edges: segments of 0, 1, a tile, a tile + 1, a chunk, a chunk + 1
+    and three chunks, over 1, 2, 5 and 16 K steps (fewer than the loads run ahead, and more).  The
+    output of gate||up and of down equals the oracle's bf16-weight restatement as in the tests above."""
+    E, N = 12, 256
+    tiles = {4: 1, 10: 2, 20: 3, 40: 4, 60: 6, 120: 10}[mean]
+    cnt = np.array([0, 1, 16, 17, 16 * tiles, 16 * tiles + 1, 48 * tiles - 1, 0, 0, 0, 0, 0])
+    rest = mean * E - int(cnt.sum())
+    if rest > 0:
+        cnt[7:11] = [rest // 4, rest // 4, rest // 4, rest - 3 * (rest // 4)]
+    P = int(cnt.sum())
+    inds = np.random.default_rng(mean + K).permutation(np.repeat(np.arange(E), cnt)).astype(np.int32).reshape(P, 1)
+    gu_h, dn_h = _stack(E, N, K, mean + K), _stack(E, N, K, mean + K + 1)
+    x = normal_bf16((P, K), seed=mean)
+    pk = ops.moe_pack(torch.from_numpy(inds).to(DEV), E)
+    opk = oracle.moe_pack(inds.view(np.uint32), E)
+    h = ops.expert_gate_up(bf16_tensor(x, DEV), ops.prepack(gu_h.to(DEV)), pk, seg=True)
+    want = oracle.moe_gate_up(x, inds.view(np.uint32), opk, *stack_np(gu_h), bf16w=True)
+    st = assert_close_bf16(u16(h), want, what=f"gate_up mean {mean} K {K}")
+    assert st["bit_equal"] > 0.9, st
+    xs = bf16_tensor(x[opk["order"]], DEV)
+    r = ops.expert_down(xs, ops.prepack(dn_h.to(DEV)), pk, seg=True)
+    want = oracle.moe_down(u16(xs), inds.view(np.uint32), opk, *stack_np(dn_h), bf16w=True)
+    st = assert_close_bf16(u16(r), want, what=f"down mean {mean} K {K}")
+    assert st["bit_equal"] > 0.9, st
+
+
+@pytest.mark.parametrize("T,N,K", [(1, 256, 128), (40, 256, 256), (192, 5120, 2048), (300, 5120, 2048), (512, 5120, 2048),
+                                   (1024, 5120, 2048), (4000, 2048, 384)])
+def test_dense_segment_gemm_shapes(T, N, K):
+    """The dense launch's chunk lengths (2, 3, 4, 6, 8 and 10 tiles by estimated time) against float64
+    sums over the same bf16 weights: one bf16 rounding, and fp32 accumulation of K products."""
+    from jitengine_amd.quant import dequantize4
+
+    q = random_quantized((N, K), T + K, device=DEV)
+    x = bf16_tensor(normal_bf16((T, K), seed=T), DEV)
+    w = dequantize4(q).to(torch.bfloat16).double()  # (s q + b is exact in float32 for these weights' range)
+    want = x.double() @ w.t().contiguous()
+    got = ops.qmm(x, ops.prepack(q), seg=True).double()
+    tol = want.abs() * 2.0 ** -8 + K * 2.0 ** -24 * (x.double().abs() @ w.abs().t().contiguous())
+    assert bool(((got - want).abs() <= tol).all())
