@@ -566,6 +566,174 @@ int launch_qmm(const QmmArgs &a, int E, hipStream_t st, const char *what, int zs
   return jit::check_launch(what);
 }
 
+// A tall packed matrix (an lm_head's vocabulary) over a decode batch: persistent workgroups hold their
+// waves' K slices of 16 TT tokens' activations in registers and walk row tiles of 16 NB rows (blockIdx.x,
+// + gridDim.x, ..) with the next tile's weight slice in flight.  qmm_kernel gives every row tile a
+// workgroup, which reads all of its tokens' activations for 32 rows of weights -- at 32 tokens 128 KB from
+// L2 for 37 KB of weights, and the weights once more for every 16 tokens.  Each output's sum is
+// qmm_kernel's, in its order: the same bits.  Measured at N = 151,936, K = 2048 (175 MB of weights, 27 us
+// at 6.5 TB/s), qmm_kernel -> here: 1 row 37.4 -> 31.3 us (two workgroups a CU), 8 rows 40.9 -> 31.1, 32
+// rows 94 -> 45, 64 rows 184 -> 68, 100 rows 403 -> 127.  Now bound by issue (unpacking, MFMAs and the
+// reduction) past 16 rows: two tiles ahead, or the groups' activation sums kept in registers, change nothing.
+template <int NB, int GPW, int TT>
+__global__ __launch_bounds__(512) void qmm_walk_kernel(const QmmArgs a) {
+  static_assert(GPW % 2 == 0 && GPW / 2 <= 4, "one scale load covers at most 4 group pairs");
+  extern __shared__ float red[];  // [2][ksplit][TT][NB][4][64]
+  const int ksplit = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id();
+  const int lr = l & 15, lg = l >> 4;
+  const int GP = a.K >> 7;
+  const int g0 = wave * GPW;
+  const int t0 = 16 * TT * blockIdx.y, cnt = a.T;
+  const int tiles = (a.N + 16 * NB - 1) / (16 * NB), stride = gridDim.x;
+
+  struct Slice {  // a row tile's weights of this wave's K slice
+    uint2 w[GPW][NB];
+    uint2 sb[NB];  // 8 bytes of the block's scale tile, shuffled when used
+  };
+  Slice sl[2];
+  auto load = [&](Slice &v, int tile) {
+    const int n0 = min(tile, tiles - 1) * 16 * NB;  // (past the last tile: loaded and unused)
+#pragma unroll
+    for (int rb = 0; rb < NB; rb++) {
+      const int rowb = n0 + 16 * rb < a.N ? n0 + 16 * rb : n0;  // rows past N read block n0, never stored
+      const uint8_t *blk = (const uint8_t *)a.w + (long long)(rowb >> 4) * GP * kTileBytes;
+      v.sb[rb] =
+          ld_stream8(blk + (long long)GP * kNibbleBytes + ((g0 >> 1) + min(lg, GPW / 2 - 1)) * kScaleBytes + 8 * lr);
+#pragma unroll
+      for (int j = 0; j < GPW / 2; j++) {
+        const uint4 q = ld_stream16(blk + ((g0 >> 1) + j) * kNibbleBytes + 16 * l);
+        v.w[2 * j][rb] = make_uint2(q.x, q.y);
+        v.w[2 * j + 1][rb] = make_uint2(q.z, q.w);
+      }
+    }
+  };
+
+  // the activations (padding tokens read zeros: offsets past the buffer's range)
+  const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc((void *)a.x, (short)0, 0x7fffffff, 0x00020000);
+  Frag8 xa[TT][GPW][2];
+#pragma unroll
+  for (int tt = 0; tt < TT; tt++) {
+    const int tok = t0 + 16 * tt + lr;
+    const uint32_t xo = (tok < cnt ? (uint32_t)tok * (uint32_t)a.K * 2u : kXOutOfRange) + 2u * (64 * g0 + 16 * lg);
+#pragma unroll
+    for (int g = 0; g < GPW; g++) {
+      const u32x4 v0 = __builtin_amdgcn_raw_buffer_load_b128(xbuf, xo + 128 * g, 0, 0);
+      const u32x4 v1 = __builtin_amdgcn_raw_buffer_load_b128(xbuf, xo + 128 * g + 16, 0, 0);
+      xa[tt][g][0].q = make_uint4(v0.x, v0.y, v0.z, v0.w);
+      xa[tt][g][1].q = make_uint4(v1.x, v1.y, v1.z, v1.w);
+    }
+  }
+  Frag8 ones;
+#pragma unroll
+  for (int i = 0; i < 4; i++) ones.u[i] = 0x3F803F80u;
+  UNPACK_CONSTANTS(um, uc);
+
+  auto step = [&](const Slice &v, int tile, int parity) {
+    f32x4 acc[TT][NB];
+#pragma unroll
+    for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+      for (int rb = 0; rb < NB; rb++) acc[tt][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    uint32_t sv[NB][GPW / 2], bv[NB][GPW / 2];
+#pragma unroll
+    for (int rb = 0; rb < NB; rb++)
+#pragma unroll
+      for (int j = 0; j < GPW / 2; j++) {
+        sv[rb][j] = (uint32_t)__shfl((int)v.sb[rb].x, 16 * j + lr, 64);
+        bv[rb][j] = (uint32_t)__shfl((int)v.sb[rb].y, 16 * j + lr, 64);
+      }
+#pragma unroll
+    for (int g = 0; g < GPW; g++) {
+      f32x4 X[TT];
+#pragma unroll
+      for (int tt = 0; tt < TT; tt++) {
+        X[tt] = mfma16x16x32(xa[tt][g][0], ones, f32x4{0.f, 0.f, 0.f, 0.f});
+        X[tt] = mfma16x16x32(xa[tt][g][1], ones, X[tt]);
+      }
+#pragma unroll
+      for (int rb = 0; rb < NB; rb++) {
+        const Frag8 B0 = unpack_nibbles(v.w[g][rb].x, um, uc), B1 = unpack_nibbles(v.w[g][rb].y, um, uc);
+        const float sc = (g & 1) ? bf2f_hi(sv[rb][g >> 1]) : bf2f(sv[rb][g >> 1] & 0xffffu);
+        const float bi = (g & 1) ? bf2f_hi(bv[rb][g >> 1]) : bf2f(bv[rb][g >> 1] & 0xffffu);
+        const float bq = fmaf(-128.0f, sc, bi);
+#pragma unroll
+        for (int tt = 0; tt < TT; tt++) {
+          f32x4 C = mfma16x16x32(xa[tt][g][0], B0, f32x4{0.f, 0.f, 0.f, 0.f});
+          C = mfma16x16x32(xa[tt][g][1], B1, C);
+#pragma unroll
+          for (int i = 0; i < 4; i++) acc[tt][rb][i] = fmaf(bq, X[tt][i], fmaf(sc, C[i], acc[tt][rb][i]));
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the waves' partial sums meet in one of two LDS buffers: a buffer's readers are past the next
+    // tile's barrier before it is written again, so one barrier a tile orders both.  (Issued bare: a
+    // __syncthreads fence would wait for the weights in flight.)
+    float *buf = red + parity * ksplit * TT * NB * 4 * 64;
+#pragma unroll
+    for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+      for (int rb = 0; rb < NB; rb++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) buf[(((wave * TT + tt) * NB + rb) * 4 + i) * 64 + l] = acc[tt][rb][i];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const int n0 = tile * 16 * NB;
+    // 8 adjacent outputs a thread: (tile, token, row octet) items, the slices added in wave order
+    for (int it = threadIdx.x; it < TT * 16 * 2 * NB; it += ksplit * 64) {
+      const int half = it & 1, ob = (it >> 1) % NB, rest = (it >> 1) / NB, tok = rest & 15, tt = rest >> 4;
+      const int t = t0 + 16 * tt + tok;
+      if (n0 + 16 * ob >= a.N || t >= cnt) continue;
+      const int lane0 = 16 * (tok >> 2) + 8 * half;
+      float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      for (int ks = 0; ks < ksplit; ks++) {
+        const float *pr = buf + (((ks * TT + tt) * NB + ob) * 4 + (tok & 3)) * 64 + lane0;
+        const float4 p0 = *(const float4 *)pr, p1 = *(const float4 *)(pr + 4);
+        o[0] += p0.x;
+        o[1] += p0.y;
+        o[2] += p0.z;
+        o[3] += p0.w;
+        o[4] += p1.x;
+        o[5] += p1.y;
+        o[6] += p1.z;
+        o[7] += p1.w;
+      }
+      *(uint4 *)(a.out + (long long)t * a.N + n0 + 16 * ob + 8 * half) =
+          make_uint4(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]), pack_bf16x2(o[4], o[5]), pack_bf16x2(o[6], o[7]));
+    }
+  };
+
+  load(sl[0], blockIdx.x);
+  for (int tile = blockIdx.x; tile < tiles;) {
+#pragma unroll
+    for (int d = 0; d < 2; d++) {  // (the slices alternate by unrolling)
+      if (tile >= tiles) break;
+      load(sl[1 - d], tile + stride);
+      asm volatile("" ::: "memory");  // (the loads stay ahead of this tile's arithmetic)
+      step(sl[d], tile, d);
+      tile += stride;
+    }
+  }
+}
+
+template <int NB, int GPW, int TT>
+int launch_walk(const QmmArgs &a, int per_cu, hipStream_t st, const char *what) {
+  const int ksplit = a.K / 64 / GPW;
+  const size_t lds = (size_t)2 * ksplit * TT * NB * 4 * 64 * sizeof(float);
+  static const bool done = [] {  // (four token tiles take more LDS than the static limit)
+    (void)hipFuncSetAttribute((const void *)&qmm_walk_kernel<NB, GPW, TT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              2 * 8 * TT * NB * 4 * 64 * (int)sizeof(float));
+    return true;
+  }();
+  (void)done;
+  const int tiles = (a.N + 16 * NB - 1) / (16 * NB), wgs = per_cu * jit::cu_count();
+  const dim3 grid(tiles < wgs ? tiles : wgs, (a.T + 16 * TT - 1) / (16 * TT));
+  qmm_walk_kernel<NB, GPW, TT><<<grid, 64 * ksplit, lds, st>>>(a);
+  return jit::check_launch(what);
+}
+
 // Groups per wave for a dense projection: the smallest even slice that splits K over at
 // most 8 waves (the packed and direct layouts use the same split, so they agree bit for bit).
 int dense_gpw(int K) {
@@ -575,28 +743,46 @@ int dense_gpw(int K) {
   return 0;
 }
 
-// Dense launch shape: up to two token tiles per pass (one reduction round for a
-// 32-row decode batch), and 32 output rows per workgroup for a wide matrix with a
-// short K-slice per wave (the activations each workgroup pulls through L2 then
-// serve twice the rows).  The shape never changes a result: each output sums the
-// same groups in the same order.
+// Dense launch shape, by the rows, the matrix and the K slice of a wave: see the measured lines below.
+// The shape never changes a result: each output sums the same groups in the same order.
 #ifndef JIT_DENSE_ZMAX
 #define JIT_DENSE_ZMAX 4
 #endif
 #ifndef JIT_DENSE_WIDE_N
 #define JIT_DENSE_WIDE_N 4096
 #endif
+#ifndef JIT_DENSE_WALK_N
+#define JIT_DENSE_WALK_N 16384
+#endif
 template <bool PACKED, int GPW>
 int launch_dense_gpw(const QmmArgs &a, hipStream_t st, const char *what) {
+  // (16-byte output stores: an output that is not 16-byte aligned keeps qmm_kernel's 2-byte ones)
+  const bool aligned = ((uintptr_t)a.out & 15) == 0;
+  // a tall matrix: two row tiles of 32 rows a CU or more (N = 16,384: 32 rows 13.0 -> 10.1 us, 64 rows 22 ->
+  // 15; below, workgroups of one or two tiles do not repay the walk).  K slices of 6 or 8 groups a wave
+  // would not leave registers for the activations of 64 tokens.
+  if constexpr (PACKED && GPW <= 4) {
+    if (aligned && a.N >= JIT_DENSE_WALK_N) {
+      if (a.T <= 16) return launch_walk<2, GPW, 1>(a, 2, st, what);
+      if (a.T <= 32) return launch_walk<2, GPW, 2>(a, 1, st, what);
+      return launch_walk<2, GPW, 4>(a, 1, st, what);
+    }
+  }
   // a decode batch's 16-token tiles go to separate workgroups (up to JIT_DENSE_ZMAX), so a
-  // matrix of few row blocks still fills the chip and each workgroup pulls one tile's
-  // activations; longer batches take two tiles per pass
-  // (a prefill-sized batch spreads its 32-token passes over workgroups too: one pass each)
+  // matrix of few row blocks still fills the chip and each workgroup pulls one tile's activations
   const int tiles = (a.T + 15) / 16;
   const bool wide = GPW <= 4 && a.N >= JIT_DENSE_WIDE_N;
   if (tiles <= JIT_DENSE_ZMAX)
     return wide ? launch_qmm<2, GPW, false, PACKED, 1>(a, 1, st, what, tiles)
                 : launch_qmm<1, GPW, false, PACKED, 1>(a, 1, st, what, tiles);
+  // longer batches take 64-row workgroups: what bounds them is the activations, which each workgroup pulls
+  // through L2 for all its rows.  Two token tiles a pass where the K slice is short (N = 5120, K = 2048: 100
+  // rows 16.7 -> 13.9 us, 160 rows 24.4 -> 16.1; N = 128, 2,108 rows 15 -> 10), one where it is long (N = 2048,
+  // K = 4096: 100 rows 19.4 -> 10.7 us, 160 rows 28.5 -> 19.1; two tiles 24.5 and 27.2).
+  if (aligned) {
+    constexpr int TT = GPW <= 4 ? 2 : 1;
+    return launch_qmm<4, GPW, false, PACKED, TT>(a, 1, st, what, (tiles + TT - 1) / TT);
+  }
   const int passes = (tiles + 1) / 2;
   return wide ? launch_qmm<2, GPW, false, PACKED, 2>(a, 1, st, what, passes)
               : launch_qmm<1, GPW, false, PACKED, 2>(a, 1, st, what, passes);
