@@ -318,6 +318,10 @@ int jit_attn_plan(const int32_t *lens_host, int B, int32_t *chunk_start_host,
 
 /* Workspace bytes jit_paged_decode_attn needs for `total_chunks` chunks. */
 int64_t jit_attn_workspace_bytes(int total_chunks, int H);
+/* Workspace bytes with which jit_paged_decode_attn_ws / _qkv_ws take the finest split of a plan of
+ * `total_chunks` chunks: a plan of few chunks is spread over four times the workgroups, each leaving
+ * a partial; otherwise jit_attn_workspace_bytes. */
+int64_t jit_attn_split_workspace_bytes(int total_chunks, int H, int Hkv);
 
 /* Paged GQA decode attention, one query per row: out[b, h] =
  * softmax(scale * q[b, h] . K_b^T) . V_b over the first lens[b] tokens of
@@ -336,6 +340,14 @@ int jit_paged_decode_attn(const uint16_t *q, const uint16_t *pool, const int32_t
                           int max_pages, const int32_t *lens, const int32_t *chunk_start,
                           const int32_t *chunk_seq, int B, int H, int Hkv, float scale,
                           int total_chunks, void *workspace, uint16_t *out, void *stream);
+/* The same with the workspace's size: at least jit_attn_workspace_bytes (JIT_EINVAL), and with
+ * jit_attn_split_workspace_bytes a plan of few chunks runs on more workgroups.  The bits are the same
+ * for any size. */
+int jit_paged_decode_attn_ws(const uint16_t *q, const uint16_t *pool, const int32_t *page_table,
+                             int max_pages, const int32_t *lens, const int32_t *chunk_start,
+                             const int32_t *chunk_seq, int B, int H, int Hkv, float scale,
+                             int total_chunks, void *workspace, int64_t workspace_bytes, uint16_t *out,
+                             void *stream);
 
 /* jit_paged_decode_attn fused with the step's own token's jit_qk_norm_rope_append: qkv holds
  * the step's raw rows [B, (H + 2 Hkv) * 128] (the qkv projection's output) instead of q.  Row b's
@@ -350,6 +362,13 @@ int jit_paged_decode_attn_qkv(const uint16_t *qkv, const uint16_t *q_norm_w, con
                               int max_pages, const int32_t *lens, const int32_t *chunk_start,
                               const int32_t *chunk_seq, int B, int H, int Hkv, float scale,
                               int total_chunks, void *workspace, uint16_t *out, void *stream);
+/* The same with the workspace's size, as jit_paged_decode_attn_ws. */
+int jit_paged_decode_attn_qkv_ws(const uint16_t *qkv, const uint16_t *q_norm_w, const uint16_t *k_norm_w,
+                                 float eps, const float *inv_freq, uint16_t *pool, const int32_t *page_table,
+                                 int max_pages, const int32_t *lens, const int32_t *chunk_start,
+                                 const int32_t *chunk_seq, int B, int H, int Hkv, float scale,
+                                 int total_chunks, void *workspace, int64_t workspace_bytes, uint16_t *out,
+                                 void *stream);
 
 /* jit_paged_decode_attn without a workspace argument: the same kernels and the same bits,
  * with the fp32 split-K partials in a file-scope device array of JIT_ATTN_SCRATCH_BYTES

@@ -55,6 +55,10 @@ _SIGNATURES = {
     "jit_attn_chunk_tokens": [_I],
     "jit_attn_plan": [_P, _I, _P, _P, _I],
     "jit_attn_workspace_bytes": [_I, _I],
+    "jit_attn_split_workspace_bytes": [_I, _I, _I],
+    "jit_paged_decode_attn_ws": [_P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _F, _I, _P, ctypes.c_int64, _P, _P],
+    "jit_paged_decode_attn_qkv_ws": [_P, _P, _P, _F, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _F, _I, _P, ctypes.c_int64,
+                                     _P, _P],
     "jit_paged_decode_attn": [_P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _F, _I, _P, _P, _P],
     "jit_paged_decode_attn_qkv": [_P, _P, _P, _F, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _F, _I, _P, _P, _P],
     "jit_paged_decode_attn_noalloc": [_P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _F, _I, _P, _P],
@@ -74,6 +78,7 @@ _SIGNATURES = {
     "jit_kv_copy_pages": [_P, _I, _I, _P, _P, _I, _P],
 }
 _RESTYPES = {"jit_last_error": ctypes.c_char_p, "jit_attn_workspace_bytes": ctypes.c_int64,
+             "jit_attn_split_workspace_bytes": ctypes.c_int64,
              "jit_prefill_workspace_bytes": ctypes.c_int64,
              "jit_q4_packed_bytes": ctypes.c_int64, "jit_moe_pack_workspace_bytes": ctypes.c_int64,
              "jit_sampler_workspace_bytes": ctypes.c_int64}

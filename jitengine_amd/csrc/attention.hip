@@ -8,9 +8,10 @@
 // group are 512 B contiguous.
 //
 // Attention work item: one workgroup per chunk (1536 keys; longer for sequences past
-// 196,608 keys) of one sequence and 2 kv heads, 4 waves per kv head, each wave streaming
-// a quarter of the chunk (384 keys) two 16-key
-// pages (32 keys) per step; the 4 waves' states meet in LDS:
+// 196,608 keys) of one sequence and 1 or 2 kv heads, 4 waves per kv head, each wave streaming
+// a quarter of the chunk (384 keys, three sub-runs of 128 with a softmax state each) two 16-key
+// pages (32 keys) per step; the 4 waves' states meet in LDS.  (A plan of few chunks gives every
+// sub-run a wave and every quarter a workgroup.)
 //   S^T[16 keys x 16 q heads] = K_page . Q^T      (4 MFMA 16x16x32 per page)
 //   online softmax in the exp2 domain (fp32 running max / sum per q head)
 //   O^T[128 d x 16 q heads] += V^T . P^T           (16 MFMA 16x16x32, all 32 keys: P as a
@@ -28,6 +29,7 @@
 #include "common.hpp"
 
 #include <mutex>
+#include <type_traits>
 
 namespace {
 
@@ -68,6 +70,16 @@ __host__ __device__ __forceinline__ int chunk_tokens(int len) {
   return c < kChunkMax ? c : kChunkMax;
 }
 
+// A chunk of kChunk keys is kAttnSplits groups of kGroup keys, a group kSubs sub-runs of kSubRun keys.
+// Every sub-run keeps an online-softmax state of its own, a group's state is its sub-runs' merged in
+// order, a chunk's its groups' in order (the chunks of longer sequences, not kChunk keys, have one
+// sub-run a group).  The results are therefore the same whether a wave walks a group's sub-runs one after
+// another or every sub-run has a wave and every group a workgroup of its own (paged_attn_kernel<FINE>): the
+// launch picks by how many workgroups the plan makes.
+constexpr int kSubs = 3;
+constexpr int kGroup = kChunk / kAttnSplits, kSubRun = kGroup / kSubs;
+static_assert(kSubRun * kSubs * kAttnSplits == kChunk && kSubRun % 32 == 0, "sub-runs are whole 32-key steps");
+
 __device__ __forceinline__ int k_off(int slot, int d) { return k_page_offset(slot, d); }
 
 }  // namespace
@@ -103,8 +115,8 @@ struct AttnArgs {
   const int32_t *lens;
   const int32_t *chunk_start;
   const int32_t *chunk_seq;
-  float *part_o;   // [total_chunks][H][128]
-  float *part_ml;  // [total_chunks][H][2]
+  float *part_o;   // [total_chunks][H][128] (fine: [total_chunks][kAttnSplits][H][128])
+  float *part_ml;  // [total_chunks][H][2]   (fine: [total_chunks][kAttnSplits][H][2])
   uint16_t *out;
   int max_pages, H, Hkv, G;
   float qk_scale;  // scale * log2(e)
@@ -196,8 +208,57 @@ __device__ uint64_t g_attn_stamps[kAttnStampSlots][8];
   } while (0)
 #endif
 
-template <int WS>
-__global__ __launch_bounds__(512) void paged_attn_kernel(const AttnArgs a) {
+// A merged state of one q head's keys: the lane's 32 of O^T, the running max and the sum over every lane
+// group.  add() merges the state (o, m, l) of the next keys; each step is written as one operation, so that
+// every kernel that merges gets the same bits.
+struct AttnState {
+  f32x4 O[8];
+  float M, L;
+  __device__ __forceinline__ void clear() {
+    M = -INFINITY;
+    L = 0.0f;
+#pragma unroll
+    for (int cc = 0; cc < 8; cc++) O[cc] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  __device__ __forceinline__ void add(const f32x4 (&o)[8], float m, float l) {
+    const float mn = fmaxf(M, m);  // (a state added holds a key: mn is finite)
+    const float f0 = exp2f(M - mn), f1 = exp2f(m - mn);
+#pragma unroll
+    for (int cc = 0; cc < 8; cc++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) O[cc][i] = __builtin_fmaf(o[cc][i], f1, O[cc][i] * f0);
+    L = __builtin_fmaf(l, f1, L * f0);
+    M = mn;
+  }
+  // as a wave's LDS slot [kStateFloats][64]
+  __device__ __forceinline__ void put(float *st) const {
+#pragma unroll
+    for (int cc = 0; cc < 8; cc++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) st[(4 * cc + i) * 64] = O[cc][i];
+    st[32 * 64] = M;
+    st[33 * 64] = L;
+  }
+  __device__ __forceinline__ void add_slot(const float *st) {
+    f32x4 o[8];
+#pragma unroll
+    for (int cc = 0; cc < 8; cc++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) o[cc][i] = st[(4 * cc + i) * 64];
+    add(o, st[32 * 64], st[33 * 64]);
+  }
+};
+
+// How a launch splits a plan (the results are the same bits):
+//   coarse: a workgroup a chunk and hb kv heads, kAttnSplits waves a head, each walking a group's sub-runs;
+//   FINE: a workgroup a group and kv head, a wave a sub-run; its state is a partial of the merge.
+// One CU reads at about 46 GB/s however many waves or loads ahead it has, 25 GB/s when all of them read: a
+// plan of few chunks is bound by the CUs it reaches, so it takes more and smaller workgroups (attn_split).
+constexpr int attn_waves(bool fine) { return fine ? kSubs : kAttnSplits; }
+
+template <bool FINE>
+__global__ __launch_bounds__(FINE ? 64 * kSubs : 512) void paged_attn_kernel(const AttnArgs a) {
+  constexpr int WS = attn_waves(FINE);
 #if JIT_ATTN_STAMPS
   uint64_t ts[5] = {__builtin_amdgcn_s_memrealtime(), 0, 0, 0, 0};
   auto stamp_out = [&]() {
@@ -211,9 +272,8 @@ __global__ __launch_bounds__(512) void paged_attn_kernel(const AttnArgs a) {
     }
   };
 #endif
-  static_assert(WS == kAttnSplits, "the chunk rule rounds to whole 32-key steps of each of WS waves");
   extern __shared__ float xstate[];  // [WS - 1][hb][kStateFloats][64]
-  const int gc = blockIdx.x;
+  const int gc = FINE ? blockIdx.x / kAttnSplits : blockIdx.x, group = FINE ? blockIdx.x % kAttnSplits : 0;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id();
   const int hb = a.hb;
   const int kvl = wave % hb, split = wave / hb;
@@ -222,12 +282,20 @@ __global__ __launch_bounds__(512) void paged_attn_kernel(const AttnArgs a) {
   const int b = a.chunk_seq[gc];
   const int L = a.lens[b];
   const int c = gc - a.chunk_start[b];
-  const int ck = chunk_tokens(L), kRun = ck / WS;
+  const int ck = FINE ? kChunk : chunk_tokens(L), kRun = FINE ? kSubRun : ck / WS;
   const int nchunks = (L + ck - 1) / ck;
   const int lr = l & 15, lg = l >> 4;
   const int G = a.G;
-  const int wk0 = c * ck + split * kRun;
-  const int wk1 = min(c * ck + (split + 1) * kRun, L);
+  const int b0 = c * ck + group * kGroup, b1 = min(FINE ? b0 + kGroup : b0 + ck, L);  // the workgroup's keys
+  if (FINE && b0 >= L) {  // a group without keys (the last chunk's): an empty partial (uniform)
+    if ((int)threadIdx.x < G) {
+      const long long r = (long long)blockIdx.x * a.H + kvh * G + threadIdx.x;
+      *(float2 *)(a.part_ml + r * 2) = make_float2(-INFINITY, 0.0f);
+    }
+    return;
+  }
+  const int wk0 = b0 + split * kRun;
+  const int wk1 = min(wk0 + kRun, b1);
   const int npg = wk1 > wk0 ? (wk1 - wk0 + kPage - 1) / kPage : 0;  // split 0 always holds a key
   const int nst = live ? (npg + 1) >> 1 : 0;                          // 32-key steps
   // the run's page ids, one per lane (at most kRun / 16 <= 64)
@@ -273,7 +341,7 @@ __global__ __launch_bounds__(512) void paged_attn_kernel(const AttnArgs a) {
     const uint16_t *row = a.qkv + (long long)b * nh * kD;
     uint16_t *qs = (uint16_t *)(xstate + (WS - 1) * hb * kStateFloats * 64);  // [hb][G][128], past the states
     constexpr int kQHeads = (16 + WS - 1) / WS;  // q heads a wave norms (G <= 16)
-    const bool writer = live && c == nchunks - 1 && split < 2;  // the token's K (split 0) or V (split 1)
+    const bool writer = live && c == nchunks - 1 && b1 == L && split < 2;  // the token's K (split 0) or V (split 1)
     uint16_t qx[kQHeads][2], tx[2] = {0, 0}, qw[2] = {0, 0}, kw[2] = {0, 0};
     float fr = 0.0f;
     int pg = 0;
@@ -348,7 +416,32 @@ __global__ __launch_bounds__(512) void paged_attn_kernel(const AttnArgs a) {
   asm volatile("" ::: "memory");
   ATTN_STAMP(1);
 #endif
-  for (int st = 0; st < nst; st++) {
+  AttnState S;  // the sub-runs so far
+  S.clear();
+  bool first = true;
+  // the end of a sub-run: its state joins S (the first is S) and the next one starts afresh
+  auto flush = [&]() {
+    const float l_sub = sum_xor32(sum_xor16(l_run));
+    if (first) {
+#pragma unroll
+      for (int cc = 0; cc < 8; cc++) S.O[cc] = o[cc];
+      S.M = m_run;
+      S.L = l_sub;
+    } else {
+      S.add(o, m_run, l_sub);
+    }
+    first = false;
+    m_run = -INFINITY;
+    l_run = 0.0f;
+#pragma unroll
+    for (int cc = 0; cc < 8; cc++) o[cc] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  const bool subs = !FINE && ck == kChunk;
+  // One step; MORE: another follows, whose K and V are requested here.  (The run's last step is a copy of its
+  // own without the requests: behind a branch in one body they would make the waits before P.V count no load
+  // in flight, and requested for nothing they cost a step's reads and hold the registers of the merge below.)
+  auto step = [&](const int st, auto more) {
+    constexpr bool MORE = decltype(more)::value;
     const int k0 = wk0 + 32 * st;
     f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -357,7 +450,7 @@ __global__ __launch_bounds__(512) void paged_attn_kernel(const AttnArgs a) {
       s1 = mfma16x16x32(kf[1][cc], qf[cc], s1);
     }
     // K registers are free: the next step's K is in flight during softmax and P.V
-    load_k2(kf, a.pool, a.Hkv, kvh, page(2 * st + 2), page(2 * st + 3), lr, lg);
+    if constexpr (MORE) load_k2(kf, a.pool, a.Hkv, kvh, page(2 * st + 2), page(2 * st + 3), lr, lg);
     // keys past the run are masked on its last step only; the scale is applied inside the
     // exponent's fma (the max of the raw scores times the positive scale is the scaled max)
     float p0[4], p1[4];
@@ -387,7 +480,7 @@ __global__ __launch_bounds__(512) void paged_attn_kernel(const AttnArgs a) {
       p1[i] = __builtin_amdgcn_exp2f(fmaf(p1[i], a.qk_scale, -m_new));
       psum += p0[i] + p1[i];
     }
-    l_run = l_run * alpha + psum;
+    l_run = __builtin_fmaf(l_run, alpha, psum);
     m_run = m_new;
     // P^T fragments (B operand): head lr, k slots 8*lg + j = key 4*lg + j of the first
     // page (j < 4) and of the second (j >= 4) -- the lane's own probabilities, as bf16
@@ -432,66 +525,49 @@ __global__ __launch_bounds__(512) void paged_attn_kernel(const AttnArgs a) {
     }
 #pragma unroll
     for (int cc = 0; cc < 8; cc++) o[cc] = mfma16x16x32(vf[cc], pl, o[cc]);
-    load_v2(vv, a.pool, a.Hkv, kvh, page(2 * st + 2), page(2 * st + 3), lr, lg);
+    if constexpr (MORE) load_v2(vv, a.pool, a.Hkv, kvh, page(2 * st + 2), page(2 * st + 3), lr, lg);
     // keep these loads in this step: sunk into the next step they would only be
     // issued once that step's K has arrived
     asm volatile("" ::: "memory");
+    if (MORE && subs && (st + 1) % (kSubRun / 32) == 0) flush();  // (uniform)
+  };
+  for (int st = 0; st + 1 < nst; st++) step(st, std::true_type{});
+  if (nst > 0) {
+    step(nst - 1, std::false_type{});
+    flush();
   }
   ATTN_STAMP(2);
-  if (WS > 1) {  // the splits' states meet: split 0 of each kv head adds splits 1.. in order
-    if (split > 0) {
-      float *st = xstate + (((split - 1) * hb + kvl) * kStateFloats) * 64 + l;
+  // the waves' states meet in LDS: split 0 of each kv head adds the others in order (the sub-runs of a group
+  // as far as they hold keys, as a wave that walks them does; every group of a chunk)
+  auto slot = [&](int sp) { return xstate + (((sp - 1) * hb + kvl) * kStateFloats) * 64 + l; };
+  if (split > 0) S.put(slot(split));
+  __syncthreads();
+  if (split == 0)
 #pragma unroll
-      for (int cc = 0; cc < 8; cc++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) st[(4 * cc + i) * 64] = o[cc][i];
-      st[32 * 64] = m_run;
-      st[33 * 64] = l_run;
-    }
-    __syncthreads();
-    ATTN_STAMP(3);
-    if (split > 0 || !live) return;
-#pragma unroll
-    for (int sp = 1; sp < WS; sp++) {
-      const float *st = xstate + (((sp - 1) * hb + kvl) * kStateFloats) * 64 + l;
-      const float m2 = st[32 * 64], l2 = st[33 * 64];
-      const float M = fmaxf(m_run, m2);  // split 0 holds a key: M is finite
-      const float f0 = exp2f(m_run - M), f1 = exp2f(m2 - M);
-#pragma unroll
-      for (int cc = 0; cc < 8; cc++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) o[cc][i] = o[cc][i] * f0 + st[(4 * cc + i) * 64] * f1;
-      l_run = l_run * f0 + l2 * f1;
-      m_run = M;
-    }
-  } else if (!live) {
-    return;
-  }
+    for (int sp = 1; sp < WS; sp++)
+      if (!FINE || b0 + sp * kRun < b1) S.add_slot(slot(sp));
+  ATTN_STAMP(3);
+  if (split > 0 || !live) return;
 #if JIT_ATTN_STAMPS
   if (wave == 0) stamp_out();
 #endif
-  // per-head sum over the four lane groups
-  const float l_tot = sum_xor32(sum_xor16(l_run));
   if (lr >= G) return;
   const long long row = (long long)b * a.H + kvh * G + lr;  // this lane's q head
-  if (nchunks == 1) {
-    const float inv = 1.0f / l_tot;
+  if (!FINE && nchunks == 1) {
+    const float inv = 1.0f / S.L;
 #pragma unroll
     for (int cc = 0; cc < 8; cc++) {
       uint2 w;
-      w.x = pack_bf16x2(o[cc][0] * inv, o[cc][1] * inv);
-      w.y = pack_bf16x2(o[cc][2] * inv, o[cc][3] * inv);
+      w.x = pack_bf16x2(S.O[cc][0] * inv, S.O[cc][1] * inv);
+      w.y = pack_bf16x2(S.O[cc][2] * inv, S.O[cc][3] * inv);
       *(uint2 *)(a.out + row * kD + 16 * cc + 4 * lg) = w;
     }
   } else {
-    const long long r = (long long)gc * a.H + kvh * G + lr;
+    const long long r = (long long)blockIdx.x * a.H + kvh * G + lr;
 #pragma unroll
     for (int cc = 0; cc < 8; cc++)
-      *(float4 *)(a.part_o + r * kD + 16 * cc + 4 * lg) = make_float4(o[cc][0], o[cc][1], o[cc][2], o[cc][3]);
-    if (lg == 0) {
-      a.part_ml[r * 2 + 0] = m_run;
-      a.part_ml[r * 2 + 1] = l_tot;
-    }
+      *(float4 *)(a.part_o + r * kD + 16 * cc + 4 * lg) = make_float4(S.O[cc][0], S.O[cc][1], S.O[cc][2], S.O[cc][3]);
+    if (lg == 0) *(float2 *)(a.part_ml + r * 2) = make_float2(S.M, S.L);
   }
 }
 
@@ -502,8 +578,11 @@ __global__ __launch_bounds__(512) void paged_attn_kernel(const AttnArgs a) {
 // instead of one per chunk in a serial chain.  Lane j merges chunks j, j + 16, ...
 // online (running max, one pass over the partials), and the 16 lane states are
 // merged in lane order: a fixed order that depends only on the sequence's chunk count.
+// FINE: a chunk's partial is first put together from its groups', in order and with AttnState's operations
+// (group 0 always holds a key; a group without one left (-inf, 0)).
 constexpr int kMergeLanes = 16;
 
+template <bool FINE>
 __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t *__restrict__ chunk_start,
                                                          const float *__restrict__ part_o,
                                                          const float *__restrict__ part_ml, int H,
@@ -513,7 +592,7 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t *__restri
   // lens[b] and then the prefix were two round trips in a row; the plan is lens' chunk split)
   const long long c0 = chunk_start[b];
   const int n = chunk_start[b + 1] - (int)c0;
-  if (n <= 1) return;
+  if (FINE ? n < 1 : n <= 1) return;
   __shared__ float4 s_o[kMergeLanes][32];
   __shared__ float s_m[kMergeLanes], s_l[kMergeLanes];
   const int cl = t >> 5, dq = t & 31;
@@ -522,20 +601,55 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t *__restri
   // four iterations' loads go out together (bs = 1's 128 chunks, 8 a lane: attention 88.6 -> 88.1-88.3
   // us; 2 before).  8 would take the kernel past 64 VGPRs, one wave a SIMD fewer, and cost config 2's
   // 1,024 merge workgroups 0.7 us.  The arithmetic and its order are the same at any unroll.
-#pragma unroll 4
+#pragma unroll(FINE ? 1 : 4)
   for (int c = cl; c < n; c += kMergeLanes) {
-    const long long r = (c0 + c) * H + h;
-    const float2 ml = *(const float2 *)(part_ml + r * 2);
-    const float4 o = *(const float4 *)(part_o + r * kD + 4 * dq);
+    float2 ml;
+    float4 o;
+    if constexpr (FINE) {
+      float2 gm[kAttnSplits];
+      float4 go[kAttnSplits];
+#pragma unroll
+      for (int w = 0; w < kAttnSplits; w++) {
+        const long long r = ((c0 + c) * kAttnSplits + w) * H + h;
+        gm[w] = *(const float2 *)(part_ml + r * 2);
+        go[w] = *(const float4 *)(part_o + r * kD + 4 * dq);
+      }
+      ml = gm[0];
+      o = go[0];
+#pragma unroll
+      for (int w = 1; w < kAttnSplits; w++) {
+        if (gm[w].y == 0.0f && gm[w].x == -INFINITY) go[w] = make_float4(0.f, 0.f, 0.f, 0.f);  // (nothing was stored)
+        const float mg = fmaxf(ml.x, gm[w].x);
+        const float f0 = exp2f(ml.x - mg), f1 = exp2f(gm[w].x - mg);
+        o.x = __builtin_fmaf(go[w].x, f1, o.x * f0);
+        o.y = __builtin_fmaf(go[w].y, f1, o.y * f0);
+        o.z = __builtin_fmaf(go[w].z, f1, o.z * f0);
+        o.w = __builtin_fmaf(go[w].w, f1, o.w * f0);
+        ml = make_float2(mg, __builtin_fmaf(gm[w].y, f1, ml.y * f0));
+      }
+      if (n == 1) {  // the whole result (chunk lane 0 alone is here)
+        const float inv = 1.0f / ml.y;
+        uint2 w;
+        w.x = pack_bf16x2(o.x * inv, o.y * inv);
+        w.y = pack_bf16x2(o.z * inv, o.w * inv);
+        *(uint2 *)(out + ((long long)b * H + h) * kD + 4 * dq) = w;
+        break;
+      }
+    } else {
+      const long long r = (c0 + c) * H + h;
+      ml = *(const float2 *)(part_ml + r * 2);
+      o = *(const float4 *)(part_o + r * kD + 4 * dq);
+    }
     const float mn = fmaxf(m_run, ml.x);
     const float fa = exp2f(m_run - mn), fb = exp2f(ml.x - mn);
-    Ls = Ls * fa + ml.y * fb;
-    O.x = O.x * fa + o.x * fb;
-    O.y = O.y * fa + o.y * fb;
-    O.z = O.z * fa + o.z * fb;
-    O.w = O.w * fa + o.w * fb;
+    Ls = __builtin_fmaf(ml.y, fb, Ls * fa);
+    O.x = __builtin_fmaf(o.x, fb, O.x * fa);
+    O.y = __builtin_fmaf(o.y, fb, O.y * fa);
+    O.z = __builtin_fmaf(o.z, fb, O.z * fa);
+    O.w = __builtin_fmaf(o.w, fb, O.w * fa);
     m_run = mn;
   }
+  if (FINE && n == 1) return;  // (uniform)
   s_o[cl][dq] = O;
   if (dq == 0) {
     s_m[cl] = m_run;
@@ -552,11 +666,11 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t *__restri
   for (int j = 0; j < kMergeLanes; j++) {  // lanes without a chunk hold m = -inf: weight 0
     const float f = exp2f(s_m[j] - M);
     const float4 v = s_o[j][t];
-    acc.x += v.x * f;
-    acc.y += v.y * f;
-    acc.z += v.z * f;
-    acc.w += v.w * f;
-    lsum += s_l[j] * f;
+    acc.x = __builtin_fmaf(v.x, f, acc.x);
+    acc.y = __builtin_fmaf(v.y, f, acc.y);
+    acc.z = __builtin_fmaf(v.z, f, acc.z);
+    acc.w = __builtin_fmaf(v.w, f, acc.w);
+    lsum = __builtin_fmaf(s_l[j], f, lsum);
   }
   const float inv = 1.0f / lsum;
   uint2 w;
@@ -1023,8 +1137,25 @@ extern "C" int jit_attn_plan(const int32_t *lens_host, int B, int32_t *chunk_sta
   return total;
 }
 
+namespace {
+// Whether a plan of total_chunks chunks takes the fine split (given a workspace for its partials): up to
+// 192 chunks x kv heads, i.e. while the coarse split with one kv head a workgroup leaves CUs without
+// one.  Kernel + merge at Hkv = 4, us, before (two kv heads a workgroup) / one kv head a workgroup / fine: 1
+// sequence of 1,536 keys 33.9 / 18.1 / 10.7, of 4,096 keys 36.9 / 22.2 / 12.1, of 32,768 keys 40.3 / 25.0 / 20.0; 8
+// of 4,096 40.0 / 26.8 / 20.2; 48 chunks 42.7 / 28.5 / 28.5, 56 chunks 41.9 / 27.0 / 29.2.
+constexpr int kFewWorkgroups = 256;
+constexpr int kMaxFineChunks = 118;  // (a sequence of longer chunks, which has no groups, has at least 119)
+bool attn_fine(int total_chunks, int Hkv) {
+  return total_chunks <= kMaxFineChunks && (long long)total_chunks * Hkv <= 192;
+}
+}  // namespace
+
 extern "C" int64_t jit_attn_workspace_bytes(int total_chunks, int H) {
   return (int64_t)total_chunks * H * (kD + 2) * (int64_t)sizeof(float);
+}
+
+extern "C" int64_t jit_attn_split_workspace_bytes(int total_chunks, int H, int Hkv) {
+  return (attn_fine(total_chunks, Hkv) ? kAttnSplits : 1) * jit_attn_workspace_bytes(total_chunks, H);
 }
 
 namespace {
@@ -1041,12 +1172,19 @@ struct FusedQkv {
 
 int decode_attn_launch(const uint16_t *q, const uint16_t *pool, const int32_t *page_table, int max_pages,
                        const int32_t *lens, const int32_t *chunk_start, const int32_t *chunk_seq, int B, int H,
-                       int Hkv, float scale, int total_chunks, void *workspace, uint16_t *out, hipStream_t st,
-                       const char *what, const FusedQkv *fq = nullptr) {
+                       int Hkv, float scale, int total_chunks, void *workspace, int64_t workspace_bytes, uint16_t *out,
+                       hipStream_t st, const char *what, const FusedQkv *fq = nullptr) {
+  const bool fine =
+      attn_fine(total_chunks, Hkv) && workspace_bytes >= jit_attn_split_workspace_bytes(total_chunks, H, Hkv);
+  const int slots = total_chunks * (fine ? kAttnSplits : 1);
   float *part_o = (float *)workspace;
-  float *part_ml = part_o + (long long)total_chunks * H * kD;
-  constexpr int WS = kAttnSplits;
-  const int hb = Hkv < kAttnHeadsPerBlock ? Hkv : kAttnHeadsPerBlock;  // kv heads per workgroup (WS waves each)
+  float *part_ml = part_o + (long long)slots * H * kD;
+  const int WS = attn_waves(fine);
+  // kv heads per workgroup (WS waves each): one while that leaves no CU with two workgroups (64 chunks of
+  // 1,500 keys at Hkv = 4: 43.9 -> 37.6 us; 66 chunks 45.2 -> 50.5)
+  const int hb = fine || (long long)total_chunks * Hkv <= kFewWorkgroups
+                     ? 1
+                     : (Hkv < kAttnHeadsPerBlock ? Hkv : kAttnHeadsPerBlock);
   AttnArgs a{q, pool, page_table, lens, chunk_start, chunk_seq, part_o, part_ml, out,
              max_pages, H, Hkv, H / Hkv, scale * 1.44269504088896341f, hb,
              fq ? fq->qkv : nullptr, fq ? fq->q_norm_w : nullptr, fq ? fq->k_norm_w : nullptr,
@@ -1054,10 +1192,17 @@ int decode_attn_launch(const uint16_t *q, const uint16_t *pool, const int32_t *p
   // the splits' states, and with fq the staged q heads of the workgroup's kv heads
   const size_t lds = (size_t)(WS - 1) * hb * kStateFloats * 64 * sizeof(float) +
                      (fq ? (size_t)hb * (H / Hkv) * kD * sizeof(uint16_t) : 0);
-  paged_attn_kernel<WS><<<dim3(total_chunks, (Hkv + hb - 1) / hb), 64 * hb * WS, lds, st>>>(a);
+  const dim3 grid(slots, (Hkv + hb - 1) / hb);
+  if (fine)
+    paged_attn_kernel<true><<<grid, 64 * WS, lds, st>>>(a);
+  else
+    paged_attn_kernel<false><<<grid, 64 * hb * WS, lds, st>>>(a);
   int rc = jit::check_launch(what);
   if (rc) return rc;
-  attn_merge_kernel<<<dim3(B, H), 512, 0, st>>>(chunk_start, part_o, part_ml, H, out);
+  if (fine)
+    attn_merge_kernel<true><<<dim3(B, H), 512, 0, st>>>(chunk_start, part_o, part_ml, H, out);
+  else
+    attn_merge_kernel<false><<<dim3(B, H), 512, 0, st>>>(chunk_start, part_o, part_ml, H, out);
   return jit::check_launch(what);
 }
 
@@ -1105,18 +1250,52 @@ int scratch_of_current_device(void **ptr, const char *what) {
 
 }  // namespace
 
-extern "C" int jit_paged_decode_attn(const uint16_t *q, const uint16_t *pool,
-                                     const int32_t *page_table, int max_pages, const int32_t *lens,
-                                     const int32_t *chunk_start, const int32_t *chunk_seq, int B,
-                                     int H, int Hkv, float scale, int total_chunks, void *workspace,
-                                     uint16_t *out, void *stream) {
+extern "C" int jit_paged_decode_attn_ws(const uint16_t *q, const uint16_t *pool, const int32_t *page_table,
+                                        int max_pages, const int32_t *lens, const int32_t *chunk_start,
+                                        const int32_t *chunk_seq, int B, int H, int Hkv, float scale,
+                                        int total_chunks, void *workspace, int64_t workspace_bytes, uint16_t *out,
+                                        void *stream) {
   int rc = decode_attn_contract(B, H, Hkv, max_pages, total_chunks, "paged_decode_attn");
   if (rc) return rc;
   if (B == 0 || total_chunks == 0) return JIT_OK;
+  if (workspace_bytes < jit_attn_workspace_bytes(total_chunks, H))
+    return jit::fail(JIT_EINVAL, "paged_decode_attn: workspace of %lld bytes for %d chunks of %d heads",
+                     (long long)workspace_bytes, total_chunks, H);
   if (!q || !pool || !page_table || !lens || !chunk_start || !chunk_seq || !workspace || !out)
     return jit::fail(JIT_EINVAL, "paged_decode_attn: null pointer");
   return decode_attn_launch(q, pool, page_table, max_pages, lens, chunk_start, chunk_seq, B, H, Hkv, scale,
-                            total_chunks, workspace, out, (hipStream_t)stream, "jit_paged_decode_attn");
+                            total_chunks, workspace, workspace_bytes, out, (hipStream_t)stream,
+                            "jit_paged_decode_attn");
+}
+
+extern "C" int jit_paged_decode_attn(const uint16_t *q, const uint16_t *pool, const int32_t *page_table,
+                                     int max_pages, const int32_t *lens, const int32_t *chunk_start,
+                                     const int32_t *chunk_seq, int B, int H, int Hkv, float scale, int total_chunks,
+                                     void *workspace, uint16_t *out, void *stream) {
+  return jit_paged_decode_attn_ws(q, pool, page_table, max_pages, lens, chunk_start, chunk_seq, B, H, Hkv, scale,
+                                  total_chunks, workspace, jit_attn_workspace_bytes(total_chunks, H), out, stream);
+}
+
+extern "C" int jit_paged_decode_attn_qkv_ws(const uint16_t *qkv, const uint16_t *q_norm_w, const uint16_t *k_norm_w,
+                                            float eps, const float *inv_freq, uint16_t *pool,
+                                            const int32_t *page_table, int max_pages, const int32_t *lens,
+                                            const int32_t *chunk_start, const int32_t *chunk_seq, int B, int H,
+                                            int Hkv, float scale,
+                                            int total_chunks, void *workspace, int64_t workspace_bytes,
+                                            uint16_t *out, void *stream) {
+  int rc = decode_attn_contract(B, H, Hkv, max_pages, total_chunks, "paged_decode_attn_qkv");
+  if (rc) return rc;
+  if (B == 0 || total_chunks == 0) return JIT_OK;
+  if (workspace_bytes < jit_attn_workspace_bytes(total_chunks, H))
+    return jit::fail(JIT_EINVAL, "paged_decode_attn_qkv: workspace of %lld bytes for %d chunks of %d heads",
+                     (long long)workspace_bytes, total_chunks, H);
+  if (!qkv || !q_norm_w || !k_norm_w || !inv_freq || !pool || !page_table || !lens || !chunk_start || !chunk_seq ||
+      !workspace || !out)
+    return jit::fail(JIT_EINVAL, "paged_decode_attn_qkv: null pointer");
+  const FusedQkv fq{qkv, q_norm_w, k_norm_w, inv_freq, eps};
+  return decode_attn_launch(nullptr, pool, page_table, max_pages, lens, chunk_start, chunk_seq, B, H, Hkv, scale,
+                            total_chunks, workspace, workspace_bytes, out, (hipStream_t)stream,
+                            "jit_paged_decode_attn_qkv", &fq);
 }
 
 extern "C" int jit_paged_decode_attn_qkv(const uint16_t *qkv, const uint16_t *q_norm_w, const uint16_t *k_norm_w,
@@ -1124,15 +1303,9 @@ extern "C" int jit_paged_decode_attn_qkv(const uint16_t *qkv, const uint16_t *q_
                                          int max_pages, const int32_t *lens, const int32_t *chunk_start,
                                          const int32_t *chunk_seq, int B, int H, int Hkv, float scale,
                                          int total_chunks, void *workspace, uint16_t *out, void *stream) {
-  int rc = decode_attn_contract(B, H, Hkv, max_pages, total_chunks, "paged_decode_attn_qkv");
-  if (rc) return rc;
-  if (B == 0 || total_chunks == 0) return JIT_OK;
-  if (!qkv || !q_norm_w || !k_norm_w || !inv_freq || !pool || !page_table || !lens || !chunk_start || !chunk_seq ||
-      !workspace || !out)
-    return jit::fail(JIT_EINVAL, "paged_decode_attn_qkv: null pointer");
-  const FusedQkv fq{qkv, q_norm_w, k_norm_w, inv_freq, eps};
-  return decode_attn_launch(nullptr, pool, page_table, max_pages, lens, chunk_start, chunk_seq, B, H, Hkv, scale,
-                            total_chunks, workspace, out, (hipStream_t)stream, "jit_paged_decode_attn_qkv", &fq);
+  return jit_paged_decode_attn_qkv_ws(qkv, q_norm_w, k_norm_w, eps, inv_freq, pool, page_table, max_pages, lens,
+                                      chunk_start, chunk_seq, B, H, Hkv, scale, total_chunks, workspace,
+                                      jit_attn_workspace_bytes(total_chunks, H), out, stream);
 }
 
 extern "C" int jit_paged_decode_attn_noalloc(const uint16_t *q, const uint16_t *pool, const int32_t *page_table,
@@ -1154,7 +1327,7 @@ extern "C" int jit_paged_decode_attn_noalloc(const uint16_t *q, const uint16_t *
   rc = scratch_of_current_device(&ws, "paged_decode_attn_noalloc");
   if (rc) return rc;
   return decode_attn_launch(q, pool, page_table, max_pages, lens, chunk_start, chunk_seq, B, H, Hkv, scale,
-                            total_chunks, ws, out, (hipStream_t)stream, "jit_paged_decode_attn_noalloc");
+                            total_chunks, ws, need, out, (hipStream_t)stream, "jit_paged_decode_attn_noalloc");
 }
 
 #if JIT_ATTN_STAMPS

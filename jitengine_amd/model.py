@@ -90,7 +90,8 @@ def make_step_state(cfg: MoEConfig, pos_host, page_table: torch.Tensor) -> StepS
     pos_host = np.asarray(pos_host, np.int32)
     dev = page_table.device
     plan = ops.attn_plan(pos_host + 1, dev)
-    ws = torch.empty(max(ops.attn_workspace_bytes(plan.total, cfg.heads), 4), dtype=torch.uint8, device=dev)
+    ws = torch.empty(max(ops.attn_split_workspace_bytes(plan.total, cfg.heads, cfg.kv_heads), 4), dtype=torch.uint8,
+                     device=dev)
     return StepState(ops.upload(pos_host, dev), page_table, plan, ws)
 
 
@@ -126,7 +127,8 @@ def make_mixed_state(cfg: MoEConfig, chunks, seq_table_host, dec_pos_host, dec_t
     table_rows = np.concatenate([np.stack(rows) if rows else np.zeros((0, dec_table_host.shape[1]), np.int32),
                                  dec_table_host]).astype(np.int32)
     dplan = ops.attn_plan(dec_pos + 1, device)
-    ws = torch.empty(max(ops.attn_workspace_bytes(dplan.total, cfg.heads), 4), dtype=torch.uint8, device=device)
+    ws = torch.empty(max(ops.attn_split_workspace_bytes(dplan.total, cfg.heads, cfg.kv_heads), 4), dtype=torch.uint8,
+                     device=device)
     # (pinned, asynchronous uploads: the host does not wait for the steps still queued)
     return MixedState(P, ops.upload(pos_rows, device), ops.upload(table_rows, device),
                       ops.upload(seq_table_host, device), ops.prefill_plan(chunks, cfg.heads, cfg.kv_heads, device),

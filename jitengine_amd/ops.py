@@ -632,6 +632,19 @@ def attn_workspace_bytes(total_chunks: int, H: int) -> int:
     return int(_lib.lib().jit_attn_workspace_bytes(int(total_chunks), int(H)))
 
 
+def attn_split_workspace_bytes(total_chunks: int, H: int, Hkv: int) -> int:
+    """Workspace bytes with which decode attention runs a plan of few chunks on more workgroups (the same
+    bits; any workspace of attn_workspace_bytes or more serves)."""
+    return int(_lib.lib().jit_attn_split_workspace_bytes(int(total_chunks), int(H), int(Hkv)))
+
+
+def _attn_workspace(workspace, plan, H: int, Hkv: int, device) -> torch.Tensor:
+    """The caller's workspace if the plan's partials fit it, else a new one."""
+    if workspace is not None and workspace.numel() * workspace.element_size() >= attn_workspace_bytes(plan.total, H):
+        return workspace
+    return torch.empty(max(attn_split_workspace_bytes(plan.total, H, Hkv), 4), dtype=torch.uint8, device=device)
+
+
 @dataclass
 class PrefillPlan:
     """Chunks (seq, ctx, length) of a prefill step in q-row order and their work items for
@@ -731,14 +744,13 @@ def paged_decode_attention(q: torch.Tensor, pool: torch.Tensor, page_table: torc
                          f"{int((plan.lens_host.max() + PAGE - 1) // PAGE)}")
     if H % Hkv:
         raise ValueError(f"{H} query heads over a pool of {Hkv} kv heads")
-    need = attn_workspace_bytes(plan.total, H)
-    if workspace is None or workspace.numel() * workspace.element_size() < need:
-        workspace = torch.empty(max(need, 4), dtype=torch.uint8, device=q.device)
+    workspace = _attn_workspace(workspace, plan, H, Hkv, q.device)
     out = torch.empty_like(q)
     _lib.check(
-        _lib.lib().jit_paged_decode_attn(
+        _lib.lib().jit_paged_decode_attn_ws(
             _p(q), _p(pool), _p(page_table), page_table.shape[1], _p(plan.lens), _p(plan.chunk_start),
-            _p(plan.chunk_seq), B, H, Hkv, float(scale), plan.total, _p(workspace), _p(out), _stream(),
+            _p(plan.chunk_seq), B, H, Hkv, float(scale), plan.total, _p(workspace),
+            workspace.numel() * workspace.element_size(), _p(out), _stream(),
         ),
         "paged_decode_attn",
     )
@@ -763,15 +775,13 @@ def paged_decode_attention_qkv(qkv: torch.Tensor, H: int, Hkv: int, q_norm: torc
     if B and int((plan.lens_host.max() + PAGE - 1) // PAGE) > page_table.shape[1]:
         raise ValueError(f"page_table has {page_table.shape[1]} columns, the longest sequence needs "
                          f"{int((plan.lens_host.max() + PAGE - 1) // PAGE)}")
-    need = attn_workspace_bytes(plan.total, H)
-    if workspace is None or workspace.numel() * workspace.element_size() < need:
-        workspace = torch.empty(max(need, 4), dtype=torch.uint8, device=qkv.device)
+    workspace = _attn_workspace(workspace, plan, H, Hkv, qkv.device)
     out = torch.empty((B, H, HEAD_DIM), dtype=torch.bfloat16, device=qkv.device)
     _lib.check(
-        _lib.lib().jit_paged_decode_attn_qkv(
+        _lib.lib().jit_paged_decode_attn_qkv_ws(
             _p(qkv), _p(q_norm), _p(k_norm), float(eps), _p(inv_freq), _p(pool), _p(page_table), page_table.shape[1],
             _p(plan.lens), _p(plan.chunk_start), _p(plan.chunk_seq), B, H, Hkv, float(scale), plan.total,
-            _p(workspace), _p(out), _stream(),
+            _p(workspace), workspace.numel() * workspace.element_size(), _p(out), _stream(),
         ),
         "paged_decode_attn_qkv",
     )
