@@ -698,9 +698,7 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t *__restri
 constexpr int kPfWaves = 8, kPfTiles = 2;
 constexpr int kPfHalves = 4;                                           // 32-key halves of a step
 constexpr int kPfStages = 2;                                           // LDS ring depth (steps)
-constexpr int kPfChunks = kPfHalves * 4 * kPageHead * 2 / 1024 / kPfWaves;  // 1 KB chunks of a step per wave
-// each wave stages the K and V of one page per step (4 parts of 4 KB in 1 KB chunks)
-static_assert(kPfChunks == 8 && kPfWaves == 2 * kPfHalves, "one page per wave per step");
+constexpr int kPfPages = 2 * kPfHalves;  // pages of a step, each 8 chunks of 1 KB (K, then V)
 static_assert(kPfStages == 2, "the page-id prefetch below runs one step ahead of the staging");
 
 // Key parts.  A token's keys are cut at the fixed positions kPfPartKeys, 2 kPfPartKeys, ...
@@ -732,7 +730,12 @@ struct PrefillArgs {
   float qk_scale;             // scale * log2(e)
 };
 
-__global__ __launch_bounds__(64 * kPfWaves) void prefill_attn_kernel(const PrefillArgs a) {
+// A workgroup takes WAVES x TILES of a row block's kPfWaves x kPfTiles q tiles (a block's pieces are
+// workgroups of their own; rows are independent, so the bits do not depend on the cut).
+template <int WAVES, int TILES>
+__global__ __launch_bounds__(64 * WAVES) void prefill_attn_kernel(const PrefillArgs a) {
+  constexpr int kSub = kPfWaves * kPfTiles / (WAVES * TILES);  // workgroups a row block
+  constexpr int kPfTiles = TILES;
   // a ring of kPfStages steps of kPfHalves x 32 keys, each half K0, V0, K1, V1 of its two pages
   // (4 KB each), filled by direct global->LDS loads kPfStages - 1 steps ahead of the step
   // being computed
@@ -740,25 +743,26 @@ __global__ __launch_bounds__(64 * kPfWaves) void prefill_attn_kernel(const Prefi
   // one dimension, the kv heads of an item adjacent: the hardware dispatches workgroups in index
   // order, so the plan's longest-first order holds across the kv heads (a (item, kv head) grid
   // dispatched every item of kv head 0 before any of kv head 1)
-  const int item = blockIdx.x / a.Hkv, kvh = blockIdx.x % a.Hkv;
-  const int ch = a.blk_chunk[item], q0 = a.blk_q0[item], part = a.blk_part[item];
+  const int item = blockIdx.x / (kSub * a.Hkv), rest = blockIdx.x % (kSub * a.Hkv), kvh = rest % a.Hkv;
+  const int ch = a.blk_chunk[item], part = a.blk_part[item];
   const int seq = a.chunk_seq[ch], ctx = a.chunk_ctx[ch], len = a.chunk_len[ch], row0 = a.chunk_row[ch];
   const int G = a.G, TR = 16 / G, tpw = kPfTiles * TR;
+  const int q0 = a.blk_q0[item] + (rest / a.Hkv) * WAVES * tpw;
+  if (kSub > 1 && q0 >= len) return;  // (uniform)
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = lane_id();
   const int lr = l & 15, lg = l >> 4;
-  const int tlast = min(q0 + kPfWaves * tpw, len) - 1;  // the workgroup's last token
+  const int tlast = min(q0 + WAVES * tpw, len) - 1;     // the workgroup's last token
   const int kend = ctx + tlast + 1;                     // its keys: [0, kend)
   const int nst = (kend + 32 * kPfHalves - 1) / (32 * kPfHalves), npages = (kend + 15) >> 4;
   // this item's steps: part `part` of the keys (the plan makes an item only for parts that hold a
   // key of the block's last token)
   const int st0 = part * kPfPartSteps, st1 = min(nst, st0 + kPfPartSteps);
+  if (kSub > 1 && st0 >= st1) return;  // (uniform: an earlier piece of a block whose last token alone reaches the part)
   const int32_t *prow = a.page_table + (long long)seq * a.max_pages;
-  // wave w stages on step st page 2 kPfHalves st + w of the workgroup's keys (a page past the keys
-  // repeats the last one); lane i reads the page of wave i % kPfWaves, so that the ids stay in a
+  // wave w stages on step st pages kPfPages st + kPfPages / WAVES w .. of the workgroup's keys (a page past the
+  // keys repeats the last one); lane i reads the step's page i % kPfPages, so that the ids stay in a
   // vector register until the step that stages them reads its lane
-  auto pages_of_step = [&](int st) {
-    return prow[min(2 * kPfHalves * st + (l & (kPfWaves - 1)), npages - 1)];
-  };
+  auto pages_of_step = [&](int st) { return prow[min(kPfPages * st + (l & (kPfPages - 1)), npages - 1)]; };
 
   // the lane's q row in tile j: token t (clamped into the chunk), head kvh * G + lr % G
   int tok[kPfTiles];
@@ -785,26 +789,24 @@ __global__ __launch_bounds__(64 * kPfWaves) void prefill_attn_kernel(const Prefi
   for (int j = 0; j < kPfTiles; j++) tile_first[j] = ctx + min(q0 + wave * tpw + j * TR, len - 1);
   __syncthreads();
 
-  // staging of step st into stage st % kPfStages: chunk c = kPfChunks * wave + u (1 KB, one
-  // load instruction of the wave) of the step's four parts -- K of page 2st, V of page 2st, K of
-  // page 2st + 1, V of page 2st + 1 (a page past the keys repeats the last one: its slots are
-  // masked, and the steps past the end are loaded and never read, so every wave always has
-  // (kPfStages - 1) * kPfChunks loads issued after a step's own)
+  // staging of step st into stage st % kPfStages: chunk c = 8 page + u (1 KB, one load instruction of
+  // the wave) of the step's pages, K then V of each (a page past the keys repeats the last one: its slots
+  // are masked, and the steps past the end are loaded and never read)
   // The loads are issued from inline assembly: the compiler then keeps no track of them (its
   // own waits would otherwise include them before every LDS read, as it cannot tell the
   // stages apart), and the explicit waits below order them; its waits for other loads only
   // grow more conservative.
   const uint32_t kvs_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)&kvs[0][0];
-#define PF_STAGE(st, pv)                                                                               \
-  {                                                                                                    \
-  const int pg = __builtin_amdgcn_readlane(pv, wave);                                                  \
-  _Pragma("unroll") for (int u = 0; u < kPfChunks; u++) {                                              \
-    const int c = kPfChunks * wave + u, part = c >> 2;  /* part: K or V (part & 1) of page pg */       \
-    const uint16_t *src = head_part(a.pool, pg, a.Hkv, kvh) + (part & 1) * kPageHead + (c & 3) * 512 + 8 * l; \
-    const uint32_t dst = __builtin_amdgcn_readfirstlane(                                               \
-        kvs_lds + 2 * (((st) % kPfStages) * kPfHalves * 4 * kPageHead + 512 * c));                     \
+#define PF_STAGE(st, pv)                                                                                      \
+  _Pragma("unroll") for (int i = 0; i < kPfPages / WAVES; i++) {                                              \
+  const int pgi = kPfPages / WAVES * wave + i, pg = __builtin_amdgcn_readlane(pv, pgi);                       \
+  _Pragma("unroll") for (int u = 0; u < 8; u++) {                                                             \
+    const int c = 8 * pgi + u;  /* K or V: u >> 2 */                                                          \
+    const uint16_t *src = head_part(a.pool, pg, a.Hkv, kvh) + (u >> 2) * kPageHead + (u & 3) * 512 + 8 * l;   \
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(                                                      \
+        kvs_lds + 2 * (((st) % kPfStages) * kPfHalves * 4 * kPageHead + 512 * c));                            \
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(dst) : "memory", "m0"); \
-  }                                                                                                    \
+  }                                                                                                           \
   }
   // the q fragments have landed before the first staged load is issued: the compiler's waits
   // for them would otherwise sit inside the loop, where they would also wait for the staging
@@ -819,7 +821,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void prefill_attn_kernel(const Prefi
   int pv_next = pages_of_step(st0 + 1);
   // the wait that leaves the loads of the next kPfStages - 2 steps in flight, and no lgkm or
   // export wait (vmcnt is split over bits 3:0 and 15:14)
-  constexpr int kPfVm = (kPfStages - 2) * kPfChunks;
+  constexpr int kPfVm = (kPfStages - 2) * 8 * kPfPages / WAVES;
   constexpr int kPfWait = (kPfVm & 15) | ((kPfVm >> 4) << 14) | (7 << 4) | (15 << 8);
   for (int st = st0; st < st1; st++) {
     // this wave's loads of step st have landed and its reads of step st - 1 are done; after
@@ -840,7 +842,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void prefill_attn_kernel(const Prefi
     // (one more barrier, on that step only)
     if (k0 + 32 * kPfHalves > kend) {
       uint16_t *vst = kvs[st % kPfStages];
-      for (int e = tid; e < kPfHalves * 2 * kPageHead; e += 64 * kPfWaves) {
+      for (int e = tid; e < kPfHalves * 2 * kPageHead; e += 64 * WAVES) {
         const int slot = e % kPage, dim = (e / kPage) % kD, pgh = e / kPageHead;  // pgh: page 2 h + p of the step
         if (k0 + kPage * pgh + slot >= kend) vst[(2 * pgh + 1) * kPageHead + dim * kPage + slot] = 0;
       }
@@ -1095,7 +1097,19 @@ extern "C" int jit_paged_prefill_attn(const uint16_t *q, const uint16_t *pool, c
     return jit::fail(JIT_EINVAL, "paged_prefill_attn: null pointer");
   const PrefillArgs a{q, pool, page_table, blk_chunk, blk_q0, blk_part, chunk_seq, chunk_ctx, chunk_len, chunk_row,
                       out, (float *)workspace, max_pages, H, Hkv, H / Hkv, pmax, scale * 1.44269504088896341f};
-  prefill_attn_kernel<<<dim3(nblk * Hkv), 64 * kPfWaves, 0, (hipStream_t)stream>>>(a);
+  const hipStream_t st = (hipStream_t)stream;
+  // few work items leave CUs idle (a workgroup's LDS fills a CU): their row blocks are cut into 2 or 4
+  // workgroups while those fit the CUs in one round.  A step of 128 keys takes 5.0 us with 8 waves of two
+  // tiles, 3.0 with 8 of one and 2.4 with 4 of one (half and a quarter of the rows), so a cut that needs a second
+  // round loses.  512 rows after 1,843 keys (64 workgroups): 99 -> 49 us (8 x 1: 62, 4 x 2: 72); after 8,000 (128):
+  // 235 -> 145; 2 x 512 after up to 3,000: 138 -> 88.
+  const int wgs = nblk * Hkv, cus = jit::cu_count();
+  if (4 * wgs <= cus)
+    prefill_attn_kernel<4, 1><<<dim3(4 * wgs), 64 * 4, 0, st>>>(a);
+  else if (2 * wgs <= cus)
+    prefill_attn_kernel<8, 1><<<dim3(2 * wgs), 64 * 8, 0, st>>>(a);
+  else
+    prefill_attn_kernel<kPfWaves, kPfTiles><<<dim3(wgs), 64 * kPfWaves, 0, st>>>(a);
   int rc = jit::check_launch("jit_paged_prefill_attn");
   if (rc || pmax == 1 || max_len == 0) return rc;
   prefill_merge_kernel<<<dim3(max_len, C), 8 * H, 0, (hipStream_t)stream>>>(chunk_ctx, chunk_len, chunk_row,

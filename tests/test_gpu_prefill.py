@@ -234,3 +234,22 @@ def test_prefill_and_mixed_step_past_4096_pages():
     assert_attention_parity(attn[:30], ex_pre, what="mixed prefill rows")
     _, ex_dec = oracle.paged_decode_attn(qh[30:], pool_after, table[1:], np.array(dec_pos) + 1, SCALE, exact=True)
     assert_attention_parity(attn[30:], ex_dec, what="mixed decode row of 70,001 keys")
+
+
+@pytest.mark.parametrize("H,Hkv,ctx,n", [(32, 4, 0, 33), (32, 4, 6100, 75), (8, 8, 300, 259), (16, 1, 1000, 17),
+                                         (32, 4, 12287, 3)])
+def test_prefill_row_block_cuts_agree(H, Hkv, ctx, n):
+    """A plan of few work items cuts its row blocks into 4 or 2 workgroups: the same bits as whole blocks,
+    with partial blocks, the causal diagonal inside a piece, key parts only a block's last tokens reach,
+    and every size of a tile's token group.  The chunk is repeated until the plan fills the CUs."""
+    pool, table = _pool([ctx + n], seed=H + ctx, Hkv=Hkv)
+    q = normal_bf16((n, H, 128), seed=n)
+    items = ops.prefill_plan([(0, ctx, n)], H, Hkv, DEV).blocks.shape[1] * Hkv
+    whole = None
+    for copies in (257 // items + 1, max(1, 100 // items), 1):
+        got = _run(np.concatenate([q] * copies), pool, table, [(0, ctx, n)] * copies, H, Hkv).reshape(copies, n, H, 128)
+        whole = got[0] if whole is None else whole
+        for c in range(copies):
+            assert np.array_equal(got[c], whole), (copies, c)
+    want, exact = oracle.paged_prefill_attn(q, pool, table, [(0, ctx, n)], SCALE, exact=True)
+    assert_attention_parity(whole, exact, what="cut row blocks")
