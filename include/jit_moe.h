@@ -319,8 +319,8 @@ int jit_attn_plan(const int32_t *lens_host, int B, int32_t *chunk_start_host,
 /* Workspace bytes jit_paged_decode_attn needs for `total_chunks` chunks. */
 int64_t jit_attn_workspace_bytes(int total_chunks, int H);
 /* Workspace bytes with which jit_paged_decode_attn_ws / _qkv_ws take the finest split of a plan of
- * `total_chunks` chunks: a plan of few chunks is spread over four times the workgroups, each leaving
- * a partial; otherwise jit_attn_workspace_bytes. */
+ * `total_chunks` chunks: a plan of few chunks runs a workgroup a quarter chunk, each leaving a partial;
+ * otherwise jit_attn_workspace_bytes. */
 int64_t jit_attn_split_workspace_bytes(int total_chunks, int H, int Hkv);
 
 /* Paged GQA decode attention, one query per row: out[b, h] =
@@ -501,6 +501,49 @@ int jit_threefry_uniform(const uint32_t *keys, int B, float *u, void *stream);
  * page is copied.  A page id outside [0, num_pages) copies nothing. */
 int jit_kv_copy_pages(uint16_t *pool, int num_pages, int Hkv, const int32_t *src, const int32_t *dst, int n,
                       void *stream);
+
+/* ------------------------------------------------------------ whole layers --
+ * One decoder layer per call (Q36/model/model.py:65-80): the launches above, in their order, issued from
+ * native code.  All weights are packed matrices and stacks (jit_q4_prepack). */
+typedef struct {
+  int D, H, Hkv, E, k, I, norm_topk; /* hidden, heads, experts, top-k and its renormalisation, expert width */
+  float eps, scale;                  /* RMSNorm's eps, the attention scale */
+  const uint16_t *input_norm, *q_norm, *k_norm, *post_norm;
+  const float *inv_freq;
+  const void *qkv, *o, *router, *gate_up, *down;
+} jit_layer;
+
+/* The decode rows of a step: B sequences with their attention plan (jit_attn_plan) and workspace. */
+typedef struct {
+  int B, max_pages, total_chunks;
+  const int32_t *page_table, *lens, *chunk_start, *chunk_seq;
+  void *workspace;
+  int64_t workspace_bytes;
+} jit_decode_rows;
+
+/* The prompt rows of a mixed step (the first `rows` rows) with the arguments of jit_paged_prefill_attn, and
+ * pos [T], table_rows [T, table_rows_pages] of every row of the step (jit_qk_norm_rope_append). */
+typedef struct {
+  int rows, C, nblk, pmax, max_len, seq_pages, table_rows_pages;
+  const int32_t *pos, *table_rows, *seq_table;
+  const int32_t *chunk_seq, *chunk_ctx, *chunk_len, *chunk_row;
+  const int32_t *blk_chunk, *blk_q0, *blk_part;
+  void *workspace;
+} jit_prompt_rows;
+
+/* Scratch bytes of the two calls below for `rows` rows (256-byte aligned device memory). */
+int64_t jit_layer_scratch_bytes(const jit_layer *layer, int rows, int mixed);
+
+/* A decode step's layer: x [B, D] (xn: its normed rows, or NULL) -> y [B, D], and with next_norm also the
+ * rows normed for the next layer, xn_next.  One row: defer leaves the closing combine to the next layer,
+ * which takes this call's scratch as `prev` (x and xn unused, y and xn_next not written). */
+int jit_decode_layer(const jit_layer *layer, const jit_decode_rows *d, uint16_t *pool, const uint16_t *x,
+                     const uint16_t *xn, const void *prev, int defer, const uint16_t *next_norm,
+                     void *scratch, uint16_t *y, uint16_t *xn_next, void *stream);
+
+/* A mixed prompt + decode step's layer over x [T, D], T = p->rows + d->B -> y [T, D]. */
+int jit_mixed_layer(const jit_layer *layer, const jit_prompt_rows *p, const jit_decode_rows *d, uint16_t *pool,
+                    const uint16_t *x, void *scratch, uint16_t *y, void *stream);
 
 #ifdef __cplusplus
 }

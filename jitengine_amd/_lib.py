@@ -21,6 +21,31 @@ _P = ctypes.c_void_p
 _I = ctypes.c_int
 _F = ctypes.c_float
 
+_L = ctypes.c_int64
+
+
+class Layer(ctypes.Structure):
+    """jit_layer"""
+    _fields_ = [(n, _I) for n in ("D", "H", "Hkv", "E", "k", "I", "norm_topk")] + [("eps", _F), ("scale", _F)] + [
+        (n, _P) for n in ("input_norm", "q_norm", "k_norm", "post_norm", "inv_freq", "qkv", "o", "router", "gate_up",
+                          "down")]
+
+
+class DecodeRows(ctypes.Structure):
+    """jit_decode_rows"""
+    _fields_ = [(n, _I) for n in ("B", "max_pages", "total_chunks")] + [
+        (n, _P) for n in ("page_table", "lens", "chunk_start", "chunk_seq", "workspace")] + [("workspace_bytes", _L)]
+
+
+class PromptRows(ctypes.Structure):
+    """jit_prompt_rows"""
+    _fields_ = [(n, _I) for n in ("rows", "C", "nblk", "pmax", "max_len", "seq_pages", "table_rows_pages")] + [
+        (n, _P) for n in ("pos", "table_rows", "seq_table", "chunk_seq", "chunk_ctx", "chunk_len", "chunk_row",
+                          "blk_chunk", "blk_q0", "blk_part", "workspace")]
+
+
+_PL, _PD, _PP = ctypes.POINTER(Layer), ctypes.POINTER(DecodeRows), ctypes.POINTER(PromptRows)
+
 # name -> argtypes (restype int unless listed in _RESTYPES)
 _SIGNATURES = {
     "jit_last_error": [],
@@ -56,6 +81,9 @@ _SIGNATURES = {
     "jit_attn_plan": [_P, _I, _P, _P, _I],
     "jit_attn_workspace_bytes": [_I, _I],
     "jit_attn_split_workspace_bytes": [_I, _I, _I],
+    "jit_layer_scratch_bytes": [_PL, _I, _I],
+    "jit_decode_layer": [_PL, _PD, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P],
+    "jit_mixed_layer": [_PL, _PP, _PD, _P, _P, _P, _P, _P],
     "jit_paged_decode_attn_ws": [_P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _F, _I, _P, ctypes.c_int64, _P, _P],
     "jit_paged_decode_attn_qkv_ws": [_P, _P, _P, _F, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _F, _I, _P, ctypes.c_int64,
                                      _P, _P],
@@ -78,7 +106,7 @@ _SIGNATURES = {
     "jit_kv_copy_pages": [_P, _I, _I, _P, _P, _I, _P],
 }
 _RESTYPES = {"jit_last_error": ctypes.c_char_p, "jit_attn_workspace_bytes": ctypes.c_int64,
-             "jit_attn_split_workspace_bytes": ctypes.c_int64,
+             "jit_attn_split_workspace_bytes": ctypes.c_int64, "jit_layer_scratch_bytes": ctypes.c_int64,
              "jit_prefill_workspace_bytes": ctypes.c_int64,
              "jit_q4_packed_bytes": ctypes.c_int64, "jit_moe_pack_workspace_bytes": ctypes.c_int64,
              "jit_sampler_workspace_bytes": ctypes.c_int64}

@@ -31,6 +31,7 @@ ARCH = "gfx950"
 
 SOURCES = {
     "errors.cpp": [],
+    "layer.cpp": [],
     "router.hip": ["-ffp-contract=off"],
     "qmm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "qmm_seg.hip": [],

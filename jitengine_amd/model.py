@@ -11,12 +11,13 @@ no output gate and no shared expert.  Embedding and lm_head are outside the step
 
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 
 import numpy as np
 import torch
 
-from . import ops
+from . import _lib, ops
 from .moe import MoEBlock
 from .quant import QLinear, random_quantized
 
@@ -150,6 +151,27 @@ class DecoderLayer:
         self.moe = MoEBlock(w["router"], w["gate_up"], w["down"], cfg.top_k, cfg.norm_topk, prepack=prepack)
         self.inv_freq = torch.from_numpy(rope_inv_freq(cfg.rope_theta, cfg.head_dim)).to(self.input_norm.device)
 
+    def native(self):
+        """The layer as jit_decode_layer / jit_mixed_layer take it, or None where its weights are not all packed
+        matrices of the geometry (the op-by-op path then serves, and names what does not fit)."""
+        cfg, moe = self.cfg, self.moe
+        D, E, I, Hd = cfg.hidden, moe.num_experts, moe.down.in_dims, cfg.heads * cfg.head_dim
+        for w, stack, N, K in ((self.qkv, False, cfg.qkv_rows, D), (self.o, False, D, Hd), (moe.router, False, E, D),
+                               (moe.gate_up, True, 2 * I, D), (moe.down, True, D, I)):
+            if not isinstance(w, ops.PackedQ4) or w.stacked != stack or w.N != N or w.K != K or (stack and w.E != E):
+                return None
+        for w, n in ((self.input_norm, D), (self.post_norm, D), (self.q_norm, 128), (self.k_norm, 128)):
+            if w.dtype != torch.bfloat16 or not w.is_cuda or w.numel() != n or not w.is_contiguous():
+                return None
+        if cfg.head_dim != ops.HEAD_DIM or self.inv_freq.dtype != torch.float32 or not self.inv_freq.is_cuda \
+                or self.inv_freq.numel() != 64 or not self.inv_freq.is_contiguous():
+            return None
+        return _lib.Layer(D, cfg.heads, cfg.kv_heads, E, moe.top_k, I, int(moe.norm_topk), cfg.eps,
+                          cfg.head_dim ** -0.5, self.input_norm.data_ptr(), self.q_norm.data_ptr(),
+                          self.k_norm.data_ptr(), self.post_norm.data_ptr(), self.inv_freq.data_ptr(),
+                          self.qkv.data.data_ptr(), self.o.data.data_ptr(), moe.router.data.data_ptr(),
+                          moe.gate_up.data.data_ptr(), moe.down.data.data_ptr())
+
     def step(self, x: torch.Tensor, pool: torch.Tensor, st: StepState, debug: dict | None = None) -> torch.Tensor:
         """x [B, D] -> the layer's output rows (Q36/model/model.py:65-80 order: attention
         sub-block, residual, MoE sub-block, residual); `debug` receives every intermediate."""
@@ -228,6 +250,10 @@ class DecoderLayer:
         (Q36/model/moe.py:161-190)."""
         cfg = self.cfg
         T = x.shape[0]
+        if debug is None and T:
+            lay = self.native()
+            if lay is not None:
+                return self._mixed_native(lay, x, pool, ms)
         xn = ops.rmsnorm(x, self.input_norm, cfg.eps)
         qkv = ops.qmm(xn, self.qkv)
         q = ops.qk_norm_rope_append(qkv, cfg.heads, cfg.kv_heads, self.q_norm, self.k_norm, cfg.eps,
@@ -253,6 +279,53 @@ class DecoderLayer:
         return y
 
 
+    def _mixed_native(self, lay, x: torch.Tensor, pool: torch.Tensor, ms: MixedState) -> torch.Tensor:
+        """mixed as one native call (the same launches and bits; the attention halves write one buffer)."""
+        T, D, dev, pf = x.shape[0], self.cfg.hidden, x.device, ms.prefill
+        _rows_contract(x, D, pool, self.cfg.kv_heads)
+        for t, n in ((ms.pos_rows, "pos"), (ms.table_rows, "table_rows"), (ms.seq_table, "seq_table")):
+            ops._need(t, torch.int32, n)
+        if T != ms.pos_rows.numel() or T != ms.table_rows.shape[0] or pf.rows != ms.P or T != ms.P + ms.decode.lens.shape[0]:
+            raise ValueError(f"x has {T} rows, the step {ms.P} prompt and {ms.decode.lens.shape[0]} decode rows")
+        ops.prefill_contract(pf, ms.seq_table)
+        need = ops.prefill_workspace_bytes(pf, self.cfg.heads) if ms.P else 0
+        pws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+        tb, bl = pf.tables.data_ptr(), pf.blocks.data_ptr()
+        C, nblk = pf.tables.shape[1], pf.blocks.shape[1]
+        p = _lib.PromptRows(ms.P, C, nblk, pf.pmax, pf.max_len, ms.seq_table.shape[1], ms.table_rows.shape[1],
+                            ms.pos_rows.data_ptr(), ms.table_rows.data_ptr(), ms.seq_table.data_ptr(), tb, tb + 4 * C,
+                            tb + 8 * C, tb + 12 * C, bl, bl + 4 * nblk, bl + 8 * nblk,
+                            pws.data_ptr() if need else None)
+        d, dws = _decode_rows(self.cfg, ms.dec_table, ms.decode, ms.workspace, dev)
+        lib = _lib.lib()
+        scratch = torch.empty(lib.jit_layer_scratch_bytes(ctypes.byref(lay), T, 1), dtype=torch.uint8, device=dev)
+        y = torch.empty_like(x)
+        _lib.check(lib.jit_mixed_layer(ctypes.byref(lay), ctypes.byref(p), ctypes.byref(d), pool.data_ptr(),
+                                       x.data_ptr(), scratch.data_ptr(), y.data_ptr(), ops._stream()), "mixed_layer")
+        return y
+
+
+def _rows_contract(x: torch.Tensor | None, D: int, pool: torch.Tensor, Hkv: int) -> None:
+    """The checks of a layer's calls on its rows (None: rows a call has written) and pool (ValueError)."""
+    if x is not None:
+        ops._need(x, torch.bfloat16, "x")
+        if x.dim() != 2 or x.shape[1] != D:
+            raise ValueError(f"x {tuple(x.shape)} must be [rows, {D}]")
+    ops._need(pool, torch.bfloat16, "pool")
+    if ops._pool_heads(pool) != Hkv:
+        raise ValueError(f"the pool has {pool.shape[1]} kv heads, the layer {Hkv}")
+
+
+def _decode_rows(cfg: MoEConfig, table: torch.Tensor, plan: ops.AttnPlan, workspace, device):
+    """(jit_decode_rows, the workspace it points to) of a step's decode rows."""
+    B = plan.lens.shape[0]
+    ops._need(table, torch.int32, "page_table")
+    ops.decode_contract(B, table, plan)
+    ws = ops._attn_workspace(workspace, plan, cfg.heads, cfg.kv_heads, device)
+    return _lib.DecodeRows(B, table.shape[1], plan.total, table.data_ptr(), plan.lens.data_ptr(),
+                           plan.chunk_start.data_ptr(), plan.chunk_seq.data_ptr(), ws.data_ptr(), ws.nbytes), ws
+
+
 class Model:
     """A stack of decoder layers and the ragged batched decode step."""
 
@@ -265,6 +338,9 @@ class Model:
 
     def decode_step(self, x: torch.Tensor, pools: list, st: StepState) -> torch.Tensor:
         """x [B, D] bf16 hidden rows -> the last layer's output rows; pools[l] is layer l's KV pool."""
+        lays = [layer.native() for layer in self.layers] if x.shape[0] else [None]
+        if lays and None not in lays:
+            return self._decode_native(lays, x, pools, st)
         one = x.shape[0] == 1
         xn, carry = None, None
         for i, (layer, pool) in enumerate(zip(self.layers, pools)):
@@ -274,6 +350,35 @@ class Model:
             y, out = layer.run(x, pool, st, xn=xn, carry=carry, defer=defer,
                                next_norm=None if (defer or nxt is None) else nxt.input_norm)
             x, xn, carry = (None, None, out) if defer else (y, out, None)
+        return x
+
+
+    def _decode_native(self, lays: list, x: torch.Tensor, pools: list, st: StepState) -> torch.Tensor:
+        """decode_step with a native call a layer (the same launches and bits)."""
+        cfg, lib, stream, dev = self.cfg, _lib.lib(), ops._stream(), x.device
+        B, D = x.shape[0], cfg.hidden
+        d, ws = _decode_rows(cfg, st.page_table, st.plan, st.workspace, dev)
+        if B != d.B:
+            raise ValueError(f"x has {B} rows, the step {d.B}")
+        dp, xn, prev = ctypes.byref(d), None, None
+        n = min(len(lays), len(pools))
+        for i, (lay, pool) in enumerate(zip(lays, pools)):
+            # (x is the step's input, or the rows the previous call wrote; a deferred combine keeps its scratch)
+            _rows_contract(x if i == 0 else None, D, pool, cfg.kv_heads)
+            last = i + 1 == n
+            defer = B == 1 and not last and ops.row_prologue_fits(self.layers[i + 1].qkv, D)
+            lp = ctypes.byref(lay)
+            scratch = torch.empty(lib.jit_layer_scratch_bytes(lp, B, 0), dtype=torch.uint8, device=dev)
+            out = None if defer else torch.empty((1 if last else 2, B, D), dtype=torch.bfloat16, device=dev)
+            _lib.check(lib.jit_decode_layer(
+                lp, dp, pool.data_ptr(), x.data_ptr(), ops._p(xn), ops._p(prev), int(defer),
+                None if last else self.layers[i + 1].input_norm.data_ptr(), scratch.data_ptr(),
+                None if defer else out[0].data_ptr(), None if defer or last else out[1].data_ptr(), stream),
+                "decode_layer")
+            if defer:
+                xn, prev = None, scratch
+            else:
+                x, xn, prev = out[0], (None if last else out[1]), None
         return x
 
 

@@ -640,7 +640,7 @@ def attn_split_workspace_bytes(total_chunks: int, H: int, Hkv: int) -> int:
 
 def _attn_workspace(workspace, plan, H: int, Hkv: int, device) -> torch.Tensor:
     """The caller's workspace if the plan's partials fit it, else a new one."""
-    if workspace is not None and workspace.numel() * workspace.element_size() >= attn_workspace_bytes(plan.total, H):
+    if workspace is not None and workspace.nbytes >= plan.total * H * (HEAD_DIM + 2) * 4:  # (attn_workspace_bytes)
         return workspace
     return torch.empty(max(attn_split_workspace_bytes(plan.total, H, Hkv), 4), dtype=torch.uint8, device=device)
 
@@ -693,6 +693,13 @@ def prefill_workspace_bytes(plan: PrefillPlan, H: int) -> int:
     return int(_lib.lib().jit_prefill_workspace_bytes(plan.rows, plan.pmax, H))
 
 
+def prefill_contract(plan: PrefillPlan, page_table: torch.Tensor) -> None:
+    """Every chunk of the plan lies inside the page table (ValueError)."""
+    for seq, ctx, length in plan.chunks:
+        if seq >= page_table.shape[0] or (ctx + length + PAGE - 1) // PAGE > page_table.shape[1]:
+            raise ValueError(f"chunk ({seq}, {ctx}, {length}) is outside page_table {tuple(page_table.shape)}")
+
+
 def paged_prefill_attention(q: torch.Tensor, pool: torch.Tensor, page_table: torch.Tensor, plan: PrefillPlan,
                             scale: float, workspace: torch.Tensor | None = None) -> torch.Tensor:
     """q [T, H, 128] bf16 (the plan's chunk rows) -> out [T, H, 128]: causal attention of each chunk
@@ -707,9 +714,7 @@ def paged_prefill_attention(q: torch.Tensor, pool: torch.Tensor, page_table: tor
         raise _lib.UnsupportedShape(f"paged_prefill_attention covers head_dim 128, got {Dh}")
     if T != plan.rows:
         raise ValueError(f"q has {T} rows, the plan's chunks {plan.rows}")
-    for seq, ctx, length in plan.chunks:
-        if seq >= page_table.shape[0] or (ctx + length + PAGE - 1) // PAGE > page_table.shape[1]:
-            raise ValueError(f"chunk ({seq}, {ctx}, {length}) is outside page_table {tuple(page_table.shape)}")
+    prefill_contract(plan, page_table)
     need = prefill_workspace_bytes(plan, H)
     if need > 0 and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
@@ -726,6 +731,14 @@ def paged_prefill_attention(q: torch.Tensor, pool: torch.Tensor, page_table: tor
     return out
 
 
+def decode_contract(B: int, page_table: torch.Tensor, plan: AttnPlan) -> None:
+    """B rows, their page table and their plan agree, and the table covers the longest sequence (ValueError)."""
+    if plan.lens.shape[0] != B or page_table.shape[0] != B:
+        raise ValueError("the rows, page_table and plan disagree on the number of sequences")
+    if B and (pages := (int(plan.lens_host.max()) + PAGE - 1) // PAGE) > page_table.shape[1]:
+        raise ValueError(f"page_table has {page_table.shape[1]} columns, the longest sequence needs {pages}")
+
+
 def paged_decode_attention(q: torch.Tensor, pool: torch.Tensor, page_table: torch.Tensor,
                            plan: AttnPlan, scale: float, workspace: torch.Tensor | None = None):
     """q [B, H, 128] bf16 -> out [B, H, 128] bf16 over each sequence's first lens[b] keys of the
@@ -737,11 +750,7 @@ def paged_decode_attention(q: torch.Tensor, pool: torch.Tensor, page_table: torc
     Hkv = _pool_heads(pool)
     if Dh != HEAD_DIM:
         raise _lib.UnsupportedShape(f"paged_decode_attention covers head_dim 128, got {Dh}")
-    if plan.lens.shape[0] != B or page_table.shape[0] != B:
-        raise ValueError("q, page_table and plan disagree on the number of sequences")
-    if B and int((plan.lens_host.max() + PAGE - 1) // PAGE) > page_table.shape[1]:
-        raise ValueError(f"page_table has {page_table.shape[1]} columns, the longest sequence needs "
-                         f"{int((plan.lens_host.max() + PAGE - 1) // PAGE)}")
+    decode_contract(B, page_table, plan)
     if H % Hkv:
         raise ValueError(f"{H} query heads over a pool of {Hkv} kv heads")
     workspace = _attn_workspace(workspace, plan, H, Hkv, q.device)
@@ -750,7 +759,7 @@ def paged_decode_attention(q: torch.Tensor, pool: torch.Tensor, page_table: torc
         _lib.lib().jit_paged_decode_attn_ws(
             _p(q), _p(pool), _p(page_table), page_table.shape[1], _p(plan.lens), _p(plan.chunk_start),
             _p(plan.chunk_seq), B, H, Hkv, float(scale), plan.total, _p(workspace),
-            workspace.numel() * workspace.element_size(), _p(out), _stream(),
+            workspace.nbytes, _p(out), _stream(),
         ),
         "paged_decode_attn",
     )
@@ -770,18 +779,14 @@ def paged_decode_attention_qkv(qkv: torch.Tensor, H: int, Hkv: int, q_norm: torc
     B = qkv.shape[0]
     if qkv.shape[1] != (H + 2 * Hkv) * HEAD_DIM or _pool_heads(pool) != Hkv or inv_freq.numel() != HEAD_DIM // 2:
         raise ValueError("qkv / pool / inv_freq do not match the head geometry")
-    if plan.lens.shape[0] != B or page_table.shape[0] != B:
-        raise ValueError("qkv, page_table and plan disagree on the number of sequences")
-    if B and int((plan.lens_host.max() + PAGE - 1) // PAGE) > page_table.shape[1]:
-        raise ValueError(f"page_table has {page_table.shape[1]} columns, the longest sequence needs "
-                         f"{int((plan.lens_host.max() + PAGE - 1) // PAGE)}")
+    decode_contract(B, page_table, plan)
     workspace = _attn_workspace(workspace, plan, H, Hkv, qkv.device)
     out = torch.empty((B, H, HEAD_DIM), dtype=torch.bfloat16, device=qkv.device)
     _lib.check(
         _lib.lib().jit_paged_decode_attn_qkv_ws(
             _p(qkv), _p(q_norm), _p(k_norm), float(eps), _p(inv_freq), _p(pool), _p(page_table), page_table.shape[1],
             _p(plan.lens), _p(plan.chunk_start), _p(plan.chunk_seq), B, H, Hkv, float(scale), plan.total,
-            _p(workspace), workspace.numel() * workspace.element_size(), _p(out), _stream(),
+            _p(workspace), workspace.nbytes, _p(out), _stream(),
         ),
         "paged_decode_attn_qkv",
     )
@@ -803,11 +808,7 @@ def paged_decode_attention_noalloc(q: torch.Tensor, pool: torch.Tensor, page_tab
         raise _lib.UnsupportedShape(f"paged_decode_attention covers head_dim 128, got {Dh}")
     if out.shape != q.shape:
         raise ValueError(f"out {tuple(out.shape)} must match q {tuple(q.shape)}")
-    if plan.lens.shape[0] != B or page_table.shape[0] != B:
-        raise ValueError("q, page_table and plan disagree on the number of sequences")
-    if B and int((plan.lens_host.max() + PAGE - 1) // PAGE) > page_table.shape[1]:
-        raise ValueError(f"page_table has {page_table.shape[1]} columns, the longest sequence needs "
-                         f"{int((plan.lens_host.max() + PAGE - 1) // PAGE)}")
+    decode_contract(B, page_table, plan)
     _lib.check(
         _lib.lib().jit_paged_decode_attn_noalloc(
             _p(q), _p(pool), _p(page_table), page_table.shape[1], _p(plan.lens), _p(plan.chunk_start),

@@ -306,3 +306,58 @@ def test_layer_packed_equals_mlx_layout_layer():
         assert torch.equal(da[name], db[name]), name
     assert torch.equal(ya, yb)
     assert torch.equal(pa, pb)
+
+
+@pytest.mark.parametrize("B", [1, 2, 4, 5, 33, 257])
+def test_native_decode_step_matches_the_op_by_op_layers(B):
+    """Model.decode_step issues a layer per native call: the rows and the pools are those of the op-by-op
+    layers (DecoderLayer.step with a debug dict), bit for bit, with one row's deferred combines, the one-launch
+    routing of small steps and a packing workspace (257 rows) among them."""
+    from jitengine_amd.model import Model, MoEConfig, random_layer_weights
+
+    cfg = MoEConfig(experts=32, layers=3)
+    model = Model(cfg, [random_layer_weights(cfg, 60 + l, DEV) for l in range(3)])
+    rng = np.random.default_rng(B)
+    pos = rng.integers(0, 200, B).astype(np.int32)
+    table = torch.arange(B * 13, dtype=torch.int32, device=DEV).view(B, 13)
+    st = model.make_state(pos, table)
+    gen = torch.Generator(device=DEV).manual_seed(B)
+    pools = [torch.randn((B * 13, 4, 2, 2048), generator=gen, device=DEV).to(torch.bfloat16) for _ in range(3)]
+    x = torch.randn((B, cfg.hidden), generator=gen, device=DEV).to(torch.bfloat16)
+    got_pools = [p.clone() for p in pools]
+    got = model.decode_step(x, got_pools, st)
+    want = x
+    for layer, pool in zip(model.layers, pools):
+        want = layer.step(want, pool, st, debug={})
+    assert torch.equal(got, want)
+    for a, b in zip(got_pools, pools):
+        assert torch.equal(a, b)
+    with pytest.raises(ValueError):
+        model.decode_step(x.float(), pools, st)
+    with pytest.raises(ValueError):
+        model.decode_step(torch.cat([x, x]), pools, st)
+    with pytest.raises(ValueError):
+        model.decode_step(x, [p[:, :2].contiguous() for p in pools], st)
+
+
+@pytest.mark.parametrize("chunks,dec_pos", [([(0, 0, 9)], []), ([(0, 30, 40), (1, 6100, 64)], [100, 7, 3000]),
+                                            ([(0, 5, 200)], [50]), ([], [12, 90])])
+def test_native_mixed_layer_matches_op_by_op(chunks, dec_pos):
+    """DecoderLayer.mixed issues its launches from one native call: the rows and the pool are those of the
+    op-by-op path (with a debug dict), for prompt rows alone, both kinds, a batch that takes the tile
+    GEMMs, key parts, and decode rows alone."""
+    from jitengine_amd.model import DecoderLayer, MoEConfig, make_mixed_state, random_layer_weights
+
+    cfg = MoEConfig(experts=32, layers=1)
+    layer = DecoderLayer(cfg, random_layer_weights(cfg, 71, DEV))
+    keys = [c + n for _, c, n in chunks] + [p + 1 for p in dec_pos]
+    width = max(-(-k // 16) for k in keys)
+    table = np.arange(len(keys) * width, dtype=np.int32).reshape(len(keys), width)
+    ms = make_mixed_state(cfg, chunks, table[:len(chunks)], dec_pos, table[len(chunks):], DEV)
+    gen = torch.Generator(device=DEV).manual_seed(72)
+    pool = torch.randn((table.size, 4, 2, 2048), generator=gen, device=DEV).to(torch.bfloat16)
+    x = torch.randn((ms.P + len(dec_pos), cfg.hidden), generator=gen, device=DEV).to(torch.bfloat16)
+    other = pool.clone()
+    got = layer.mixed(x, other, ms)
+    assert torch.equal(got, layer.mixed(x, pool, ms, debug={}))
+    assert torch.equal(other, pool)
