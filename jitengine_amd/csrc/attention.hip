@@ -9,9 +9,8 @@
 //
 // Attention work item: one workgroup per chunk (1536 keys; longer for sequences past
 // 196,608 keys) of one sequence and 1 or 2 kv heads, 4 waves per kv head, each wave streaming
-// a quarter of the chunk (384 keys, three sub-runs of 128 with a softmax state each) two 16-key
-// pages (32 keys) per step; the 4 waves' states meet in LDS.  (A plan of few chunks gives every
-// sub-run a wave and every quarter a workgroup.)
+// a quarter of the chunk (384 keys) two 16-key pages (32 keys) per step; the 4 waves' states meet in
+// LDS.  (A plan of few chunks gives every quarter and kv head a workgroup of its own.)
 //   S^T[16 keys x 16 q heads] = K_page . Q^T      (4 MFMA 16x16x32 per page)
 //   online softmax in the exp2 domain (fp32 running max / sum per q head)
 //   O^T[128 d x 16 q heads] += V^T . P^T           (16 MFMA 16x16x32, all 32 keys: P as a
@@ -70,16 +69,6 @@ __host__ __device__ __forceinline__ int chunk_tokens(int len) {
   return c < kChunkMax ? c : kChunkMax;
 }
 
-// A chunk of kChunk keys is kAttnSplits groups of kGroup keys, a group kSubs sub-runs of kSubRun keys.
-// Every sub-run keeps an online-softmax state of its own, a group's state is its sub-runs' merged in
-// order, a chunk's its groups' in order (the chunks of longer sequences, not kChunk keys, have one
-// sub-run a group).  The results are therefore the same whether a wave walks a group's sub-runs one after
-// another or every sub-run has a wave and every group a workgroup of its own (paged_attn_kernel<FINE>): the
-// launch picks by how many workgroups the plan makes.
-constexpr int kSubs = 3;
-constexpr int kGroup = kChunk / kAttnSplits, kSubRun = kGroup / kSubs;
-static_assert(kSubRun * kSubs * kAttnSplits == kChunk && kSubRun % 32 == 0, "sub-runs are whole 32-key steps");
-
 __device__ __forceinline__ int k_off(int slot, int d) { return k_page_offset(slot, d); }
 
 }  // namespace
@@ -115,8 +104,8 @@ struct AttnArgs {
   const int32_t *lens;
   const int32_t *chunk_start;
   const int32_t *chunk_seq;
-  float *part_o;   // [total_chunks][H][128] (fine: [total_chunks][kAttnSplits][H][128])
-  float *part_ml;  // [total_chunks][H][2]   (fine: [total_chunks][kAttnSplits][H][2])
+  float *part_o;   // [total_chunks][H][128] (FINE: [total_chunks][kAttnSplits][H][128])
+  float *part_ml;  // [total_chunks][H][2]   (FINE: [total_chunks][kAttnSplits][H][kFineMl])
   uint16_t *out;
   int max_pages, H, Hkv, G;
   float qk_scale;  // scale * log2(e)
@@ -208,57 +197,25 @@ __device__ uint64_t g_attn_stamps[kAttnStampSlots][8];
   } while (0)
 #endif
 
-// A merged state of one q head's keys: the lane's 32 of O^T, the running max and the sum over every lane
-// group.  add() merges the state (o, m, l) of the next keys; each step is written as one operation, so that
-// every kernel that merges gets the same bits.
-struct AttnState {
-  f32x4 O[8];
-  float M, L;
-  __device__ __forceinline__ void clear() {
-    M = -INFINITY;
-    L = 0.0f;
-#pragma unroll
-    for (int cc = 0; cc < 8; cc++) O[cc] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  __device__ __forceinline__ void add(const f32x4 (&o)[8], float m, float l) {
-    const float mn = fmaxf(M, m);  // (a state added holds a key: mn is finite)
-    const float f0 = exp2f(M - mn), f1 = exp2f(m - mn);
-#pragma unroll
-    for (int cc = 0; cc < 8; cc++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) O[cc][i] = __builtin_fmaf(o[cc][i], f1, O[cc][i] * f0);
-    L = __builtin_fmaf(l, f1, L * f0);
-    M = mn;
-  }
-  // as a wave's LDS slot [kStateFloats][64]
-  __device__ __forceinline__ void put(float *st) const {
-#pragma unroll
-    for (int cc = 0; cc < 8; cc++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) st[(4 * cc + i) * 64] = O[cc][i];
-    st[32 * 64] = M;
-    st[33 * 64] = L;
-  }
-  __device__ __forceinline__ void add_slot(const float *st) {
-    f32x4 o[8];
-#pragma unroll
-    for (int cc = 0; cc < 8; cc++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) o[cc][i] = st[(4 * cc + i) * 64];
-    add(o, st[32 * 64], st[33 * 64]);
-  }
-};
+// The merge of two partial sums under their weights.  Written as the operations it is, so that every kernel
+// that merges gets the same bits.
+__device__ __forceinline__ float merge2(float a, float fa, float b, float fb) {
+  return __builtin_fmaf(a, fa, b * fb);
+}
 
 // How a launch splits a plan (the results are the same bits):
-//   coarse: a workgroup a chunk and hb kv heads, kAttnSplits waves a head, each walking a group's sub-runs;
-//   FINE: a workgroup a group and kv head, a wave a sub-run; its state is a partial of the merge.
+//   coarse: a workgroup a chunk and hb kv heads, kAttnSplits waves a head;
+//   FINE: a workgroup of one wave a quarter chunk and kv head, whose state is a partial of the merge.
 // One CU reads at about 46 GB/s however many waves or loads ahead it has, 25 GB/s when all of them read: a
-// plan of few chunks is bound by the CUs it reaches, so it takes more and smaller workgroups (attn_split).
-constexpr int attn_waves(bool fine) { return fine ? kSubs : kAttnSplits; }
+// plan of few chunks is bound by the CUs it reaches, so it takes more and smaller workgroups
+// (decode_attn_launch).  A lone wave is bound by its loads' latency: it keeps AHEAD = 2 steps of them in
+// flight, for which the coarse split has no registers (and, with 8 waves a CU, no use).
+constexpr int attn_waves(bool fine) { return fine ? 1 : kAttnSplits; }
+constexpr int kFineMl = 8;  // a FINE partial's max, and the sums of the four lane groups
 
 template <bool FINE>
-__global__ __launch_bounds__(FINE ? 64 * kSubs : 512) void paged_attn_kernel(const AttnArgs a) {
-  constexpr int WS = attn_waves(FINE);
+__global__ __launch_bounds__(FINE ? 64 : 512) void paged_attn_kernel(const AttnArgs a) {
+  constexpr int WS = attn_waves(FINE), AHEAD = FINE ? 2 : 1;
 #if JIT_ATTN_STAMPS
   uint64_t ts[5] = {__builtin_amdgcn_s_memrealtime(), 0, 0, 0, 0};
   auto stamp_out = [&]() {
@@ -282,20 +239,20 @@ __global__ __launch_bounds__(FINE ? 64 * kSubs : 512) void paged_attn_kernel(con
   const int b = a.chunk_seq[gc];
   const int L = a.lens[b];
   const int c = gc - a.chunk_start[b];
-  const int ck = FINE ? kChunk : chunk_tokens(L), kRun = FINE ? kSubRun : ck / WS;
+  const int ck = chunk_tokens(L), kRun = ck / kAttnSplits;
   const int nchunks = (L + ck - 1) / ck;
   const int lr = l & 15, lg = l >> 4;
   const int G = a.G;
-  const int b0 = c * ck + group * kGroup, b1 = min(FINE ? b0 + kGroup : b0 + ck, L);  // the workgroup's keys
-  if (FINE && b0 >= L) {  // a group without keys (the last chunk's): an empty partial (uniform)
-    if ((int)threadIdx.x < G) {
-      const long long r = (long long)blockIdx.x * a.H + kvh * G + threadIdx.x;
-      *(float2 *)(a.part_ml + r * 2) = make_float2(-INFINITY, 0.0f);
+  const int wk0 = c * ck + (FINE ? group : split) * kRun;
+  const int wk1 = min(wk0 + kRun, L);
+  if (FINE && wk0 >= L) {  // a quarter without keys (of the last chunk): an empty partial
+    if (l < G) {
+      float *ml = a.part_ml + ((long long)blockIdx.x * a.H + kvh * G + l) * kFineMl;
+      *(float4 *)ml = make_float4(-INFINITY, 0.f, 0.f, 0.f);
+      ml[4] = 0.0f;
     }
     return;
   }
-  const int wk0 = b0 + split * kRun;
-  const int wk1 = min(wk0 + kRun, b1);
   const int npg = wk1 > wk0 ? (wk1 - wk0 + kPage - 1) / kPage : 0;  // split 0 always holds a key
   const int nst = live ? (npg + 1) >> 1 : 0;                          // 32-key steps
   // the run's page ids, one per lane (at most kRun / 16 <= 64)
@@ -305,14 +262,18 @@ __global__ __launch_bounds__(FINE ? 64 * kSubs : 512) void paged_attn_kernel(con
   // masked, so prefetches need no branch)
   auto page = [&](int i) { return __builtin_amdgcn_readlane(my_page, min(i, last)); };
 
-  Frag8 kf[2][4];
-  uint2 vv[2][8];
+  Frag8 kbuf[AHEAD][2][4];
+  uint2 vbuf[AHEAD][2][8];
   // K before V, as in the loop, so a step's K wait leaves its V loads in flight
   auto first_loads = [&]() {
     if (nst > 0) {
-      load_k2(kf, a.pool, a.Hkv, kvh, page(0), page(1), lr, lg);
-      asm volatile("" ::: "memory");
-      load_v2(vv, a.pool, a.Hkv, kvh, page(0), page(1), lr, lg);
+#pragma unroll
+      for (int j = 0; j < AHEAD; j++) {
+        if (j) asm volatile("" ::: "memory");
+        load_k2(kbuf[j], a.pool, a.Hkv, kvh, page(2 * j), page(2 * j + 1), lr, lg);
+        asm volatile("" ::: "memory");
+        load_v2(vbuf[j], a.pool, a.Hkv, kvh, page(2 * j), page(2 * j + 1), lr, lg);
+      }
     }
   };
   // Q^T fragments (B operand of S^T = K . Q^T): q head lr, dims 8*lg.. of each chunk
@@ -331,18 +292,19 @@ __global__ __launch_bounds__(FINE ? 64 * kSubs : 512) void paged_attn_kernel(con
     // rotates its q heads (qk_head_norm_rope, as jit_qk_norm_rope_append does: the same bits) into
     // LDS, and the workgroup of the sequence's last chunk first writes the token's K and V of its
     // kv heads into the pool.  The barrier's fence orders those stores before this workgroup's
-    // reads of the token's page; other workgroups never read it.  A wave whose first step holds
-    // that page issues its first loads after the barrier, the others right after requesting the
+    // reads of the token's page; other workgroups never read it.  A wave whose first loads hold
+    // that page issues them after the barrier, the others right after requesting the
     // token's values: vector loads complete in order, so values requested behind the first K/V
     // loads would be waited for only once those had landed.
     const int tok = L - 1;
-    const bool defer = wk1 == L && tok < wk0 + 32;
+    const bool defer = wk1 == L && tok < wk0 + 32 * AHEAD;
     const int nh = a.H + 2 * a.Hkv;
     const uint16_t *row = a.qkv + (long long)b * nh * kD;
     uint16_t *qs = (uint16_t *)(xstate + (WS - 1) * hb * kStateFloats * 64);  // [hb][G][128], past the states
     constexpr int kQHeads = (16 + WS - 1) / WS;  // q heads a wave norms (G <= 16)
-    const bool writer = live && c == nchunks - 1 && b1 == L && split < 2;  // the token's K (split 0) or V (split 1)
-    uint16_t qx[kQHeads][2], tx[2] = {0, 0}, qw[2] = {0, 0}, kw[2] = {0, 0};
+    // the token's K (split 0) and V (split 1; FINE: the one wave both), in the quarter or chunk that holds it
+    const bool writer = live && c == nchunks - 1 && split < 2 && (!FINE || wk1 == L);
+    uint16_t qx[kQHeads][2], tx[2] = {0, 0}, vx[2] = {0, 0}, qw[2] = {0, 0}, kw[2] = {0, 0};
     float fr = 0.0f;
     int pg = 0;
     if (live) {
@@ -367,6 +329,10 @@ __global__ __launch_bounds__(FINE ? 64 * kSubs : 512) void paged_attn_kernel(con
           kw[0] = a.kn_w[l];
           kw[1] = a.kn_w[l + 64];
         }
+        if (FINE) {
+          vx[0] = src[a.Hkv * kD + l];
+          vx[1] = src[a.Hkv * kD + l + 64];
+        }
       }
     }
     asm volatile("" ::: "memory");  // (the token's loads stay ahead of the first K/V)
@@ -381,9 +347,10 @@ __global__ __launch_bounds__(FINE ? 64 * kSubs : 512) void paged_attn_kernel(con
           qk_head_norm_rope(bf2f(tx[0]), bf2f(tx[1]), bf2f(kw[0]), bf2f(kw[1]), a.eps, ang, o1, o2);
           hp[k_page_offset(slot, l)] = (uint16_t)o1;
           hp[k_page_offset(slot, l + 64)] = (uint16_t)o2;
-        } else {  // V: as it is, into the dim-major V part
-          hp[kPageHead + l * kPage + slot] = tx[0];
-          hp[kPageHead + (l + 64) * kPage + slot] = tx[1];
+        }
+        if (FINE || split) {  // V: as it is, into the dim-major V part
+          hp[kPageHead + l * kPage + slot] = FINE ? vx[0] : tx[0];
+          hp[kPageHead + (l + 64) * kPage + slot] = FINE ? vx[1] : tx[1];
         }
       }
 #pragma unroll
@@ -416,31 +383,11 @@ __global__ __launch_bounds__(FINE ? 64 * kSubs : 512) void paged_attn_kernel(con
   asm volatile("" ::: "memory");
   ATTN_STAMP(1);
 #endif
-  AttnState S;  // the sub-runs so far
-  S.clear();
-  bool first = true;
-  // the end of a sub-run: its state joins S (the first is S) and the next one starts afresh
-  auto flush = [&]() {
-    const float l_sub = sum_xor32(sum_xor16(l_run));
-    if (first) {
-#pragma unroll
-      for (int cc = 0; cc < 8; cc++) S.O[cc] = o[cc];
-      S.M = m_run;
-      S.L = l_sub;
-    } else {
-      S.add(o, m_run, l_sub);
-    }
-    first = false;
-    m_run = -INFINITY;
-    l_run = 0.0f;
-#pragma unroll
-    for (int cc = 0; cc < 8; cc++) o[cc] = f32x4{0.f, 0.f, 0.f, 0.f};
-  };
-  const bool subs = !FINE && ck == kChunk;
-  // One step; MORE: another follows, whose K and V are requested here.  (The run's last step is a copy of its
-  // own without the requests: behind a branch in one body they would make the waits before P.V count no load
-  // in flight, and requested for nothing they cost a step's reads and hold the registers of the merge below.)
-  auto step = [&](const int st, auto more) {
+  // One step on a buffer's K and V; MORE: step st + AHEAD exists, and is requested into it here.  (The run's last
+  // steps are copies of their own without the requests: behind a branch in one body they would make the
+  // waits before P.V count no load in flight, and requested for nothing they cost a twelfth of the reads
+  // and hold the registers of the merge below.)
+  auto step = [&](const int st, Frag8 (&kf)[2][4], uint2 (&vv)[2][8], auto more) {
     constexpr bool MORE = decltype(more)::value;
     const int k0 = wk0 + 32 * st;
     f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -450,7 +397,8 @@ __global__ __launch_bounds__(FINE ? 64 * kSubs : 512) void paged_attn_kernel(con
       s1 = mfma16x16x32(kf[1][cc], qf[cc], s1);
     }
     // K registers are free: the next step's K is in flight during softmax and P.V
-    if constexpr (MORE) load_k2(kf, a.pool, a.Hkv, kvh, page(2 * st + 2), page(2 * st + 3), lr, lg);
+    if constexpr (MORE)
+      load_k2(kf, a.pool, a.Hkv, kvh, page(2 * (st + AHEAD)), page(2 * (st + AHEAD) + 1), lr, lg);
     // keys past the run are masked on its last step only; the scale is applied inside the
     // exponent's fma (the max of the raw scores times the positive scale is the scaled max)
     float p0[4], p1[4];
@@ -525,49 +473,86 @@ __global__ __launch_bounds__(FINE ? 64 * kSubs : 512) void paged_attn_kernel(con
     }
 #pragma unroll
     for (int cc = 0; cc < 8; cc++) o[cc] = mfma16x16x32(vf[cc], pl, o[cc]);
-    if constexpr (MORE) load_v2(vv, a.pool, a.Hkv, kvh, page(2 * st + 2), page(2 * st + 3), lr, lg);
+    if constexpr (MORE)
+      load_v2(vv, a.pool, a.Hkv, kvh, page(2 * (st + AHEAD)), page(2 * (st + AHEAD) + 1), lr, lg);
     // keep these loads in this step: sunk into the next step they would only be
     // issued once that step's K has arrived
     asm volatile("" ::: "memory");
-    if (MORE && subs && (st + 1) % (kSubRun / 32) == 0) flush();  // (uniform)
   };
-  for (int st = 0; st + 1 < nst; st++) step(st, std::true_type{});
-  if (nst > 0) {
-    step(nst - 1, std::false_type{});
-    flush();
+  {
+    const std::true_type more;
+    const std::false_type done;
+    int st = 0;
+    for (; st + 2 * AHEAD <= nst; st += AHEAD)
+#pragma unroll
+      for (int j = 0; j < AHEAD; j++) step(st + j, kbuf[j], vbuf[j], more);
+    if constexpr (AHEAD == 1) {
+      if (st < nst) step(st, kbuf[0], vbuf[0], done);
+    } else if (nst - st == 3) {
+      step(st, kbuf[0], vbuf[0], more);
+      step(st + 1, kbuf[1], vbuf[1], done);
+      step(st + 2, kbuf[0], vbuf[0], done);
+    } else if (nst > st) {
+      step(st, kbuf[0], vbuf[0], done);
+      if (nst - st == 2) step(st + 1, kbuf[1], vbuf[1], done);
+    }
   }
   ATTN_STAMP(2);
-  // the waves' states meet in LDS: split 0 of each kv head adds the others in order (the sub-runs of a group
-  // as far as they hold keys, as a wave that walks them does; every group of a chunk)
-  auto slot = [&](int sp) { return xstate + (((sp - 1) * hb + kvl) * kStateFloats) * 64 + l; };
-  if (split > 0) S.put(slot(split));
-  __syncthreads();
-  if (split == 0)
+  if constexpr (!FINE) {  // the waves' states meet: split 0 of each kv head adds splits 1.. in order
+    if (split > 0) {
+      float *st = xstate + (((split - 1) * hb + kvl) * kStateFloats) * 64 + l;
 #pragma unroll
-    for (int sp = 1; sp < WS; sp++)
-      if (!FINE || b0 + sp * kRun < b1) S.add_slot(slot(sp));
-  ATTN_STAMP(3);
-  if (split > 0 || !live) return;
+      for (int cc = 0; cc < 8; cc++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) st[(4 * cc + i) * 64] = o[cc][i];
+      st[32 * 64] = m_run;
+      st[33 * 64] = l_run;
+    }
+    __syncthreads();
+    ATTN_STAMP(3);
+    if (split > 0 || !live) return;
+#pragma unroll
+    for (int sp = 1; sp < WS; sp++) {
+      const float *st = xstate + (((sp - 1) * hb + kvl) * kStateFloats) * 64 + l;
+      const float m2 = st[32 * 64], l2 = st[33 * 64];
+      const float M = fmaxf(m_run, m2);  // split 0 holds a key: M is finite
+      const float f0 = exp2f(m_run - M), f1 = exp2f(m2 - M);
+#pragma unroll
+      for (int cc = 0; cc < 8; cc++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[cc][i] = merge2(o[cc][i], f0, st[(4 * cc + i) * 64], f1);
+      l_run = merge2(l_run, f0, l2, f1);
+      m_run = M;
+    }
+  }
 #if JIT_ATTN_STAMPS
   if (wave == 0) stamp_out();
 #endif
+  // per-head sum over the four lane groups (FINE: the merge adds them up, after the quarters)
+  const float l_tot = FINE ? l_run : sum_xor32(sum_xor16(l_run));
   if (lr >= G) return;
   const long long row = (long long)b * a.H + kvh * G + lr;  // this lane's q head
   if (!FINE && nchunks == 1) {
-    const float inv = 1.0f / S.L;
+    const float inv = 1.0f / l_tot;
 #pragma unroll
     for (int cc = 0; cc < 8; cc++) {
       uint2 w;
-      w.x = pack_bf16x2(S.O[cc][0] * inv, S.O[cc][1] * inv);
-      w.y = pack_bf16x2(S.O[cc][2] * inv, S.O[cc][3] * inv);
+      w.x = pack_bf16x2(o[cc][0] * inv, o[cc][1] * inv);
+      w.y = pack_bf16x2(o[cc][2] * inv, o[cc][3] * inv);
       *(uint2 *)(a.out + row * kD + 16 * cc + 4 * lg) = w;
     }
   } else {
     const long long r = (long long)blockIdx.x * a.H + kvh * G + lr;
 #pragma unroll
     for (int cc = 0; cc < 8; cc++)
-      *(float4 *)(a.part_o + r * kD + 16 * cc + 4 * lg) = make_float4(S.O[cc][0], S.O[cc][1], S.O[cc][2], S.O[cc][3]);
-    if (lg == 0) *(float2 *)(a.part_ml + r * 2) = make_float2(S.M, S.L);
+      *(float4 *)(a.part_o + r * kD + 16 * cc + 4 * lg) = make_float4(o[cc][0], o[cc][1], o[cc][2], o[cc][3]);
+    if (FINE) {
+      if (lg == 0) a.part_ml[r * kFineMl] = m_run;
+      a.part_ml[r * kFineMl + 1 + lg] = l_run;
+    } else if (lg == 0) {
+      a.part_ml[r * 2 + 0] = m_run;
+      a.part_ml[r * 2 + 1] = l_tot;
+    }
   }
 }
 
@@ -578,8 +563,9 @@ __global__ __launch_bounds__(FINE ? 64 * kSubs : 512) void paged_attn_kernel(con
 // instead of one per chunk in a serial chain.  Lane j merges chunks j, j + 16, ...
 // online (running max, one pass over the partials), and the 16 lane states are
 // merged in lane order: a fixed order that depends only on the sequence's chunk count.
-// FINE: a chunk's partial is first put together from its groups', in order and with AttnState's operations
-// (group 0 always holds a key; a group without one left (-inf, 0)).
+// FINE: a chunk's partial is first put together from its quarters', in order and with the operations of the
+// coarse split's waves (quarter 0 always holds a key; one without left a max of -inf and sums of 0, and
+// no o).
 constexpr int kMergeLanes = 16;
 
 template <bool FINE>
@@ -606,27 +592,34 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t *__restri
     float2 ml;
     float4 o;
     if constexpr (FINE) {
-      float2 gm[kAttnSplits];
+      float m[kAttnSplits], ls[kAttnSplits][4];
       float4 go[kAttnSplits];
 #pragma unroll
       for (int w = 0; w < kAttnSplits; w++) {
         const long long r = ((c0 + c) * kAttnSplits + w) * H + h;
-        gm[w] = *(const float2 *)(part_ml + r * 2);
+        const float4 m4 = *(const float4 *)(part_ml + r * kFineMl);
+        m[w] = m4.x;
+        ls[w][0] = m4.y;
+        ls[w][1] = m4.z;
+        ls[w][2] = m4.w;
+        ls[w][3] = part_ml[r * kFineMl + 4];
         go[w] = *(const float4 *)(part_o + r * kD + 4 * dq);
       }
-      ml = gm[0];
       o = go[0];
 #pragma unroll
       for (int w = 1; w < kAttnSplits; w++) {
-        if (gm[w].y == 0.0f && gm[w].x == -INFINITY) go[w] = make_float4(0.f, 0.f, 0.f, 0.f);  // (nothing was stored)
-        const float mg = fmaxf(ml.x, gm[w].x);
-        const float f0 = exp2f(ml.x - mg), f1 = exp2f(gm[w].x - mg);
-        o.x = __builtin_fmaf(go[w].x, f1, o.x * f0);
-        o.y = __builtin_fmaf(go[w].y, f1, o.y * f0);
-        o.z = __builtin_fmaf(go[w].z, f1, o.z * f0);
-        o.w = __builtin_fmaf(go[w].w, f1, o.w * f0);
-        ml = make_float2(mg, __builtin_fmaf(gm[w].y, f1, ml.y * f0));
+        if (m[w] == -INFINITY && ls[w][0] == 0.0f) go[w] = make_float4(0.f, 0.f, 0.f, 0.f);  // (nothing was stored)
+        const float M = fmaxf(m[0], m[w]);
+        const float f0 = exp2f(m[0] - M), f1 = exp2f(m[w] - M);
+        o.x = merge2(o.x, f0, go[w].x, f1);
+        o.y = merge2(o.y, f0, go[w].y, f1);
+        o.z = merge2(o.z, f0, go[w].z, f1);
+        o.w = merge2(o.w, f0, go[w].w, f1);
+#pragma unroll
+        for (int g = 0; g < 4; g++) ls[0][g] = merge2(ls[0][g], f0, ls[w][g], f1);
+        m[0] = M;
       }
+      ml = make_float2(m[0], (ls[0][0] + ls[0][1]) + (ls[0][2] + ls[0][3]));
       if (n == 1) {  // the whole result (chunk lane 0 alone is here)
         const float inv = 1.0f / ml.y;
         uint2 w;
@@ -642,11 +635,11 @@ __global__ __launch_bounds__(512) void attn_merge_kernel(const int32_t *__restri
     }
     const float mn = fmaxf(m_run, ml.x);
     const float fa = exp2f(m_run - mn), fb = exp2f(ml.x - mn);
-    Ls = __builtin_fmaf(ml.y, fb, Ls * fa);
-    O.x = __builtin_fmaf(o.x, fb, O.x * fa);
-    O.y = __builtin_fmaf(o.y, fb, O.y * fa);
-    O.z = __builtin_fmaf(o.z, fb, O.z * fa);
-    O.w = __builtin_fmaf(o.w, fb, O.w * fa);
+    Ls = merge2(Ls, fa, ml.y, fb);
+    O.x = merge2(O.x, fa, o.x, fb);
+    O.y = merge2(O.y, fa, o.y, fb);
+    O.z = merge2(O.z, fa, o.z, fb);
+    O.w = merge2(O.w, fa, o.w, fb);
     m_run = mn;
   }
   if (FINE && n == 1) return;  // (uniform)
@@ -1152,15 +1145,14 @@ extern "C" int jit_attn_plan(const int32_t *lens_host, int B, int32_t *chunk_sta
 }
 
 namespace {
-// Whether a plan of total_chunks chunks takes the fine split (given a workspace for its partials): up to
-// 192 chunks x kv heads, i.e. while the coarse split with one kv head a workgroup leaves CUs without
-// one.  Kernel + merge at Hkv = 4, us, before (two kv heads a workgroup) / one kv head a workgroup / fine: 1
-// sequence of 1,536 keys 33.9 / 18.1 / 10.7, of 4,096 keys 36.9 / 22.2 / 12.1, of 32,768 keys 40.3 / 25.0 / 20.0; 8
-// of 4,096 40.0 / 26.8 / 20.2; 48 chunks 42.7 / 28.5 / 28.5, 56 chunks 41.9 / 27.0 / 29.2.
-constexpr int kFewWorkgroups = 256;
-constexpr int kMaxFineChunks = 118;  // (a sequence of longer chunks, which has no groups, has at least 119)
-bool attn_fine(int total_chunks, int Hkv) {
-  return total_chunks <= kMaxFineChunks && (long long)total_chunks * Hkv <= 192;
+// Whether a plan of total_chunks chunks may take the fine split (given a workspace for its partials).  It
+// does if it has a sequence of several chunks: kernel + merge at Hkv = 4, us, coarse with two kv heads a workgroup
+// (before) / with one / fine: one sequence of 4,096 keys 36.7 / 22.0 / 16.3, of 32,768 keys 40.2 / 24.8 / 21.5, 8
+// of 4,096 keys 39.9 / 26.7 / 21.7; 48 chunks 42.6 / 28.4 / 31.0.  Sequences of one chunk are mostly short: 100
+// keys 10.0 / 9.7 / 11.5, 32 of 1,000 keys 29.9 / 20.4 / 21.2 (1,536 keys 33.8 / 18.3 / 15.5).
+bool attn_fine(int total_chunks, int Hkv) { return (long long)total_chunks * Hkv <= 112; }
+int64_t attn_fine_bytes(int total_chunks, int H) {
+  return (int64_t)total_chunks * kAttnSplits * H * (kD + kFineMl) * (int64_t)sizeof(float);
 }
 }  // namespace
 
@@ -1169,10 +1161,24 @@ extern "C" int64_t jit_attn_workspace_bytes(int total_chunks, int H) {
 }
 
 extern "C" int64_t jit_attn_split_workspace_bytes(int total_chunks, int H, int Hkv) {
-  return (attn_fine(total_chunks, Hkv) ? kAttnSplits : 1) * jit_attn_workspace_bytes(total_chunks, H);
+  return attn_fine(total_chunks, Hkv) ? attn_fine_bytes(total_chunks, H) : jit_attn_workspace_bytes(total_chunks, H);
 }
 
 namespace {
+
+// kv heads a workgroup of the coarse split takes.  A CU holds one workgroup of two (8 waves) or three of
+// one.  Two fill the CUs evenly when their workgroups come out just short of whole rounds; otherwise one:
+// while all of its workgroups have a CU each, and where two would leave the last of several rounds part empty.
+// Kernel + merge at Hkv = 4, us, two / one: 64 chunks 43.2 / 37.4, 66 chunks 44.8 / 50.0, 84 ragged 46.0 / 49.4, 121
+// ragged 56.1 / 56.3, 128 (262,144 keys) 86.7 / 87.0, 132 chunks 100 / 84, 139 ragged 90 / 75, 185 ragged 99 / 87, 256
+// chunks 137.0 / 137.8, 264 chunks 159 / 143, 400 short 88 / 81.
+int attn_heads_per_block(int total_chunks, int Hkv) {
+  const int two = Hkv < kAttnHeadsPerBlock ? Hkv : kAttnHeadsPerBlock, cus = jit::cu_count();
+  const long long w1 = (long long)total_chunks * Hkv, w2 = (long long)total_chunks * ((Hkv + two - 1) / two);
+  if (w1 <= cus) return 1;
+  const long long rounds = (w2 + cus - 1) / cus;
+  return rounds >= 2 && 20 * w2 < 19 * rounds * cus ? 1 : two;
+}
 
 // The two launches of a decode-attention call: the split-K chunks, then the chunk-order merge.
 // `workspace` holds the fp32 partials of multi-chunk sequences (every partial the merge reads
@@ -1189,16 +1195,12 @@ int decode_attn_launch(const uint16_t *q, const uint16_t *pool, const int32_t *p
                        int Hkv, float scale, int total_chunks, void *workspace, int64_t workspace_bytes, uint16_t *out,
                        hipStream_t st, const char *what, const FusedQkv *fq = nullptr) {
   const bool fine =
-      attn_fine(total_chunks, Hkv) && workspace_bytes >= jit_attn_split_workspace_bytes(total_chunks, H, Hkv);
+      attn_fine(total_chunks, Hkv) && total_chunks > B && workspace_bytes >= attn_fine_bytes(total_chunks, H);
   const int slots = total_chunks * (fine ? kAttnSplits : 1);
   float *part_o = (float *)workspace;
   float *part_ml = part_o + (long long)slots * H * kD;
   const int WS = attn_waves(fine);
-  // kv heads per workgroup (WS waves each): one while that leaves no CU with two workgroups (64 chunks of
-  // 1,500 keys at Hkv = 4: 43.9 -> 37.6 us; 66 chunks 45.2 -> 50.5)
-  const int hb = fine || (long long)total_chunks * Hkv <= kFewWorkgroups
-                     ? 1
-                     : (Hkv < kAttnHeadsPerBlock ? Hkv : kAttnHeadsPerBlock);
+  const int hb = fine ? 1 : attn_heads_per_block(total_chunks, Hkv);  // kv heads per workgroup (WS waves each)
   AttnArgs a{q, pool, page_table, lens, chunk_start, chunk_seq, part_o, part_ml, out,
              max_pages, H, Hkv, H / Hkv, scale * 1.44269504088896341f, hb,
              fq ? fq->qkv : nullptr, fq ? fq->q_norm_w : nullptr, fq ? fq->k_norm_w : nullptr,

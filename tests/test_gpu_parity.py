@@ -530,29 +530,29 @@ def test_dense_projection_shapes_agree(N, K):
 
 
 @pytest.mark.parametrize("lens,H,Hkv", [
-    ([1], 32, 4), ([127, 128, 129, 383, 384, 385], 32, 4), ([767, 1151, 1152, 1535, 1536, 1537, 1663], 32, 4),
-    ([4096], 32, 4), ([3000, 70], 64, 4), ([3071, 5], 8, 8), ([2000, 17], 16, 1), ([70000], 32, 4)])
+    ([1], 32, 4), ([1537], 32, 4), ([4096], 32, 4), ([1921, 383, 384, 385], 32, 4), ([1952, 2304, 2305], 32, 4),
+    ([3000, 70], 64, 4), ([3071, 5], 8, 8), ([2000, 17], 16, 1), ([40000], 32, 4), ([200003], 16, 1)])
 def test_decode_attention_splits_agree(lens, H, Hkv):
-    """A plan of few chunks runs with a wave a 128-key sub-run and a workgroup a 384-key group when the
-    workspace holds its partials, else with a wave a group: the same bits, for the plain and the fused
-    entry (outputs and pool), at the edges of sub-runs, groups and chunks.  Enough copies of the batch
-    reach the launch with one kv head a workgroup and, past it, the one with two."""
-    rng = np.random.default_rng(sum(lens) + H)
+    """A plan of few chunks runs with a workgroup a quarter chunk when the workspace holds its partials,
+    else with a workgroup a chunk and one or two kv heads: the same bits, for the plain and the fused
+    entry (outputs and pool), with lengths around a quarter's first two steps and its end, and quarters
+    without keys.  Copies of the batch reach every launch."""
     q, pool, table = _pool(lens, seed=51, H=H, Hkv=Hkv)
-    fine_plan = ops.attn_plan(lens, DEV)
-    assert ops.attn_split_workspace_bytes(fine_plan.total, H, Hkv) == 4 * ops.attn_workspace_bytes(fine_plan.total, H)
+    total = ops.attn_plan(lens, DEV).total
     qn, kn = (bf16_tensor(normal_bf16((128,), seed=s), DEV) for s in (52, 53))
     freq = torch.from_numpy((1e6 ** (-np.arange(0, 128, 2) / 128)).astype(np.float32)).to(DEV)
     qkv = normal_bf16((len(lens), (H + 2 * Hkv) * 128), seed=54)
     scale = 128 ** -0.5
     base = None
-    for copies in (1, max(1, 250 // (fine_plan.total * Hkv)), 300 // (fine_plan.total * Hkv) + 1):
+    # one copy; one kv head a workgroup (at most 256); two (at most 512); one again (two rounds of two)
+    for copies in sorted({1, max(1, 250 // (total * Hkv)), 500 // (total * Hkv) + 1, 560 // (total * Hkv) + 1}):
         ln = list(lens) * copies
         plan = ops.attn_plan(ln, DEV)
         tab = _i32(np.concatenate([table] * copies))
         qs = bf16_tensor(np.concatenate([q] * copies), DEV)
         rows = bf16_tensor(np.concatenate([qkv] * copies), DEV)
-        for ws_bytes in (ops.attn_workspace_bytes(plan.total, H), ops.attn_split_workspace_bytes(plan.total, H, Hkv)):
+        for ws_bytes in sorted({ops.attn_workspace_bytes(plan.total, H),
+                                ops.attn_split_workspace_bytes(plan.total, H, Hkv)}):
             ws = torch.full((ws_bytes,), 0xFF, dtype=torch.uint8, device=DEV)  # (NaN bits: nothing stale is read)
             pt = bf16_tensor(pool, DEV)
             out = u16(ops.paged_decode_attention(qs, pt, tab, plan, scale, ws))
