@@ -736,11 +736,12 @@ __global__ __launch_bounds__(64 * WAVES) void prefill_attn_kernel(const PrefillA
   // one dimension, the kv heads of an item adjacent: the hardware dispatches workgroups in index
   // order, so the plan's longest-first order holds across the kv heads (a (item, kv head) grid
   // dispatched every item of kv head 0 before any of kv head 1)
-  const int item = blockIdx.x / (kSub * a.Hkv), rest = blockIdx.x % (kSub * a.Hkv), kvh = rest % a.Hkv;
+  const int item = blockIdx.x / (kSub * a.Hkv), kvh = blockIdx.x % a.Hkv;
   const int ch = a.blk_chunk[item], part = a.blk_part[item];
   const int seq = a.chunk_seq[ch], ctx = a.chunk_ctx[ch], len = a.chunk_len[ch], row0 = a.chunk_row[ch];
   const int G = a.G, TR = 16 / G, tpw = kPfTiles * TR;
-  const int q0 = a.blk_q0[item] + (rest / a.Hkv) * WAVES * tpw;
+  int q0 = a.blk_q0[item];
+  if constexpr (kSub > 1) q0 += blockIdx.x / a.Hkv % kSub * WAVES * tpw;
   if (kSub > 1 && q0 >= len) return;  // (uniform)
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = lane_id();
   const int lr = l & 15, lg = l >> 4;
