@@ -99,6 +99,7 @@ struct Shared {
   float f[kWaves];
   uint64_t q[kWaves];
   uint64_t qx[kWaves];
+  uint32_t ux[kWaves];
   int cut[8];
 };
 
@@ -124,20 +125,26 @@ __device__ __forceinline__ uint64_t wg_sum(uint64_t v, Shared &sh) {
   return s;
 }
 
-// exclusive prefix over the workgroup's threads in thread order (rev: in reverse thread order)
-template <bool kRev>
-__device__ __forceinline__ uint64_t wg_excl(uint64_t v, Shared &sh) {
-  const int t = kRev ? kThreads - 1 - (int)threadIdx.x : (int)threadIdx.x;
-  // kRev: lanes and waves are walked from the top, so the wave scan runs over the mirrored lane
-  // (a shuffle of lane 63 - l) and the wave totals are combined from the last wave down
-  uint64_t x = kRev ? __shfl(v, 63 - lane_id(), 64) : v;
-  const uint64_t inc = wave_incl(x);
+// exclusive prefix over the workgroup's threads in thread order (kRev: in reverse thread order),
+// and the workgroup's total; `slot` is LDS that no other step of the workgroup uses
+template <bool kRev, typename T>
+__device__ __forceinline__ T wg_excl(T v, T *slot, T &total) {
+  // kRev: lanes are walked from the top, so the wave scan runs over the mirrored lane (a shuffle
+  // of lane 63 - l), and a wave adds the totals of the waves above it
+  const T x = kRev ? __shfl(v, 63 - lane_id(), 64) : v;
+  const T inc = wave_incl(x);
+  const int w = threadIdx.x >> 6;
+  if (lane_id() == 63) slot[w] = inc;
   __syncthreads();
-  if (lane_id() == 63) sh.qx[t >> 6] = inc;
-  __syncthreads();
-  uint64_t base = 0;
-  for (int w = 0; w < (t >> 6); w++) base += sh.qx[w];
-  const uint64_t ex = base + inc - x;
+  T base = 0, tot = 0;
+#pragma unroll
+  for (int o = 0; o < kWaves; o++) {
+    const T s = slot[o];
+    if (kRev ? o > w : o < w) base += s;
+    tot += s;
+  }
+  total = tot;
+  const T ex = base + inc - x;
   return kRev ? __shfl(ex, 63 - lane_id(), 64) : ex;
 }
 
@@ -246,8 +253,8 @@ struct SplitCut {
 struct SplitScratch {
   float max[kSplitRows][kSplitMax];
   unsigned long long sum[kSplitRows][kSplitMax];
-  int idx[kSplitRows][kSplitMax];             // greedy: first index; draws: members of key_t
-  unsigned long long wsum[kSplitRows][kSplitMax];  // draws: the slice's total weight
+  int idx[kSplitRows][kSplitMax];  // greedy: first index; draws: least value (until the cut), members of key_t
+  unsigned long long wsum[kSplitRows][kSplitMax];  // draws: the slice's weight above key_t
   SplitCut cut[kSplitRows];
   uint32_t hist[kSplitRows][kKeys];  // draws with a cut: the row's histogram of lp keys
 };
@@ -255,6 +262,41 @@ struct SplitScratch {
 // until the process ends.  On the host `g_split` names a stand-in, never device memory: host code
 // only passes the per-device address hipGetSymbolAddress returns (split_scratch_of_current_device).
 __device__ __align__(16) SplitScratch g_split;
+
+// A row's largest value, its integer sum and (kLeast, with `least`) its least value from the slice
+// partials: a row has at most a wave of slices, so every wave combines them itself, without LDS or
+// barriers.
+static_assert(kSplitMax == 64, "a lane a slice");
+struct Partials {
+  float max, least;
+  uint64_t sum;
+};
+
+__device__ __forceinline__ float row_max(const SplitScratch *sp, int b, int ns) {
+  const int l = lane_id();
+  return wave_max(l < ns ? sp->max[b][l] : -INFINITY);
+}
+
+template <bool kLeast>
+__device__ __forceinline__ Partials row_partials(const SplitScratch *sp, int b, int ns, int least) {
+  const int l = lane_id();
+  const float m = l < ns ? sp->max[b][l] : -INFINITY;
+  const uint64_t s = l < ns ? sp->sum[b][l] : 0ull;
+  const float n = kLeast && least && l < ns ? -__int_as_float(sp->idx[b][l]) : -INFINITY;
+  return Partials{wave_max(m), kLeast ? -wave_max(n) : 0.0f, wave_sum(s)};
+}
+
+// The keys a row's values can have, from its least and largest value: x - lse and its rounding are
+// monotone, so finite rows lie in [key of the least, key of the largest].  A row with a NaN (its
+// key lies below -inf's) or an infinity takes every key (least: -inf for a row with a NaN).
+struct KeyRange {
+  int lo, hi;
+};
+
+__device__ __forceinline__ KeyRange key_range(float least, float m0, float lse) {
+  if (!(least > -INFINITY) || !(m0 < INFINITY)) return KeyRange{0, kKeys - 1};
+  return KeyRange{key_of(bf16r(least - lse)), key_of(bf16r(m0 - lse))};
+}
 
 template <int kMode, bool kVec>
 __global__ __launch_bounds__(kThreads) void sample_rows_kernel(const SampleArgs a) {
@@ -267,9 +309,10 @@ __global__ __launch_bounds__(kThreads) void sample_rows_kernel(const SampleArgs 
   // (a.ns > 0: combined from the slice partials of split_max_kernel / split_sum_kernel)
   float m0 = -INFINITY;
   uint64_t S = 0;
+  float least = 0.0f;
   if (a.ns > 0) {
-    m0 = wg_max(t < a.ns ? a.sp->max[b][t] : -INFINITY, sh);
-    S = wg_sum(t < a.ns ? a.sp->sum[b][t] : 0ull, sh);
+    const Partials p = row_partials<kMode == kSample>(a.sp, b, a.ns, a.hist);
+    m0 = p.max, S = p.sum, least = p.least;
   } else {
     for_each<kVec>(row, V, [&](int, float x) { m0 = fmaxf(m0, x); });
     m0 = wg_max(m0, sh);
@@ -326,33 +369,40 @@ __global__ __launch_bounds__(kThreads) void sample_rows_kernel(const SampleArgs 
   }
 
   if constexpr (kMode == kSample) {
+    // With the histogram from split_hist_kernel this is a serial chain of reductions on one CU a
+    // row: only the row's own keys read, one barrier a scan, the tie search 64 ranks at a time
+    // (32 rows of 151,936: 12.9 -> 8.3 us).
     // bin k sits in slot hslot(k): a pad word after every 32 bins, so that the 32 bins of thread
     // t start at word 33 t and the lanes' element reads of them fall in distinct banks
     __shared__ uint32_t hist[kHistSlots];
-    if (a.hist) {  // the row's histogram from split_hist_kernel (all loads issued before the stores)
+    // The row's values sit in a narrow range of keys (a few hundred bins for logits of any
+    // spread), so the scans below give each thread a contiguous share of a range [kl, kh] that
+    // holds every non-empty key, in key order, rather than of all 32,768: the prefixes are the
+    // same (the empty bins add nothing), and the exp and roundings of the bins run in all 16 waves
+    // rather than in the one whose 32-bin stretches cover them.
+    int kl = kKeys, kh = -1;
+    if (a.hist) {
+      // the row's histogram from split_hist_kernel, over the keys the row can have: one CU reads
+      // 46 GB/s, so the whole 128 KB took 2.8 us (all loads issued before the stores)
+      const KeyRange kr = key_range(least, m0, lse);
+      kl = kr.lo, kh = kr.hi;
       constexpr int kCopy = kKeys / 4 / kThreads;
       uint4 q[kCopy];
 #pragma unroll
-      for (int i = 0; i < kCopy; i++) q[i] = ((const uint4 *)a.sp->hist[b])[t + i * kThreads];
+      for (int i = 0; i < kCopy; i++)
+        if (kl / 4 + t + i * kThreads <= kh / 4) q[i] = ((const uint4 *)a.sp->hist[b])[kl / 4 + t + i * kThreads];
 #pragma unroll
       for (int i = 0; i < kCopy; i++) {
-        uint32_t *d = hist + hslot(4 * (t + i * kThreads));  // (4 j .. 4 j + 3 lie in one run of 32)
+        if (kl / 4 + t + i * kThreads > kh / 4) break;
+        uint32_t *d = hist + hslot(4 * (kl / 4 + t + i * kThreads));  // (4 j .. 4 j + 3 lie in one run of 32)
         d[0] = q[i].x, d[1] = q[i].y, d[2] = q[i].z, d[3] = q[i].w;
       }
+      __syncthreads();
     } else {
       for (int j = t; j < kHistSlots; j += kThreads) hist[j] = 0u;
       __syncthreads();
       for_each<kVec>(row, V, [&](int, float x) { atomicAdd(&hist[hslot(key_of(bf16r(x - lse)))], 1u); });
-    }
-    __syncthreads();
-
-    // The row's values sit in a narrow range of keys (a few hundred bins for logits of any
-    // spread), so the scans below give each thread a contiguous share of the range of non-empty
-    // keys [kl, kh], in key order, rather than of all 32,768: the prefixes are the same (the
-    // empty bins add nothing), and the exp and roundings of the bins run in all 16 waves rather
-    // than in the one whose 32-bin stretches cover them.
-    int kl = kKeys, kh = -1;
-    {
+      __syncthreads();
       const uint32_t *own = hist + hslot(t * kBinsPerThread);  // (slots from 33 t: distinct banks)
       for (int j = 0; j < kBinsPerThread; j++)
         if (own[j]) kl = min(kl, t * kBinsPerThread + j), kh = max(kh, t * kBinsPerThread + j);
@@ -383,7 +433,8 @@ __global__ __launch_bounds__(kThreads) void sample_rows_kernel(const SampleArgs 
       uint64_t mass = 0;
       for (int k = kb; k < ke; k++)
         if (const uint32_t c = bin(k)) mass += (uint64_t)c * mass_of(k);
-      uint64_t cb = wg_excl<false>(mass, sh);  // (its barriers order the writes above)
+      uint64_t all;
+      uint64_t cb = wg_excl<false>(mass, sh.qx, all);  // (its barrier orders the writes above)
       int kc = -1;                             // the thread's bin where the kept mass starts
       uint64_t cbc = 0;
       for (int k = kb; k < ke; k++) {
@@ -393,17 +444,26 @@ __global__ __launch_bounds__(kThreads) void sample_rows_kernel(const SampleArgs 
         if (fix42_to_bf16(cb) <= a.thr && fix42_to_bf16(ce) > a.thr) kc = k, cbc = cb;
         cb = ce;
       }
-      if (kc >= 0) {
-        // the smallest j0 whose member (rank j0, cum cbc + (j0 + 1) Fc) survives
+      // the smallest j0 whose member (rank j0, cum cbc + (j0 + 1) Fc) survives: the wave of the
+      // thread that found the bin tries 64 ranks at a time (the last of the bin survives)
+      if (const unsigned long long m = __ballot(kc >= 0)) {
+        const int src = __builtin_ctzll(m);
+        kc = __shfl(kc, src, 64);
+        cbc = __shfl(cbc, src, 64);
         const uint64_t Fc = mass_of(kc);
         uint32_t lo = 0, hi = bin(kc) - 1;
         while (lo < hi) {
-          const uint32_t mid = (lo + hi) >> 1;
-          if (fix42_to_bf16(cbc + (uint64_t)(mid + 1) * Fc) > a.thr) hi = mid;
-          else lo = mid + 1;
+          const uint32_t step = (hi - lo + 63) / 64, j = min(hi, lo + (uint32_t)l * step);
+          const unsigned long long ok = __ballot(fix42_to_bf16(cbc + (uint64_t)(j + 1) * Fc) > a.thr);
+          if (!ok) {  // (only ranks past the last one tried are left)
+            lo = min(hi, lo + 63 * step + 1);
+            continue;
+          }
+          const uint32_t f = __builtin_ctzll(ok);
+          hi = min(hi, lo + f * step);
+          if (f) lo = lo + (f - 1) * step + 1;
         }
-        sh.cut[0] = kc;
-        sh.cut[1] = (int)lo;
+        if (l == 0) sh.cut[0] = kc, sh.cut[1] = (int)lo;
       }
     }
     __syncthreads();
@@ -421,19 +481,19 @@ __global__ __launch_bounds__(kThreads) void sample_rows_kernel(const SampleArgs 
     };
 
     // the kept set: keys above key_t, and the members of key_t's group of rank [r_lo, r_hi)
-    uint64_t nt = 0;
+    uint32_t nt = 0, n_surv;
     for (int k = kb; k < ke; k++) nt += surv(k, bin(k));
-    const uint64_t n_surv = wg_sum(nt, sh);
+    uint32_t above = wg_excl<true>(nt, sh.ux, n_surv);  // survivors in the bins of the threads above
     if (t == 0) {
       sh.cut[2] = key_p;                    // key_t
       sh.cut[3] = j0;                       // r_lo
       sh.cut[4] = (int)hist[hslot(key_p)];  // r_hi
     }
-    if (a.k > 0 && n_surv > (uint64_t)a.k) {
-      uint64_t above = wg_excl<true>(nt, sh);  // survivors in the bins of the threads above
+    if (a.k > 0 && n_surv > (uint32_t)a.k) {
+      __syncthreads();  // (thread 0's writes before the found cut's)
       for (int k = ke - 1; k >= kb; k--) {
         const uint32_t s = surv(k, bin(k));
-        if (above < (uint64_t)a.k && (uint64_t)a.k <= above + s) {
+        if (above < (uint32_t)a.k && (uint32_t)a.k <= above + s) {
           const int lo = (k == key_p) ? j0 : 0;
           sh.cut[2] = k;
           sh.cut[3] = lo;
@@ -573,47 +633,63 @@ struct SplitArgs {
   SplitScratch *sp;
 };
 
-template <bool kVec, typename F>
-__device__ __forceinline__ void slice_steps(const uint16_t *row, int lo, int hi, F &&f) {
-  for (int i0 = lo + 8 * (int)threadIdx.x; i0 < hi; i0 += 8 * kSplitThreads)
-    f(i0, load8<kVec>(row, i0, hi), min(8, hi - i0));
-}
+// A slice [lo, hi) of a row, walked by `kT` threads: kSliceAhead steps of 8 kT values are loaded
+// together, the first of them when the slice is set up, so that their latency runs beside the
+// reductions of the partials that a kernel begins with.  (kVec: lo and hi are multiples of 8.)
+constexpr int kSliceAhead = 3;
 
-template <bool kVec, typename F>
-__device__ __forceinline__ void slice_each(const uint16_t *row, int lo, int hi, F &&f) {
-  slice_steps<kVec>(row, lo, hi, [&](int i0, const Raw8 &q, int n) {
+template <bool kVec, int kT = kSplitThreads>
+struct Slice {
+  const uint16_t *row;
+  int i0, hi;  // the thread's next value
+  Raw8 q[kSliceAhead];
+
+  __device__ __forceinline__ Slice(const uint16_t *row_, int lo, int hi_)
+      : row(row_), i0(lo + 8 * (int)threadIdx.x), hi(hi_) {
+    load();
+  }
+  __device__ __forceinline__ void load() {
 #pragma unroll
-    for (int j = 0; j < 8; j++)
-      if (j < n) f(i0 + j, val(q, j));
-  });
-}
-
-__device__ __forceinline__ float split_max(float v, float *sh) {
-  v = wave_max(v);
-  __syncthreads();
-  if (lane_id() == 0) sh[threadIdx.x >> 6] = v;
-  __syncthreads();
-  float m = sh[0];
+    for (int u = 0; u < kSliceAhead; u++) q[u] = load8<kVec>(row, i0 + u * 8 * kT, hi);
+  }
+  // f(i, raw, n) for the thread's steps in order
+  template <typename F>
+  __device__ __forceinline__ void steps(F &&f) {
+    while (i0 < hi) {
 #pragma unroll
-  for (int w = 1; w < kSplitWaves; w++) m = fmaxf(m, sh[w]);
-  return m;
-}
+      for (int u = 0; u < kSliceAhead; u++) {
+        const int i = i0 + u * 8 * kT;
+        if (i < hi) f(i, q[u], kVec ? 8 : min(8, hi - i));
+      }
+      i0 += kSliceAhead * 8 * kT;
+      if (i0 < hi) load();
+    }
+  }
+  template <typename F>
+  __device__ __forceinline__ void each(F &&f) {
+    steps([&](int i, const Raw8 &r, int n) {
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        if (j < n) f(i + j, val(r, j));
+    });
+  }
+};
 
+// (`sh` is LDS that no other step of the workgroup uses)
+template <int kW = kSplitWaves>
 __device__ __forceinline__ unsigned long long split_sum(unsigned long long v, unsigned long long *sh) {
   v = wave_sum(v);
-  __syncthreads();
   if (lane_id() == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
   unsigned long long t = 0;
 #pragma unroll
-  for (int w = 0; w < kSplitWaves; w++) t += sh[w];
+  for (int w = 0; w < kW; w++) t += sh[w];
   return t;
 }
 
 __device__ __forceinline__ int split_min(int v, int *sh) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
-  __syncthreads();
   if (lane_id() == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
   int m = sh[0];
@@ -622,33 +698,36 @@ __device__ __forceinline__ int split_min(int v, int *sh) {
   return m;
 }
 
-// the row max from the slice maxima (thread t < ns reads slice t's)
-__device__ __forceinline__ float split_row_max(const SplitScratch *sp, int b, int ns, float *sh) {
-  return split_max((int)threadIdx.x < ns ? sp->max[b][threadIdx.x] : -INFINITY, sh);
-}
-
-template <bool kVec>
+template <bool kVec, bool kLeast>  // kLeast (draws with a cut): the least value too, for key_range
 __global__ __launch_bounds__(kSplitThreads) void split_max_kernel(const SplitArgs a) {
-  __shared__ float sh[kSplitWaves];
+  __shared__ float sh[kSplitWaves], shl[kSplitWaves];
   const int s = blockIdx.x, b = blockIdx.y;
-  const uint16_t *row = a.logits + (long long)b * a.V;
-  const int lo = s * a.len, hi = min(a.V, lo + a.len);
-  float m = -INFINITY;
-  slice_each<kVec>(row, lo, hi, [&](int, float x) { m = fmaxf(m, x); });
-  m = split_max(m, sh);
-  if (threadIdx.x == 0) a.sp->max[b][s] = m;
+  Slice<kVec> sl(a.logits + (long long)b * a.V, s * a.len, min(a.V, (s + 1) * a.len));
+  float m = -INFINITY, least = INFINITY;
+  sl.each([&](int, float x) {
+    m = fmaxf(m, x);
+    if (kLeast) least = x == x ? fminf(least, x) : -INFINITY;
+  });
+  m = wave_max(m);
+  if (kLeast) least = -wave_max(-least);
+  if (lane_id() == 0) sh[threadIdx.x >> 6] = m, shl[threadIdx.x >> 6] = least;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < kSplitWaves; w++) m = fmaxf(m, sh[w]), least = fminf(least, shl[w]);
+    a.sp->max[b][s] = m;
+    if (kLeast) a.sp->idx[b][s] = __float_as_int(least);
+  }
 }
 
 template <bool kVec>
 __global__ __launch_bounds__(kSplitThreads) void split_sum_kernel(const SplitArgs a) {
-  __shared__ float shf[kSplitWaves];
   __shared__ unsigned long long shq[kSplitWaves];
   const int s = blockIdx.x, b = blockIdx.y;
-  const uint16_t *row = a.logits + (long long)b * a.V;
-  const int lo = s * a.len, hi = min(a.V, lo + a.len);
-  const float m0 = split_row_max(a.sp, b, a.ns, shf);
+  Slice<kVec> sl(a.logits + (long long)b * a.V, s * a.len, min(a.V, (s + 1) * a.len));
+  const float m0 = row_max(a.sp, b, a.ns);
   uint64_t S = 0;
-  slice_each<kVec>(row, lo, hi, [&](int, float x) { S += fix42(exp_neg(x - m0)); });
+  sl.each([&](int, float x) { S += fix42(exp_neg(x - m0)); });
   S = split_sum(S, shq);
   if (threadIdx.x == 0) a.sp->sum[b][s] = S;
   if (a.hist) {  // the row's slices clear its histogram for split_hist_kernel
@@ -662,22 +741,23 @@ __global__ __launch_bounds__(kSplitThreads) void split_sum_kernel(const SplitArg
 // counts the values of hg consecutive slices in LDS and adds its non-empty bins to the row's.  The adds are system-scope
 // atomics (performed past the XCDs' L2s, so slices on different XCDs add to one copy); integer
 // adds, so the counts do not depend on their order.
+// Bound by latency, not by its 10 MB: 256 threads that cleared and read back all 32,768 bins, one
+// load in flight each, took 19.6 us at 32 rows of 151,936; 1024 threads over the keys that the row
+// can have take 6.6.
 template <bool kVec>
-__global__ __launch_bounds__(kSplitThreads) void split_hist_kernel(const SplitArgs a) {
+__global__ __launch_bounds__(kThreads) void split_hist_kernel(const SplitArgs a) {
   __shared__ __align__(16) uint32_t hist[kKeys];
-  __shared__ float shf[kSplitWaves];
-  __shared__ unsigned long long shq[kSplitWaves];
-  const int s = blockIdx.x, b = blockIdx.y, t = threadIdx.x;
-  const uint16_t *row = a.logits + (long long)b * a.V;
-  const int lo = s * a.hg * a.len, hi = min(a.V, lo + a.hg * a.len);
-  for (int i = t; i < kKeys / 4; i += kSplitThreads) ((uint4 *)hist)[i] = make_uint4(0u, 0u, 0u, 0u);
-  const float m0 = split_row_max(a.sp, b, a.ns, shf);
-  const uint64_t S = split_sum(t < a.ns ? a.sp->sum[b][t] : 0ull, shq);
-  const float lse = bf16r(m0 + log_ge1(fix42_to_f32(S)));
+  const int b = blockIdx.y, t = threadIdx.x;
+  const int lo = blockIdx.x * a.hg * a.len;
+  Slice<kVec, kThreads> sl(a.logits + (long long)b * a.V, lo, min(a.V, lo + a.hg * a.len));
+  const Partials p = row_partials<true>(a.sp, b, a.ns, 1);
+  const float lse = bf16r(p.max + log_ge1(fix42_to_f32(p.sum)));
+  const KeyRange kr = key_range(p.least, p.max, lse);
+  for (int k = kr.lo + t; k <= kr.hi; k += kThreads) hist[k] = 0u;
   __syncthreads();
-  slice_each<kVec>(row, lo, hi, [&](int, float x) { atomicAdd(&hist[key_of(bf16r(x - lse))], 1u); });
+  sl.each([&](int, float x) { atomicAdd(&hist[key_of(bf16r(x - lse))], 1u); });
   __syncthreads();
-  for (int k = t; k < kKeys; k += kSplitThreads) {
+  for (int k = kr.lo + t; k <= kr.hi; k += kThreads) {
     const uint32_t c = hist[k];
     if (c) __hip_atomic_fetch_add(&a.sp->hist[b][k], c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
@@ -685,18 +765,14 @@ __global__ __launch_bounds__(kSplitThreads) void split_hist_kernel(const SplitAr
 
 template <int kMode, bool kVec>
 __global__ __launch_bounds__(kSplitThreads) void split_final_kernel(const SplitArgs a) {
-  __shared__ float shf[kSplitWaves];
-  __shared__ unsigned long long shq[kSplitWaves];
   __shared__ int shi[kSplitWaves];
   const int s = blockIdx.x, b = blockIdx.y, t = threadIdx.x;
-  const uint16_t *row = a.logits + (long long)b * a.V;
-  const int lo = s * a.len, hi = min(a.V, lo + a.len);
-  const float m0 = split_row_max(a.sp, b, a.ns, shf);
-  const uint64_t S = split_sum(t < a.ns ? a.sp->sum[b][t] : 0ull, shq);
-  const float lse = bf16r(m0 + log_ge1(fix42_to_f32(S)));
+  Slice<kVec> sl(a.logits + (long long)b * a.V, s * a.len, min(a.V, (s + 1) * a.len));
+  const Partials p = row_partials<false>(a.sp, b, a.ns, 0);
+  const float m0 = p.max, lse = bf16r(m0 + log_ge1(fix42_to_f32(p.sum)));
   if constexpr (kMode == kLogprobs) {
     uint16_t *out = a.lp + (long long)b * a.V;
-    slice_steps<kVec>(row, lo, hi, [&](int i0, const Raw8 &q, int n) {
+    sl.steps([&](int i0, const Raw8 &q, int n) {
       uint32_t h[8];
 #pragma unroll
       for (int j = 0; j < 8; j++) h[j] = f2bf(val(q, j) - lse);
@@ -713,7 +789,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_final_kernel(const SplitA
   } else {
     const float lpmax = bf16r(m0 - lse);
     int best = a.V;
-    slice_each<kVec>(row, lo, hi, [&](int i, float x) {
+    sl.each([&](int i, float x) {
       if (bf16r(x - lse) == lpmax && i < best) best = i;
     });
     best = split_min(best, shi);
@@ -743,159 +819,112 @@ struct DrawArgs {
 
 // The row's cut: sample_rows_kernel's, or without top-p and top-k the one that keeps every value
 // (key_t 0, no partial tie group) with lse and m from the slice partials.
-__device__ __forceinline__ SplitCut split_cut(const DrawArgs &a, int b, float *shf, unsigned long long *shq) {
+__device__ __forceinline__ SplitCut split_cut(const DrawArgs &a, int b) {
   if (!a.nocut) return a.sp->cut[b];
-  const int t = threadIdx.x;
-  const float m0 = split_max(t < a.ns ? a.sp->max[b][t] : -INFINITY, shf);
-  const uint64_t S = split_sum(t < a.ns ? a.sp->sum[b][t] : 0ull, shq);
-  const float lse = bf16r(m0 + log_ge1(fix42_to_f32(S)));
-  return SplitCut{0, 0, 0, 0, 0, lse, bf16r(bf16r(m0 - lse) * a.inv_t)};
+  const Partials p = row_partials<false>(a.sp, b, a.ns, 0);
+  const float lse = bf16r(p.max + log_ge1(fix42_to_f32(p.sum)));
+  return SplitCut{0, 0, 0, 0, 0, lse, bf16r(bf16r(p.max - lse) * a.inv_t)};
 }
 
-// exclusive prefix over the workgroup's threads in thread order, and the workgroup's total
-template <typename T>
-__device__ __forceinline__ T split_excl(T v, T *sh, T &total) {
-  const T inc = wave_incl(v);
-  __syncthreads();
-  if (lane_id() == 63) sh[threadIdx.x >> 6] = inc;
-  __syncthreads();
-  T base = 0, tot = 0;
-#pragma unroll
-  for (int w = 0; w < kSplitWaves; w++) {
-    if (w < (int)(threadIdx.x >> 6)) base += sh[w];
-    tot += sh[w];
-  }
-  total = tot;
-  return base + inc - v;
+// the weight of a log-probability (kept values)
+__device__ __forceinline__ uint64_t weight_of(float lp, const SplitCut &c, float inv_t) {
+  return fix42(exp_neg(bf16r(lp * inv_t) - c.m));
 }
 
-// the members of key_t in slice s (partial cuts only)
-template <bool kVec>
-__global__ __launch_bounds__(kSplitThreads) void split_ties_kernel(const DrawArgs a) {
-  __shared__ unsigned long long sh[kSplitWaves];
-  const int s = blockIdx.x, b = blockIdx.y;
-  const SplitCut c = a.sp->cut[b];
-  if (c.done || !c.partial) return;
-  const uint16_t *row = a.logits + (long long)b * a.V;
-  const int lo = s * a.len, hi = min(a.V, lo + a.len);
-  unsigned long long n = 0;
-  slice_each<kVec>(row, lo, hi, [&](int, float x) { n += key_of(bf16r(x - c.lse)) == c.key_t; });
-  n = split_sum(n, sh);
-  if (threadIdx.x == 0) a.sp->idx[b][s] = (int)n;
-}
-
-// The weights of one 2048-value step of a slice from i0s (thread t: the 8 values from i0s + 8 t),
-// the ranks of key_t's members running on from `rank0` in vocabulary order; returns the step's
-// members.  W and the kept rule are sample_rows_kernel's.
-template <bool kVec>
-__device__ __forceinline__ uint32_t split_step_weights(const uint16_t *row, int i0s, int hi, const SplitCut &c,
-                                                       float inv_t, uint32_t rank0, uint32_t *shu, uint64_t W[8],
-                                                       int &n) {
-  const int i0 = i0s + 8 * (int)threadIdx.x;
-  const Raw8 q = load8<kVec>(row, i0, hi);
-  n = max(0, min(8, hi - i0));
-  int key[8];
-  uint32_t ties = 0;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    key[j] = j < n ? key_of(bf16r(val(q, j) - c.lse)) : -1;
-    ties += key[j] == c.key_t;
-  }
-  uint32_t total = 0;
-  uint32_t rank = c.partial ? rank0 + split_excl(ties, shu, total) : 0u;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    bool kept = key[j] > c.key_t;
-    if (key[j] == c.key_t) {
-      kept = !c.partial || ((int)rank >= c.r_lo && (int)rank < c.r_hi);
-      rank++;
-    }
-    W[j] = kept ? fix42(exp_neg(bf16r(bf16r(val(q, j) - c.lse) * inv_t) - c.m)) : 0ull;
-  }
-  return total;
-}
-
-// the members of key_t in the slices before s (partial cuts only)
-__device__ __forceinline__ uint32_t split_tie_base(const SplitScratch *sp, int b, int s, const SplitCut &c,
-                                                   unsigned long long *sh) {
-  if (!c.partial) return 0u;
-  const int t = threadIdx.x;
-  return (uint32_t)split_sum(t < s ? (unsigned long long)sp->idx[b][t] : 0ull, sh);
-}
-
-// the slice's total weight
+// The slice's weight above key_t and its members of key_t.  The members share one weight, so the
+// draw adds those of them that are kept once it has every slice's count: the counts need no launch
+// of their own before this one (4.9 + 8.9 us at 32 rows of 151,936, now 5.4).
 template <bool kVec>
 __global__ __launch_bounds__(kSplitThreads) void split_weights_kernel(const DrawArgs a) {
-  __shared__ float shf[kSplitWaves];
-  __shared__ unsigned long long shq[kSplitWaves];
-  __shared__ uint32_t shu[kSplitWaves];
+  __shared__ unsigned long long shq[2][kSplitWaves];
   const int s = blockIdx.x, b = blockIdx.y;
-  const SplitCut c = split_cut(a, b, shf, shq);
+  Slice<kVec> sl(a.logits + (long long)b * a.V, s * a.len, min(a.V, (s + 1) * a.len));
+  const SplitCut c = split_cut(a, b);
   if (c.done) return;
-  const uint16_t *row = a.logits + (long long)b * a.V;
-  const int lo = s * a.len, hi = min(a.V, lo + a.len);
-  uint32_t rank = split_tie_base(a.sp, b, s, c, shq);
-  unsigned long long tw = 0;
-  for (int i0s = lo; i0s < hi; i0s += 8 * kSplitThreads) {
-    uint64_t W[8];
-    int n;
-    rank += split_step_weights<kVec>(row, i0s, hi, c, a.inv_t, rank, shu, W, n);
-#pragma unroll
-    for (int j = 0; j < 8; j++) tw += W[j];
-  }
-  tw = split_sum(tw, shq);
-  if (threadIdx.x == 0) a.sp->wsum[b][s] = tw;
+  unsigned long long tw = 0, members = 0;
+  sl.each([&](int, float x) {
+    const float lp = bf16r(x - c.lse);
+    const int key = key_of(lp);
+    members += key == c.key_t;
+    if (key > c.key_t) tw += weight_of(lp, c, a.inv_t);
+  });
+  tw = split_sum(tw, shq[0]);
+  members = split_sum(members, shq[1]);
+  if (threadIdx.x == 0) a.sp->wsum[b][s] = tw, a.sp->idx[b][s] = (int)members;
 }
 
 // The draw: U = floor(u * total weight); the token is the number of i with C_i = sum_{j<i} W_j
 // <= U, less one.  The slices before the first slice whose prefix passes U count whole, the
-// slices after it none, and that slice is walked.
+// slices after it none, and that slice is walked, 8192 values a step, the ranks of key_t's members
+// running on from the slices before it in vocabulary order.  W and the kept rule are
+// sample_rows_kernel's.
+// A serial chain: the slices' prefixes live in a wave's lanes rather than behind barriers, and 1024
+// threads take most slices in one step (32 rows of 151,936: 8.6 -> 6.9 us; 256 threads took 3).
 template <bool kVec>
-__global__ __launch_bounds__(kSplitThreads) void split_draw_kernel(const DrawArgs a) {
-  __shared__ float shf[kSplitWaves];
-  __shared__ unsigned long long shq[kSplitWaves];
-  __shared__ uint32_t shu[kSplitWaves];
-  __shared__ unsigned long long pick[2];
-  const int b = blockIdx.x, t = threadIdx.x;
-  const SplitCut c = split_cut(a, b, shf, shq);
-  if (c.done) return;
-  const unsigned long long T = t < a.ns ? a.sp->wsum[b][t] : 0ull;
-  unsigned long long total;
-  const unsigned long long P = split_excl(T, shq, total);
+__global__ __launch_bounds__(kThreads) void split_draw_kernel(const DrawArgs a) {
+  __shared__ unsigned long long shq[2][kWaves];
+  __shared__ uint32_t shu[kWaves];
+  const int b = blockIdx.x, t = threadIdx.x, l = lane_id();
+  // the slices, one a lane, in every wave alike
+  unsigned long long T = l < a.ns ? a.sp->wsum[b][l] : 0ull;
+  const uint32_t members = l < a.ns ? (uint32_t)a.sp->idx[b][l] : 0u;
   float u = a.u[b];
+  const SplitCut c = split_cut(a, b);
+  if (c.done) return;
+  const uint32_t rank0 = wave_incl(members) - members;  // key_t's members in the slices before
+  const int kept = c.partial ? max(0, min((int)(rank0 + members), c.r_hi) - max((int)rank0, c.r_lo)) : (int)members;
+  T += (unsigned long long)kept * weight_of(value_of(c.key_t), c, a.inv_t);
+  const unsigned long long incl = wave_incl(T), P = incl - T, total = __shfl(incl, 63, 64);
   u = fminf(fmaxf(u, 0.0f), 0x1.fffffep-1f);  // (NaN -> 0)
   const uint64_t U = mul_u32_u64_hi((uint64_t)(u * 4294967296.0f), total);
-  if (t == 0) pick[0] = (unsigned long long)a.ns;
-  __syncthreads();
   // the first slice whose prefix with it passes U (the prefixes grow with the slice)
-  if (t < a.ns && P <= U && U < P + T) pick[0] = t, pick[1] = P;
-  __syncthreads();
-  const int s = (int)pick[0];
-  if (s >= a.ns) {  // (a total of 0: every C_i is 0)
+  const unsigned long long pick = __ballot(l < a.ns && P <= U && U < P + T);
+  if (!pick) {  // (a total of 0: every C_i is 0)
     if (t == 0) a.tok[b] = a.V - 1;
     return;
   }
+  const int s = __builtin_amdgcn_readfirstlane(__builtin_ctzll(pick));
   const uint16_t *row = a.logits + (long long)b * a.V;
   const int lo = s * a.len, hi = min(a.V, lo + a.len);
-  uint32_t rank = split_tie_base(a.sp, b, s, c, shq);
-  unsigned long long run = pick[1], cnt = 0;
-  for (int i0s = lo; i0s < hi; i0s += 8 * kSplitThreads) {
+  uint32_t first = __shfl(rank0, s, 64);  // the rank of the step's first member
+  unsigned long long run = __shfl(P, s, 64), cnt = 0;
+  for (int i0s = lo; i0s < hi; i0s += 8 * kThreads) {
+    const int i0 = i0s + 8 * t;
+    const Raw8 q = load8<kVec>(row, i0, hi);
+    const int n = max(0, min(8, hi - i0));
+    int key[8];
+    uint32_t ties = 0;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      key[j] = j < n ? key_of(bf16r(val(q, j) - c.lse)) : -1;
+      ties += key[j] == c.key_t;
+    }
+    uint32_t step_ties = 0;
+    uint32_t rank = c.partial ? first + wg_excl<false>(ties, shu, step_ties) : 0u;
+    first += step_ties;
     uint64_t W[8];
-    int n;
-    rank += split_step_weights<kVec>(row, i0s, hi, c, a.inv_t, rank, shu, W, n);
     unsigned long long lt = 0;
 #pragma unroll
-    for (int j = 0; j < 8; j++) lt += W[j];
+    for (int j = 0; j < 8; j++) {
+      bool kept = key[j] > c.key_t;
+      if (key[j] == c.key_t) {
+        kept = !c.partial || ((int)rank >= c.r_lo && (int)rank < c.r_hi);
+        rank++;
+      }
+      W[j] = kept ? weight_of(bf16r(val(q, j) - c.lse), c, a.inv_t) : 0ull;
+      lt += W[j];
+    }
     unsigned long long st;
-    unsigned long long cc = run + split_excl(lt, shq, st);  // C of the thread's first value
+    unsigned long long cc = run + wg_excl<false>(lt, shq[0], st);  // C of the thread's first value
 #pragma unroll
     for (int j = 0; j < 8; j++) {
       if (j < n && cc <= U) cnt++;
       cc += W[j];
     }
     run += st;
+    if (i0s + 8 * kThreads < hi) __syncthreads();  // (uniform; the next step writes the slots again)
   }
-  cnt = split_sum(cnt, shq);
+  cnt = split_sum<kWaves>(cnt, shq[1]);
   if (t == 0) a.tok[b] = (int32_t)((unsigned long long)lo + cnt - 1);
 }
 
@@ -904,10 +933,13 @@ __global__ __launch_bounds__(kSplitThreads) void split_draw_kernel(const DrawArg
 template <int kMode, bool kVec>
 int launch_split_vec(const SplitArgs &a, int B, hipStream_t st) {
   const dim3 grid(a.ns, B);
-  split_max_kernel<kVec><<<grid, kSplitThreads, 0, st>>>(a);
+  if (kMode == kSample && a.hist)
+    split_max_kernel<kVec, true><<<grid, kSplitThreads, 0, st>>>(a);
+  else
+    split_max_kernel<kVec, false><<<grid, kSplitThreads, 0, st>>>(a);
   split_sum_kernel<kVec><<<grid, kSplitThreads, 0, st>>>(a);
   if constexpr (kMode == kSample)
-    if (a.hist) split_hist_kernel<kVec><<<dim3((a.ns + a.hg - 1) / a.hg, B), kSplitThreads, 0, st>>>(a);
+    if (a.hist) split_hist_kernel<kVec><<<dim3((a.ns + a.hg - 1) / a.hg, B), kThreads, 0, st>>>(a);
   if constexpr (kMode != kSample) split_final_kernel<kMode, kVec><<<grid, kSplitThreads, 0, st>>>(a);
   if constexpr (kMode == kGreedy) split_argmin_kernel<<<B, 64, 0, st>>>(a.sp, a.ns, a.V, a.tok);
   return jit::check_launch(kMode == kGreedy ? "jit_argmax_rows" : kMode == kLogprobs ? "jit_logprobs_rows"
@@ -1020,8 +1052,8 @@ static int sample_rows(const uint16_t *logits, int B, int V, double temperature,
   // (without top-p and top-k every value is kept: no histogram, no cut)
   const int nocut = thr == 0.0f && k == 0;
   SplitArgs sa = split_args(logits, B, V, nullptr, nullptr, sp);
-  // the histogram over runs of slices, about 256 workgroups in all (each clears and scans 128 KB
-  // of LDS, so more of them with fewer values each cost more than they save)
+  // the histogram over runs of slices, about 256 workgroups in all: its 128 KB of LDS is one
+  // workgroup a CU
   sa.hist = !nocut;
   sa.hg = max(1, (sa.ns * B + 255) / 256);
   if (int rc = launch_split<kSample>(sa, B, stream)) return rc;
@@ -1033,13 +1065,11 @@ static int sample_rows(const uint16_t *logits, int B, int V, double temperature,
   const dim3 grid(sa.ns, B);
   const hipStream_t st = (hipStream_t)stream;
   if ((V & 7) == 0 && ((uintptr_t)logits & 15) == 0) {
-    if (!nocut) split_ties_kernel<true><<<grid, kSplitThreads, 0, st>>>(da);
     split_weights_kernel<true><<<grid, kSplitThreads, 0, st>>>(da);
-    split_draw_kernel<true><<<B, kSplitThreads, 0, st>>>(da);
+    split_draw_kernel<true><<<B, kThreads, 0, st>>>(da);
   } else {
-    if (!nocut) split_ties_kernel<false><<<grid, kSplitThreads, 0, st>>>(da);
     split_weights_kernel<false><<<grid, kSplitThreads, 0, st>>>(da);
-    split_draw_kernel<false><<<B, kSplitThreads, 0, st>>>(da);
+    split_draw_kernel<false><<<B, kThreads, 0, st>>>(da);
   }
   return jit::check_launch("jit_sample_rows");
 }

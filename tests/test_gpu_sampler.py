@@ -193,3 +193,33 @@ def test_sampler_contract():
     with pytest.raises(UnsupportedShape):
         ops.sample_rows(big, 1.0, 0.9, 5, u[:1])
     assert ops.sample_rows(x[:0], 1.0, 0.9, 5, u[:0]).shape == (0,)
+
+
+@pytest.mark.parametrize("V", [V_REF, 7007])
+def test_sample_rows_key_range_edges(V):
+    """Draws of up to 64 rows count and scan only the keys between a row's least and largest value;
+    65 rows take every key.  Both agree on rows with the type's lowest value, -inf, +inf or NaN as
+    masks, all equal, one value, or far below zero, cut by top-p, top-k, both or inside a tie group,
+    and on the rows without NaN or +inf with the oracle."""
+    x = sampler_logits(0, 12, V, 230, scale=3.0).astype(np.uint16)
+    bf = lambda v: f32_to_bf16(np.array([v], np.float32))[0]  # noqa: E731
+    keep = np.random.default_rng(231).random(V) < 0.2
+    x[1, ~keep] = np.uint16(0xFF7F)     # the lowest finite value
+    x[2, ~keep] = np.uint16(0xFF80)     # -inf
+    x[3, 5:] = np.uint16(0xFF80)
+    x[4] = bf(2.5)
+    x[5] = f32_to_bf16(np.random.default_rng(232).standard_normal(V).astype(np.float32) - 1000.0)
+    x[6] = f32_to_bf16(np.random.default_rng(233).standard_normal(V).astype(np.float32) * 1e-3)
+    x[7] = f32_to_bf16(np.random.default_rng(234).integers(-3, 3, V).astype(np.float32))
+    x[8] = np.uint16(0xFF80)
+    x[9, V // 2] = np.uint16(0x7FC0)    # NaN among numbers
+    x[10, 3] = np.uint16(0x7F80)        # +inf among numbers
+    x[11] = np.uint16(0x7FC0)
+    u = ((np.arange(12) * 7 % 12 + 0.5) / 12).astype(np.float32)
+    pad = np.concatenate([x, sampler_logits(5, 53, V, 235).astype(np.uint16)])
+    up = np.concatenate([u, np.full(53, 0.5, np.float32)])
+    for T, p, k in [(0.7, 0.95, 20), (1.0, 0.5, 0), (1.3, 1.0, V // 3), (1.0, 0.9, 4)]:
+        got = ops.sample_rows(bf16_tensor(x, DEV), T, p, k, torch.from_numpy(u).to(DEV)).cpu().numpy()
+        whole = ops.sample_rows(bf16_tensor(pad, DEV), T, p, k, torch.from_numpy(up).to(DEV)).cpu().numpy()[:12]
+        assert np.array_equal(got, whole), (T, p, k)
+        assert np.array_equal(got[:8], oracle.sample_rows(x[:8], T, p, k, u[:8])), (T, p, k)
