@@ -98,9 +98,9 @@ long long jit_moe_pack_workspace_bytes(int P, int E);
 
 /* jit_moe_pack with a device workspace of jit_moe_pack_workspace_bytes(P, E) bytes (contents on
  * entry do not matter): a long batch (a chunked-prefill step's B * k pairs,
- * Q36/model/moe.py:151-159 over the prefill rows) is packed by many workgroups in three launches
- * -- per-tile expert counts, one scan, per-tile placement -- instead of one workgroup walking every
- * tile.  The same tables, bit for bit (the stable order is unique).  With a workspace of 0 bytes
+ * Q36/model/moe.py:151-159 over the prefill rows) past 3,072 pairs is packed by many workgroups in three
+ * launches -- per-tile expert counts, one scan, per-tile placement -- instead of one workgroup walking every
+ * tile (up to 3,072 either entry takes one launch of a workgroup a tile).  The same tables, bit for bit (the stable order is unique).  With a workspace of 0 bytes
  * needed it is jit_moe_pack; a smaller workspace than needed returns JIT_EINVAL. */
 int jit_moe_pack_ws(const uint32_t *inds, int P, int k, int E, int32_t *order, int32_t *pair_row, int32_t *inv,
                     int32_t *expert_cnt, int32_t *expert_off, int32_t *seg_expert, int32_t *seg_start,

@@ -137,12 +137,12 @@ __device__ __forceinline__ int wave_incl_scan(int x, int l) {
 // The per-expert tables from each expert's pair count c (thread t: expert t, t < E; threads past
 // E pass c = 0): counts, first sorted positions, the ascending list of non-empty experts (their
 // segments) and meta = (segments, largest segment, bad pairs, 0).  nxt[t] receives expert t's
-// first position.  One workgroup of TH >= E threads.
+// first position.  One workgroup of TH >= E threads (write: it is the one that stores the tables).
 template <int TH>
 __device__ __forceinline__ void pack_tables(int c, int bad, int E, int *nxt, int32_t *__restrict__ expert_cnt,
                                             int32_t *__restrict__ expert_off, int32_t *__restrict__ seg_expert,
                                             int32_t *__restrict__ seg_start, int32_t *__restrict__ seg_cnt,
-                                            int32_t *__restrict__ meta) {
+                                            int32_t *__restrict__ meta, bool write = true) {
   __shared__ int wsum[(TH / 64)], wflag[(TH / 64)], wmax[(TH / 64)];
   const int t = threadIdx.x, w = t >> 6, l = t & 63;
   const int f = c > 0 ? 1 : 0;
@@ -167,6 +167,7 @@ __device__ __forceinline__ void pack_tables(int c, int bad, int E, int *nxt, int
   }
   const int off = cbase + cs - c;
   nxt[t] = off;
+  if (!write) return;
   if (t < E) {
     expert_cnt[t] = c;
     expert_off[t] = off;
@@ -257,6 +258,46 @@ __device__ __forceinline__ void pack_body(IndFn ind, int P, int k, int E, int32_
   pack_tables<TH>(cnt[t], bad, E, nxt, expert_cnt, expert_off, seg_expert, seg_start, seg_cnt, meta);
   for (int base = 0; base < P; base += TH)
     pack_place_tile<TH>(ind, base, P, k, E, nxt, wcnt, order, pair_row, inv);
+}
+
+// The packing of a middle batch in one launch, a workgroup a tile of TH pairs (TH >= E): each counts every
+// tile's pairs itself, those before its own tile apart, so its first positions need nothing from another
+// workgroup; workgroup 0 stores the tables.  Bound by the latency of the ids' loads (issued 16 at a time),
+// the LDS counts and the placement's barriers.  E = 128, us, one workgroup (to 2,048 pairs) or three launches
+// -> here: 768 pairs 5.3 -> 4.0, 1,024 6.6 -> 4.1, 2,048 11.6 -> 4.6, 2,400 8.1 -> 4.8; the experts of 192 rows
+// 105.9 -> 101.2, of 300 rows 107.7 -> 103.8, of 100 rows 82.1 -> 79.8.
+template <int TH>
+__global__ __launch_bounds__(TH) void pack_tiles_kernel(
+    const uint32_t *__restrict__ inds, int P, int k, int E, int32_t *__restrict__ order,
+    int32_t *__restrict__ pair_row, int32_t *__restrict__ inv, int32_t *__restrict__ expert_cnt,
+    int32_t *__restrict__ expert_off, int32_t *__restrict__ seg_expert,
+    int32_t *__restrict__ seg_start, int32_t *__restrict__ seg_cnt, int32_t *__restrict__ meta) {
+  __shared__ int cnt[2][TH + 1];  // [the tiles before this one][the others]; slot E: the bad pairs
+  __shared__ int nxt[TH];
+  __shared__ unsigned short wcnt[TH / 64][TH];
+  const int t = threadIdx.x, tile = blockIdx.x, tiles = gridDim.x;
+  cnt[0][t] = cnt[1][t] = 0;
+  if (t == 0) cnt[0][TH] = cnt[1][TH] = 0;
+  __syncthreads();
+  constexpr int kBatch = 16;
+  for (int i0 = 0; i0 < tiles; i0 += kBatch) {
+    int e[kBatch];
+#pragma unroll
+    for (int j = 0; j < kBatch; j++) {
+      const int p = (i0 + j) * TH + t;
+      e[j] = p < P ? (int)min(inds[p], (uint32_t)E) : -1;
+    }
+#pragma unroll
+    for (int j = 0; j < kBatch; j++)
+      if (e[j] >= 0) atomicAdd(&cnt[i0 + j < tile ? 0 : 1][e[j]], 1);
+  }
+  __syncthreads();
+  const int before = cnt[0][t];
+  pack_tables<TH>(t < E ? before + cnt[1][t] : 0, cnt[0][E] + cnt[1][E], E, nxt, expert_cnt, expert_off, seg_expert,
+                  seg_start, seg_cnt, meta, tile == 0);
+  nxt[t] += before;  // (thread t's own word)
+  __syncthreads();
+  pack_place_tile<TH>([&](int p) { return inds[p]; }, tile * TH, P, k, E, nxt, wcnt, order, pair_row, inv);
 }
 
 // The packing of a long batch over many workgroups (the one-workgroup kernel walks its tiles one
@@ -407,6 +448,28 @@ extern "C" int jit_topk(const uint16_t *gates, int rows, int N, int k, uint32_t 
   return launch_router<true>(gates, rows, N, k, 0, inds, nullptr, nullptr, (hipStream_t)stream);
 }
 
+// Batches packed in one launch of a workgroup a tile, by the tile's size; 0: not.  One tile of 256 pairs is
+// moe_pack_kernel's.  Past 3,072 pairs the launches that it saves are paid for in counts, since each workgroup counts
+// the whole batch from ids that are cold after a layer's weights: the experts of 512 rows (4,096 pairs) take 128.5 us
+// against 127.9 with three launches, of 2,108 rows 255.5 against 252.5, although the packing alone, warm, is 5.4
+// against 8.2 us and 8.9 against 9.5.
+static int pack_tile(int P, int E) {
+  if (P <= 256 || P > 3072) return 0;
+  return E <= 256 ? 256 : kPackThreads;
+}
+
+static void launch_pack_tiles(const uint32_t *inds, int P, int k, int E, int32_t *order, int32_t *pair_row,
+                              int32_t *inv, int32_t *expert_cnt, int32_t *expert_off, int32_t *seg_expert,
+                              int32_t *seg_start, int32_t *seg_cnt, int32_t *meta, hipStream_t st) {
+  const int tile = pack_tile(P, E), tiles = (P + tile - 1) / tile;
+  if (tile == 256)
+    pack_tiles_kernel<256><<<tiles, 256, 0, st>>>(inds, P, k, E, order, pair_row, inv, expert_cnt, expert_off,
+                                                  seg_expert, seg_start, seg_cnt, meta);
+  else
+    pack_tiles_kernel<kPackThreads><<<tiles, kPackThreads, 0, st>>>(inds, P, k, E, order, pair_row, inv, expert_cnt,
+                                                                    expert_off, seg_expert, seg_start, seg_cnt, meta);
+}
+
 extern "C" int jit_moe_pack(const uint32_t *inds, int P, int k, int E, int32_t *order,
                             int32_t *pair_row, int32_t *inv, int32_t *expert_cnt,
                             int32_t *expert_off, int32_t *seg_expert, int32_t *seg_start,
@@ -420,14 +483,19 @@ extern "C" int jit_moe_pack(const uint32_t *inds, int P, int k, int E, int32_t *
   if (P > 0 && (!inds || !order || !pair_row || !inv)) return jit::fail(JIT_EINVAL, "moe_pack: null pointer");
   // a decode batch's few pairs take the smallest workgroup that owns every expert (fewer waves
   // at each of the placement's barriers), and more than 128 pairs 256 threads (fewer tiles, each
-  // behind the same barriers: config 2's 256 pairs over 128 experts 3.90 -> 3.17 us); long batches
-  // take 1024 threads a tile
+  // behind the same barriers: config 2's 256 pairs over 128 experts 3.90 -> 3.17 us); batches past
+  // pack_tile's range take 1024 threads a tile
   const hipStream_t st = (hipStream_t)stream;
+  if (pack_tile(P, E)) {
+    launch_pack_tiles(inds, P, k, E, order, pair_row, inv, expert_cnt, expert_off, seg_expert, seg_start, seg_cnt, meta,
+                      st);
+    return jit::check_launch("jit_moe_pack");
+  }
 #define JIT_PACK(TH) moe_pack_kernel<TH><<<1, TH, 0, st>>>(inds, P, k, E, order, pair_row, inv, expert_cnt, \
                                                            expert_off, seg_expert, seg_start, seg_cnt, meta)
   if (P <= 128 && E <= 128)
     JIT_PACK(128);
-  else if (P <= 2048 && E <= 256)
+  else if (P <= 256 && E <= 256)
     JIT_PACK(256);
   else
     JIT_PACK(1024);
@@ -435,7 +503,8 @@ extern "C" int jit_moe_pack(const uint32_t *inds, int P, int k, int E, int32_t *
   return jit::check_launch("jit_moe_pack");
 }
 
-// Long batches take the three-launch packing over a workspace of per-tile counts.
+// The batches that ask for a workspace of per-tile counts; past pack_tile's range they take the three-launch packing
+// over it.
 static bool pack_multi(int P, int E) { return P > 2 * kPackThreads && E < kPackThreads; }
 
 extern "C" long long jit_moe_pack_workspace_bytes(int P, int E) {
@@ -460,6 +529,11 @@ extern "C" int jit_moe_pack_ws(const uint32_t *inds, int P, int k, int E, int32_
   if (!workspace || workspace_bytes < need)
     return jit::fail(JIT_EINVAL, "moe_pack: workspace of %lld bytes, %lld needed", workspace_bytes, need);
   const hipStream_t st = (hipStream_t)stream;
+  if (pack_tile(P, E)) {
+    launch_pack_tiles(inds, P, k, E, order, pair_row, inv, expert_cnt, expert_off, seg_expert, seg_start, seg_cnt, meta,
+                      st);
+    return jit::check_launch("jit_moe_pack_ws");
+  }
   const int tiles = (P + kPackThreads - 1) / kPackThreads;
   int32_t *ws = (int32_t *)workspace;
   pack_count_kernel<<<tiles, kPackThreads, 0, st>>>(inds, P, E, ws);

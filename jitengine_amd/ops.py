@@ -130,7 +130,7 @@ def moe_pack_into(inds: torch.Tensor, pk: Packing) -> None:
             "moe_pack",
         )
         return
-    # a long batch: three launches over a workspace of per-tile counts (jit_moe_pack_ws)
+    # a long batch: a workspace of per-tile counts, used past 3,072 pairs (jit_moe_pack_ws)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=inds.device)
     _lib.check(
         L.jit_moe_pack_ws(

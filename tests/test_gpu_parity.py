@@ -115,7 +115,7 @@ def test_pack_bit_exact(B, k, E):
 @pytest.mark.parametrize("P,k,E,skew,bad", [(2056, 8, 128, False, 0), (16864, 8, 128, True, 0),
                                              (50000, 5, 1023, True, 37), (3072, 1, 64, False, 5)])
 def test_pack_many_workgroups_equal_one(P, k, E, skew, bad):
-    """A long batch's three-launch packing (jit_moe_pack_ws) gives the one-workgroup kernel's
+    """A long batch's packing with a workspace (jit_moe_pack_ws) gives jit_moe_pack's
     tables bit for bit: skewed routing (segments of thousands of pairs), ids past E (dropped,
     inv = -1, counted in meta[2]), tiles that do not divide P."""
     from jitengine_amd import _lib
@@ -143,6 +143,32 @@ def test_pack_many_workgroups_equal_one(P, k, E, skew, bad):
     if bad == 0:  # (the oracle rejects ids past E)
         want = oracle.moe_pack(inds.reshape(-1, k), E)
         assert np.array_equal(multi.inv.cpu().numpy(), want["inv"])
+
+
+@pytest.mark.parametrize("E", [1, 63, 128, 256, 257, 1024])
+@pytest.mark.parametrize("P", [256, 257, 511, 512, 2048, 2049, 3072, 3073, 5121])
+def test_pack_tiles_are_the_stable_order(P, E):
+    """Packing at the edges of its tiles (256 and 1024 pairs) and of the ranges that take one workgroup, one
+    launch of many and three launches: the stable order by expert, skewed routing, ids past E dropped."""
+    rng = np.random.default_rng(P + E)
+    w = 1.0 / (1.0 + np.arange(E)) ** 1.2
+    inds = rng.choice(E, P, p=w / w.sum()).astype(np.uint32)
+    inds[rng.permutation(P)[:9]] = E + np.array([0, 1, 2, 500, 3, 0, 1 << 20, 7, 0xFFFFFFFF - E], np.uint32)
+    pk = ops.moe_pack(_i32(inds.reshape(-1, 1)), E)
+    ids = inds.astype(np.int64)
+    good = np.nonzero(ids < E)[0]
+    order = good[np.argsort(ids[good], kind="stable")]
+    cnt = np.bincount(ids[good], minlength=E)
+    off = np.cumsum(cnt) - cnt
+    inv = np.full(P, -1)
+    inv[order] = np.arange(order.size)
+    U = np.nonzero(cnt)[0]
+    got = {n: getattr(pk, n).cpu().numpy().astype(np.int64).reshape(-1) for n in (
+        "order", "pair_row", "inv", "expert_cnt", "expert_off", "seg_expert", "seg_start", "seg_cnt", "meta")}
+    assert got["meta"].tolist() == [U.size, cnt.max(), 9, 0]
+    for name, want in (("order", order), ("pair_row", order), ("inv", inv), ("expert_cnt", cnt), ("expert_off", off),
+                       ("seg_expert", U), ("seg_start", off[U]), ("seg_cnt", cnt[U])):
+        assert np.array_equal(got[name][:want.size], want), name
 
 
 # ----------------------------------------------------------------------------- projections
