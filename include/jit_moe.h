@@ -536,10 +536,11 @@ int64_t jit_layer_scratch_bytes(const jit_layer *layer, int rows, int mixed);
 
 /* A decode step's layer: x [B, D] (xn: its normed rows, or NULL) -> y [B, D], and with next_norm also the
  * rows normed for the next layer, xn_next.  One row: defer leaves the closing combine to the next layer,
- * which takes this call's scratch as `prev` (x and xn unused, y and xn_next not written). */
+ * which takes this call's scratch as `prev` and its layer as `prev_layer` (x and xn unused, y and xn_next not
+ * written).  The two layers share D; top-k, experts and widths may differ.  prev NULL: prev_layer is unused. */
 int jit_decode_layer(const jit_layer *layer, const jit_decode_rows *d, uint16_t *pool, const uint16_t *x,
-                     const uint16_t *xn, const void *prev, int defer, const uint16_t *next_norm,
-                     void *scratch, uint16_t *y, uint16_t *xn_next, void *stream);
+                     const uint16_t *xn, const jit_layer *prev_layer, const void *prev, int defer,
+                     const uint16_t *next_norm, void *scratch, uint16_t *y, uint16_t *xn_next, void *stream);
 
 /* A mixed prompt + decode step's layer over x [T, D], T = p->rows + d->B -> y [T, D]. */
 int jit_mixed_layer(const jit_layer *layer, const jit_prompt_rows *p, const jit_decode_rows *d, uint16_t *pool,

@@ -82,7 +82,7 @@ _SIGNATURES = {
     "jit_attn_workspace_bytes": [_I, _I],
     "jit_attn_split_workspace_bytes": [_I, _I, _I],
     "jit_layer_scratch_bytes": [_PL, _I, _I],
-    "jit_decode_layer": [_PL, _PD, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P],
+    "jit_decode_layer": [_PL, _PD, _P, _P, _P, _PL, _P, _I, _P, _P, _P, _P, _P],
     "jit_mixed_layer": [_PL, _PP, _PD, _P, _P, _P, _P, _P],
     "jit_paged_decode_attn_ws": [_P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _F, _I, _P, ctypes.c_int64, _P, _P],
     "jit_paged_decode_attn_qkv_ws": [_P, _P, _P, _F, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _F, _I, _P, ctypes.c_int64,

@@ -33,7 +33,7 @@ struct Scratch {
     };
     auto bf = [&](int64_t n) { return (uint16_t *)take(2 * n); };
     const int64_t B = rows, P = B * L.k, heads = (int64_t)L.H * JIT_HEAD_DIM;
-    // (what a deferred combine reads -- r, inv, scores, h -- comes first: its place depends on no flag)
+    // (what a deferred combine reads -- r, inv, scores, h -- comes first: its place depends on D and k alone)
     r = bf(P * L.D);
     h = bf(B * L.D);
     scores = bf(P);
@@ -137,8 +137,8 @@ extern "C" int64_t jit_layer_scratch_bytes(const jit_layer *layer, int rows, int
 }
 
 extern "C" int jit_decode_layer(const jit_layer *layer, const jit_decode_rows *d, uint16_t *pool, const uint16_t *x,
-                                const uint16_t *xn, const void *prev, int defer, const uint16_t *next_norm,
-                                void *scratch, uint16_t *y, uint16_t *xn_next, void *stream) {
+                                const uint16_t *xn, const jit_layer *prev_layer, const void *prev, int defer,
+                                const uint16_t *next_norm, void *scratch, uint16_t *y, uint16_t *xn_next, void *stream) {
   if (!d) return jit::fail(JIT_EINVAL, "decode_layer: null step");
   JIT_TRY(layer_check(layer, d->B, "decode_layer"));
   const jit_layer &L = *layer;
@@ -146,10 +146,16 @@ extern "C" int jit_decode_layer(const jit_layer *layer, const jit_decode_rows *d
   if ((prev || defer) && B != 1) return jit::fail(JIT_EINVAL, "decode_layer: a deferred combine takes one row");
   if (!scratch || (!prev && !x) || (!defer && !y) || (next_norm && !defer && !xn_next))
     return jit::fail(JIT_EINVAL, "decode_layer: null pointer");
+  if (prev) {
+    JIT_TRY(layer_check(prev_layer, 1, "decode_layer: previous layer"));
+    if (prev_layer->D != D)
+      return jit::fail(JIT_EINVAL, "decode_layer: a deferred row of %d for a layer of %d", prev_layer->D, D);
+  }
   const Scratch s(L, B, false, scratch);
   if (prev) {
-    const Scratch p(L, 1, false, (void *)prev);
-    JIT_TRY(jit_qmm_packed_combine_rmsnorm(p.r, p.inv, p.scores, L.k, p.h, L.input_norm, L.eps, D, L.qkv, nqkv, s.x,
+    // (the row's combine is the previous layer's: its tables, top-k and places in its scratch)
+    const Scratch p(*prev_layer, 1, false, (void *)prev);
+    JIT_TRY(jit_qmm_packed_combine_rmsnorm(p.r, p.inv, p.scores, prev_layer->k, p.h, L.input_norm, L.eps, D, L.qkv, nqkv, s.x,
                                            s.qkv, stream));
     x = s.x;
   } else {

@@ -371,7 +371,8 @@ class Model:
             scratch = torch.empty(lib.jit_layer_scratch_bytes(lp, B, 0), dtype=torch.uint8, device=dev)
             out = None if defer else torch.empty((1 if last else 2, B, D), dtype=torch.bfloat16, device=dev)
             _lib.check(lib.jit_decode_layer(
-                lp, dp, pool.data_ptr(), x.data_ptr(), ops._p(xn), ops._p(prev), int(defer),
+                lp, dp, pool.data_ptr(), x.data_ptr(), ops._p(xn), None if prev is None else ctypes.byref(lays[i - 1]),
+                ops._p(prev), int(defer),
                 None if last else self.layers[i + 1].input_norm.data_ptr(), scratch.data_ptr(),
                 None if defer else out[0].data_ptr(), None if defer or last else out[1].data_ptr(), stream),
                 "decode_layer")

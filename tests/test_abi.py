@@ -117,3 +117,24 @@ def test_workspace_bytes():
     assert lib.jit_moe_pack_workspace_bytes(16864, 128) == 17 * 129 * 4
     assert lib.jit_moe_pack_workspace_bytes(16864, 1024) == 0
     assert lib.jit_moe_pack_ws(None, 16864, 8, 128, *([None] * 9), None, 17 * 129 * 4 - 1, None) == _lib.JIT_EINVAL
+
+
+def test_deferred_rows_take_their_own_layer():
+    """A deferred combine needs the layer that left it, of the same width (its tables lie by that layer's top-k)."""
+    lib = _lib.lib()
+
+    def layer(D, k):
+        lay = _lib.Layer(D, 32, 4, 32, k, 768, 1, 1e-6, 0.1)
+        for name, ctype in lay._fields_[9:]:
+            setattr(lay, name, 256)  # (never dereferenced)
+        return lay
+
+    rows = _lib.DecodeRows(1, 1, 1)
+    one = ctypes.c_void_p(256)
+
+    def call(prev_layer):
+        return lib.jit_decode_layer(layer(2048, 8), rows, one, one, None, prev_layer, one, 0, None, one, one, None, None)
+
+    assert call(None) == _lib.JIT_EINVAL and b"previous layer" in lib.jit_last_error()
+    assert call(layer(1024, 8)) == _lib.JIT_EINVAL and b"1024" in lib.jit_last_error()
+    assert call(layer(2048, 0)) == _lib.JIT_EINVAL

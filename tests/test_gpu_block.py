@@ -361,3 +361,25 @@ def test_native_mixed_layer_matches_op_by_op(chunks, dec_pos):
     got = layer.mixed(x, other, ms)
     assert torch.equal(got, layer.mixed(x, pool, ms, debug={}))
     assert torch.equal(other, pool)
+
+
+def test_one_token_step_over_layers_of_different_top_k():
+    """Layers may differ in their top-k and their number of experts: a deferred combine takes the tables, the
+    scores and the slot count of the layer that left it (one token: the rows and pools of the op-by-op layers)."""
+    from jitengine_amd.model import DecoderLayer, Model, MoEConfig, random_layer_weights
+
+    cfgs = [MoEConfig(experts=e, layers=4, top_k=k) for e, k in ((32, 8), (32, 4), (64, 8), (32, 2))]
+    model = Model(cfgs[0], [])
+    model.layers = [DecoderLayer(c, random_layer_weights(c, 80 + l, DEV)) for l, c in enumerate(cfgs)]
+    st = model.make_state(np.array([77], np.int32), torch.arange(5, dtype=torch.int32, device=DEV).view(1, 5))
+    gen = torch.Generator(device=DEV).manual_seed(81)
+    pools = [torch.randn((5, 4, 2, 2048), generator=gen, device=DEV).to(torch.bfloat16) for _ in cfgs]
+    x = torch.randn((1, cfgs[0].hidden), generator=gen, device=DEV).to(torch.bfloat16)
+    got_pools = [p.clone() for p in pools]
+    got = model.decode_step(x, got_pools, st)
+    want = x
+    for layer, pool in zip(model.layers, pools):
+        want = layer.step(want, pool, st, debug={})
+    assert torch.equal(got, want)
+    for a, b in zip(got_pools, pools):
+        assert torch.equal(a, b)
