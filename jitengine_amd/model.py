@@ -153,8 +153,11 @@ class DecoderLayer:
 
     def native(self):
         """The layer as jit_decode_layer / jit_mixed_layer take it, or None where its weights are not all packed
-        matrices of the geometry (the op-by-op path then serves, and names what does not fit)."""
+        matrices of the geometry, or its MoE block's methods are not the ones the calls stand for (the op-by-op
+        path then serves, and names what does not fit)."""
         cfg, moe = self.cfg, self.moe
+        if _replaced(moe, MoEBlock, _MOE_METHODS):
+            return None
         D, E, I, Hd = cfg.hidden, moe.num_experts, moe.down.in_dims, cfg.heads * cfg.head_dim
         for w, stack, N, K in ((self.qkv, False, cfg.qkv_rows, D), (self.o, False, D, Hd), (moe.router, False, E, D),
                                (moe.gate_up, True, 2 * I, D), (moe.down, True, D, I)):
@@ -283,26 +286,47 @@ class DecoderLayer:
         """mixed as one native call (the same launches and bits; the attention halves write one buffer)."""
         T, D, dev, pf = x.shape[0], self.cfg.hidden, x.device, ms.prefill
         _rows_contract(x, D, pool, self.cfg.kv_heads)
-        for t, n in ((ms.pos_rows, "pos"), (ms.table_rows, "table_rows"), (ms.seq_table, "seq_table")):
+        for t, n in ((ms.pos_rows, "pos"), (ms.table_rows, "table_rows")):
             ops._need(t, torch.int32, n)
-        if T != ms.pos_rows.numel() or T != ms.table_rows.shape[0] or pf.rows != ms.P or T != ms.P + ms.decode.lens.shape[0]:
-            raise ValueError(f"x has {T} rows, the step {ms.P} prompt and {ms.decode.lens.shape[0]} decode rows")
-        ops.prefill_contract(pf, ms.seq_table)
-        need = ops.prefill_workspace_bytes(pf, self.cfg.heads) if ms.P else 0
-        pws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-        tb, bl = pf.tables.data_ptr(), pf.blocks.data_ptr()
-        C, nblk = pf.tables.shape[1], pf.blocks.shape[1]
-        p = _lib.PromptRows(ms.P, C, nblk, pf.pmax, pf.max_len, ms.seq_table.shape[1], ms.table_rows.shape[1],
-                            ms.pos_rows.data_ptr(), ms.table_rows.data_ptr(), ms.seq_table.data_ptr(), tb, tb + 4 * C,
-                            tb + 8 * C, tb + 12 * C, bl, bl + 4 * nblk, bl + 8 * nblk,
-                            pws.data_ptr() if need else None)
-        d, dws = _decode_rows(self.cfg, ms.dec_table, ms.decode, ms.workspace, dev)
+        nd = T - ms.P  # (a half without rows is not looked at: its plan and tables may be anything)
+        if (T != ms.pos_rows.numel() or T != ms.table_rows.shape[0] or nd < 0 or (ms.P and pf.rows != ms.P)
+                or (nd and ms.decode.lens.shape[0] != nd)):
+            raise ValueError(f"x has {T} rows, which the step's tables and its {ms.P} prompt rows do not match")
+        p = _lib.PromptRows(table_rows_pages=ms.table_rows.shape[1], pos=ms.pos_rows.data_ptr(),
+                            table_rows=ms.table_rows.data_ptr())
+        if ms.P:
+            ops._need(ms.seq_table, torch.int32, "seq_table")
+            ops.prefill_contract(pf, ms.seq_table)
+            need = ops.prefill_workspace_bytes(pf, self.cfg.heads)
+            pws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+            tb, bl = pf.tables.data_ptr(), pf.blocks.data_ptr()
+            C, nblk = pf.tables.shape[1], pf.blocks.shape[1]
+            p = _lib.PromptRows(ms.P, C, nblk, pf.pmax, pf.max_len, ms.seq_table.shape[1], p.table_rows_pages, p.pos,
+                                p.table_rows, ms.seq_table.data_ptr(), tb, tb + 4 * C, tb + 8 * C, tb + 12 * C, bl,
+                                bl + 4 * nblk, bl + 8 * nblk, pws.data_ptr() if need else None)
+        d, dws = _decode_rows(self.cfg, ms.dec_table, ms.decode, ms.workspace, dev) if nd else (_lib.DecodeRows(), None)
         lib = _lib.lib()
-        scratch = torch.empty(lib.jit_layer_scratch_bytes(ctypes.byref(lay), T, 1), dtype=torch.uint8, device=dev)
+        scratch = _layer_scratch(lib, lay, T, 1, dev)
         y = torch.empty_like(x)
         _lib.check(lib.jit_mixed_layer(ctypes.byref(lay), ctypes.byref(p), ctypes.byref(d), pool.data_ptr(),
                                        x.data_ptr(), scratch.data_ptr(), y.data_ptr(), ops._stream()), "mixed_layer")
         return y
+
+
+# What a layer's native calls do in place of: replaced in a subclass, an instance or the class itself, these are
+# called (the op-by-op path).
+_LAYER_METHODS = {"run": DecoderLayer.run}
+_MOE_METHODS = {"expert_mlp": MoEBlock.expert_mlp, "use_seg": MoEBlock.use_seg}
+
+
+def _replaced(obj, cls, methods: dict) -> bool:
+    return not isinstance(obj, cls) or any(
+        n in vars(obj) or getattr(type(obj), n) is not f for n, f in methods.items())
+
+
+def _layer_scratch(lib, lay, rows: int, mixed: int, device) -> torch.Tensor:
+    n = _lib.check(lib.jit_layer_scratch_bytes(ctypes.byref(lay), rows, mixed), "layer_scratch_bytes")
+    return torch.empty(n, dtype=torch.uint8, device=device)
 
 
 def _rows_contract(x: torch.Tensor | None, D: int, pool: torch.Tensor, Hkv: int) -> None:
@@ -338,8 +362,9 @@ class Model:
 
     def decode_step(self, x: torch.Tensor, pools: list, st: StepState) -> torch.Tensor:
         """x [B, D] bf16 hidden rows -> the last layer's output rows; pools[l] is layer l's KV pool."""
-        lays = [layer.native() for layer in self.layers] if x.shape[0] else [None]
-        if lays and None not in lays:
+        pools = [pool for _, pool in zip(self.layers, pools)]
+        lays = self._native_layers() if x.shape[0] else None
+        if lays:
             return self._decode_native(lays, x, pools, st)
         one = x.shape[0] == 1
         xn, carry = None, None
@@ -352,6 +377,17 @@ class Model:
             x, xn, carry = (None, None, out) if defer else (y, out, None)
         return x
 
+
+    def _native_layers(self):
+        """The layers as the native calls take them, or None where one is not of the model's geometry, has no such
+        form or replaces DecoderLayer.run."""
+        cfg, lays = self.cfg, []
+        for layer in self.layers:
+            lay = None if _replaced(layer, DecoderLayer, _LAYER_METHODS) else layer.native()
+            if lay is None or (lay.D, lay.H, lay.Hkv) != (cfg.hidden, cfg.heads, cfg.kv_heads):
+                return None
+            lays.append(lay)
+        return lays
 
     def _decode_native(self, lays: list, x: torch.Tensor, pools: list, st: StepState) -> torch.Tensor:
         """decode_step with a native call a layer (the same launches and bits)."""
@@ -368,7 +404,7 @@ class Model:
             last = i + 1 == n
             defer = B == 1 and not last and ops.row_prologue_fits(self.layers[i + 1].qkv, D)
             lp = ctypes.byref(lay)
-            scratch = torch.empty(lib.jit_layer_scratch_bytes(lp, B, 0), dtype=torch.uint8, device=dev)
+            scratch = _layer_scratch(lib, lay, B, 0, dev)
             out = None if defer else torch.empty((1 if last else 2, B, D), dtype=torch.bfloat16, device=dev)
             _lib.check(lib.jit_decode_layer(
                 lp, dp, pool.data_ptr(), x.data_ptr(), ops._p(xn), None if prev is None else ctypes.byref(lays[i - 1]),

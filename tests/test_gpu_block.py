@@ -383,3 +383,85 @@ def test_one_token_step_over_layers_of_different_top_k():
     assert torch.equal(got, want)
     for a, b in zip(got_pools, pools):
         assert torch.equal(a, b)
+
+
+def test_replaced_layer_methods_are_called():
+    """A subclass's, an instance's or a patched class's run, expert_mlp and use_seg are called by decode_step and
+    mixed, as the op-by-op path calls them; pools may be any iterable."""
+    from jitengine_amd.model import DecoderLayer, Model, MoEConfig, make_mixed_state, random_layer_weights
+    from jitengine_amd.moe import MoEBlock
+
+    calls = []
+
+    class Layer(DecoderLayer):
+        def run(self, *a, **k):
+            calls.append("run")
+            return super().run(*a, **k)
+
+    class Block(MoEBlock):
+        def expert_mlp(self, *a, **k):
+            calls.append("expert_mlp")
+            return super().expert_mlp(*a, **k)
+
+    cfg = MoEConfig(experts=32, layers=2)
+    weights = [random_layer_weights(cfg, 90 + l, DEV) for l in range(2)]
+    model = Model(cfg, weights)
+    table = np.arange(9, dtype=np.int32).reshape(3, 3)
+    gen = torch.Generator(device=DEV).manual_seed(91)
+    pools = [torch.randn((9, 4, 2, 2048), generator=gen, device=DEV).to(torch.bfloat16) for _ in range(2)]
+
+    def decode(B):
+        x = torch.randn((B, cfg.hidden), generator=torch.Generator(device=DEV).manual_seed(B), device=DEV)
+        st = model.make_state(np.array([9, 17, 30][:B], np.int32), _i32(table[:B]))
+        return model.decode_step(x.to(torch.bfloat16), (p.clone() for p in pools), st)
+
+    def mixed():
+        ms = make_mixed_state(cfg, [(0, 0, 20)], table[:1], [30], table[1:2], DEV)
+        x = torch.randn((21, cfg.hidden), generator=torch.Generator(device=DEV).manual_seed(3), device=DEV)
+        return model.layers[0].mixed(x.to(torch.bfloat16), pools[0].clone(), ms)
+
+    want = [decode(1), decode(3), mixed()]
+    assert calls == []
+
+    def check(names):
+        for got, w in zip((decode(1), decode(3), mixed()), want):
+            assert torch.equal(got, w)
+        assert set(calls) == set(names), calls
+        calls.clear()
+
+    plain = model.layers[1].moe
+    model.layers[1] = Layer(cfg, weights[1])
+    check(["run"])
+    model.layers[1] = DecoderLayer(cfg, weights[1])
+    blk = plain.expert_mlp
+    first = model.layers[0].moe
+    first.use_seg = lambda *a: calls.append("use_seg") or MoEBlock.use_seg(first, *a)
+    check(["use_seg"])
+    del first.use_seg
+    plain.expert_mlp = lambda *a, **k: calls.append("own") or blk(*a, **k)
+    model.layers[1].moe = plain
+    check(["own"])
+    model.layers[1].moe = Block(weights[1]["router"], weights[1]["gate_up"], weights[1]["down"], cfg.top_k)
+    check(["expert_mlp"])
+
+
+def test_mixed_step_without_one_half():
+    """A mixed step of prompt rows alone or decode rows alone looks at nothing of the other half."""
+    from dataclasses import replace
+
+    from jitengine_amd.model import DecoderLayer, MoEConfig, make_mixed_state, random_layer_weights
+
+    cfg = MoEConfig(experts=32, layers=1)
+    layer = DecoderLayer(cfg, random_layer_weights(cfg, 95, DEV))
+    table = np.arange(6, dtype=np.int32).reshape(2, 3)
+    pool = torch.randn((6, 4, 2, 2048), generator=torch.Generator(device=DEV).manual_seed(96), device=DEV)
+    pool = pool.to(torch.bfloat16)
+    for chunks, pos, gone in (([(0, 3, 20)], [], dict(dec_table=None, decode=None, workspace=None)),
+                              ([], [30, 4], dict(seq_table=None, prefill=None))):
+        ms = make_mixed_state(cfg, chunks, table[:len(chunks)], pos, table[:len(pos)], DEV)
+        x = torch.randn((ms.P + len(pos), cfg.hidden), device=DEV).to(torch.bfloat16)
+        a, b = pool.clone(), pool.clone()
+        assert torch.equal(layer.mixed(x, a, replace(ms, **gone)), layer.mixed(x, b, ms, debug={}))
+        assert torch.equal(a, b)
+        with pytest.raises(ValueError):
+            layer.mixed(torch.cat([x, x]), a, ms)
