@@ -119,11 +119,13 @@ struct SegShape {
 };
 
 // s_waitcnt vmcnt(N), nothing else.  Direct loads are counted by hand: the compiler does not see
-// the ones issued by inline assembly.
+// the ones issued by inline assembly, and it takes the wait itself for an instruction that touches no
+// memory: the fence after it keeps the reads of what has landed behind it.
 template <int N>
 __device__ __forceinline__ void seg_wait_vm() {
   static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+  asm volatile("" ::: "memory");
 }
 
 // s_waitcnt vmcnt(n) for a count known at run time (uniform), n in [LO, HI): the instruction's count
@@ -371,7 +373,6 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::
       if (p + DW <= last) load_w(p + DW);
       tiles(p, 0, bw0, [&](int t) { dequant_at(1, t >> 1, t & 1, bw1); });
       if (p < last) wait_w(p);
-      asm volatile("" ::: "memory");
       fetch_w(p + 1);  // (after the last step a stale stage, unused)
       tiles(p, 1, bw1, [&](int t) { dequant_at(0, t >> 1, t & 1, bw0); });
     }
