@@ -73,9 +73,9 @@ inline dim3 seg_grid(int nx, int groups) { return dim3(nx * 8 * ((groups + 7) / 
 // 8 packed-order nibbles of a word -> 8 bf16 weights bf16(s * q + b) in natural k order, 19 vector
 // instructions: a shift and a mask leave two nibbles in the low bits of a register's halves, where as
 // f16 denormals they are q 2^-24; v_fma_mix_f32 takes such a half as an operand, so s2 = 2^24 s (exact
-// for |s| < 2^104) times it plus b is the fp32 fma(s, q, b) in one instruction, where a byte conversion
-// and an fma were two (gate||up of 2,108 rows 147 -> 144 us, of 512 rows 78 -> 75 us; the same bits).
-// The weights are rounded in pairs (one v_cvt_pk_bf16_f32 each; s q + b is finite).
+// for |s| < 2^104; dequant_word_wide serves the others) times it plus b is the fp32 fma(s, q, b) in one
+// instruction, where a byte conversion and an fma were two (gate||up of 2,108 rows 147 -> 144 us, of 512 rows
+// 78 -> 75 us; the same bits).  The weights are rounded in pairs (one v_cvt_pk_bf16_f32 each).
 __device__ __forceinline__ Frag8 dequant_word(uint32_t w, float s2, float b) {
   Frag8 f;
 #pragma unroll
@@ -85,6 +85,17 @@ __device__ __forceinline__ Frag8 dequant_word(uint32_t w, float s2, float b) {
     asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(u), "v"(s2), "v"(b));
     asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(hi) : "v"(u), "v"(s2), "v"(b));
     f.u[j] = pack_bf16x2_rne(lo, hi);
+  }
+  return f;
+}
+
+// The same for any scale.
+__device__ __forceinline__ Frag8 dequant_word_wide(uint32_t w, float s, float b) {
+  Frag8 f;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const uint32_t u = w >> (4 * j);  // (q[2j] in bits 0-3, q[2j + 1] in bits 16-19)
+    f.u[j] = pack_bf16x2_rne(fmaf(s, (float)(u & 15u), b), fmaf(s, (float)((u >> 16) & 15u), b));
   }
   return f;
 }
@@ -394,9 +405,7 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::
     // (Whole tiles past the chunk are skipped: a branch uniform over the wave.)
     const __amdgpu_buffer_rsrc_t obuf = __builtin_amdgcn_make_buffer_rsrc((void *)a.out, (short)0, 0x7fffffff, 0x00020000);
     const int ntiles = (nt + 15) >> 4;
-#pragma unroll
-    for (int t = 0; t < TTS; t++) {
-      if (t >= ntiles) continue;
+    auto store_tile = [&](int t, const f32x4 (&c)[kSegRB]) {
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const int tok = 16 * t + 4 * lg + i;
@@ -404,18 +413,51 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::
         if (SWIGLU) {
           uint32_t hv;
           if constexpr (kTable)
-            hv = qtile::swiglu_bf16_tab(acc[t][0][i], acc[t][1][i], sig_tab);
+            hv = qtile::swiglu_bf16_tab(c[0][i], c[1][i], sig_tab);
           else
-            hv = qtile::swiglu_bf16(acc[t][0][i], acc[t][1][i]);
+            hv = qtile::swiglu_bf16(c[0][i], c[1][i]);
           __builtin_amdgcn_raw_buffer_store_b16((unsigned short)hv, obuf, (int)(ro + 2u * (16 * rbk[0] + lr)), 0, 0);
         } else {
 #pragma unroll
           for (int r = 0; r < kSegRB; r++)
-            __builtin_amdgcn_raw_buffer_store_b16((unsigned short)f2bf(acc[t][r][i]), obuf,
+            __builtin_amdgcn_raw_buffer_store_b16((unsigned short)f2bf(c[r][i]), obuf,
                                                   (int)(ro + 2u * (16 * rbk[r] + lr)), 0, 0);
         }
       }
+    };
+    // A scale past dequant_word's range is infinite there: its group's 64 weights are infinities and NaNs, and
+    // with them the sums of its row for every token.  So a token's sums that are not finite say that the wave's
+    // sums have to be made again: in the same order, by dequant_word_wide, a tile at a time and straight from
+    // memory (no barrier: other waves need not come here).  Inputs that are not finite come here too.
+    if (__any(!__builtin_isfinite(acc[0][0][0]) || !__builtin_isfinite(acc[0][1][0]))) {
+#pragma unroll 1
+      for (int t = 0; t < ntiles; t++) {
+        const int pos = off + c0 + min(16 * t + lr, nt - 1);
+        const uint16_t *xr = a.x + (uint32_t)(a.row_index ? a.row_index[pos] : pos) * (uint32_t)a.K + 16 * lg;
+        f32x4 c[kSegRB] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 1
+        for (int pg = 0; pg < 2 * GP; pg++) {
+          const int p = pg >> 1, g = pg & 1;
+          Frag8 xa[2];
+          xa[0].q = *(const uint4 *)(xr + 64 * pg);
+          xa[1].q = *(const uint4 *)(xr + 64 * pg + 8);
+#pragma unroll
+          for (int r = 0; r < kSegRB; r++) {
+            const uint8_t *blk = wexp + rbk[r] * tile_row;
+            const uint2 q = *(const uint2 *)(blk + p * qtile::kNibbleBytes + 16 * l + 8 * g);
+            const uint2 sb = *(const uint2 *)(blk + (long long)GP * qtile::kNibbleBytes + p * qtile::kScaleBytes + 8 * lr);
+            const float sc = bf2f((g ? sb.x >> 16 : sb.x) & 0xffffu), bi = bf2f((g ? sb.y >> 16 : sb.y) & 0xffffu);
+            c[r] = mfma16x16x32(xa[0], dequant_word_wide(q.x, sc, bi), c[r]);
+            c[r] = mfma16x16x32(xa[1], dequant_word_wide(q.y, sc, bi), c[r]);
+          }
+        }
+        store_tile(t, c);
+      }
+      continue;
     }
+#pragma unroll
+    for (int t = 0; t < TTS; t++)
+      if (t < ntiles) store_tile(t, acc[t]);
   }
 }
 

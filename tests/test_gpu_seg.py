@@ -234,3 +234,38 @@ def test_dense_segment_gemm_shapes(T, N, K):
     got = ops.qmm(x, ops.prepack(q), seg=True).double()
     tol = want.abs() * 2.0 ** -8 + K * 2.0 ** -24 * (x.double().abs() @ w.abs().t().contiguous())
     assert bool(((got - want).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("mean", [5, 9, 30, 40, 60, 120])
+def test_segment_gemm_takes_scales_of_any_size(mean):
+    """Scales from 2^104 to 2^112 (whose 2^24 multiple is past float32) in a few rows' groups, at every chunk
+    length (1, 2, 3, 4, 6 and 10 tiles), in gate rows, down rows and a dense matrix: the oracle's results, and the
+    rows and columns beside them untouched."""
+    E, N, K = 6, 256, 384
+    cnt = np.array([mean, mean - 2, mean + 3, 0, 2 * mean, mean - 1])
+    inds = np.random.default_rng(mean).permutation(np.repeat(np.arange(E), cnt)).astype(np.int32).reshape(-1, 1)
+    P = inds.size
+
+    def wide(q, rows):
+        for i, row in enumerate(rows):
+            q.scales[..., row, i % q.scales.shape[-1]] = (-1.0) ** i * 2.0 ** (104 + 8 * (i % 2))
+        return q
+
+    gu_h = wide(_stack(E, N, K, mean + 1), [0, 17, 18, 100, 127])
+    dn_h = wide(_stack(E, N, K, mean + 2), [3, 19, 130, 255])
+    x = normal_bf16((P, K), seed=mean)
+    pk = ops.moe_pack(torch.from_numpy(inds).to(DEV), E)
+    opk = oracle.moe_pack(inds.view(np.uint32), E)
+    h = ops.expert_gate_up(bf16_tensor(x, DEV), ops.prepack(gu_h.to(DEV)), pk, seg=True)
+    want = oracle.moe_gate_up(x, inds.view(np.uint32), opk, *stack_np(gu_h), bf16w=True)
+    assert assert_close_bf16(u16(h), want, what=f"wide gate_up mean {mean}")["bit_equal"] > 0.9
+    xs = bf16_tensor(x[opk["order"]], DEV)
+    r = ops.expert_down(xs, ops.prepack(dn_h.to(DEV)), pk, seg=True)
+    want = oracle.moe_down(u16(xs), inds.view(np.uint32), opk, *stack_np(dn_h), bf16w=True)
+    assert assert_close_bf16(u16(r), want, what=f"wide down mean {mean}")["bit_equal"] > 0.9
+    assert float(r[:, 3].float().abs().max()) > 2.0 ** 104 and bool(r.isfinite().all())
+    one = wide(random_quantized((512, K), mean), [0, 16, 511])
+    ids, opk = np.zeros((P, 1), np.uint32), oracle.moe_pack(np.zeros((P, 1), np.uint32), 1)
+    want = oracle.moe_down(x, ids, opk, *stack_np(QLinear(one.weight[None], one.scales[None], one.biases[None])), bf16w=True)
+    y = ops.qmm(bf16_tensor(x, DEV), ops.prepack(one.to(DEV)), seg=True)
+    assert assert_close_bf16(u16(y), want, what=f"wide dense {P} rows")["bit_equal"] > 0.9
