@@ -7,8 +7,8 @@
 // how many rows its expert has.
 //
 // Work split: a workgroup of WAVES waves (4 or 8) owns 32 WAVES weight rows of one expert (gate||up:
-// gate blocks and the up blocks of the same output columns, so SwiGLU is fused) and every token of
-// the expert's segment, in chunks of up to 16 * TTS tokens.  Each wave owns 2 row blocks (gate||up: a
+// gate blocks and the up blocks of the same output columns, so SwiGLU is fused) and one chunk of up to
+// 16 * TTS tokens of the expert's segment at a time.  Each wave owns 2 row blocks (gate||up: a
 // gate block and its up block).  K is walked in steps of one group pair (128 k): the wave
 // dequantizes its 2 row blocks' pair into bf16 MFMA B fragments once and uses them against every
 // token tile of the chunk, whose activations the workgroup stages in LDS (gathered through pair_row
@@ -25,6 +25,7 @@
 // every weight load issued before them.  128 experts, top-8, 2048 x 768, us (gate||up + down; 10 tiles
 // at every size before -> now): 64 rows 130 + 66 -> 49 + 33, 256 rows 124 + 68 -> 60 + 34, 512 rows
 // 128 + 70 -> 75 + 42, 1,024 rows 138 + 75 -> 101 + 60, 2,108 rows 153 + 93 -> 144 + 88.
+#include <algorithm>
 #include <cmath>
 
 #include "qtile.hpp"
@@ -52,6 +53,7 @@ struct SegArgs {
   int K, N;                   // N: output columns (I for gate||up, D for down)
   int T;                      // rows of a dense matrix (cnt null)
   int nx, groups;             // column blocks per group; groups = experts (or a dense matrix's token chunks)
+  int dealt;                  // groups of the grid: the experts, and groups that only take dealt chunks
 };
 
 // Workgroup -> (group, column block), XCD-aware.  MI355X deals the workgroups of a launch to its
@@ -60,12 +62,12 @@ struct SegArgs {
 // activation rows, so they are given consecutive slots of one XCD: group g goes to XCD g % 8,
 // and its nx blocks follow each other there, resident together, so the rows leave HBM (or the
 // last-level cache) once per group instead of once per column block.  The grid is padded to
-// 8 * ceil(groups / 8) groups; the padding's workgroups exit at once.
+// 8 * ceil(dealt / 8) groups; the padding's workgroups exit at once.
 __device__ __forceinline__ bool seg_block(const SegArgs &a, int &g, int &cb) {
   const int L = blockIdx.x, xcd = L & 7, slot = L >> 3;
   g = xcd + 8 * (slot / a.nx);
   cb = slot % a.nx;
-  return g < a.groups;
+  return g < a.dealt;
 }
 
 inline dim3 seg_grid(int nx, int groups) { return dim3(nx * 8 * ((groups + 7) / 8)); }
@@ -191,10 +193,49 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::
   extern __shared__ __attribute__((aligned(16))) uint8_t seg_lds[];
   int grp, cb;
   if (!seg_block(a, grp, cb)) return;  // grid padding (uniform over the workgroup)
-  const int e = DENSE ? 0 : grp;
-  const int cnt = DENSE ? a.T : a.cnt[e], off = DENSE ? 0 : a.off[e];
-  if (cnt <= 0) return;  // uniform over the workgroup
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id();
+  // Experts: a workgroup takes its expert's first chunk, and the chunks past the first of all experts are dealt
+  // to the column block's workgroups in equal runs, one more to those without a chunk of their own first (runs:
+  // the chunks of an expert that follow each other read its weights from L2).  An expert in many rows would
+  // otherwise be walked by one workgroup a column block while the chip waits, and in the shorter chunks of
+  // the mean segment: 128 experts, every row with the same 8 of them, gate||up + down, us, walked so / walked in
+  // 160 tokens / dealt: 100 rows 111 / 57 / 45, 300 rows 184 / 113 / 64, 2,108 rows 707 / 764 / 205.  Even routing pays
+  // for the count at the start (64 rows 78.3 -> 79.5).  Every wave counts for itself.
+  const int E = a.groups;
+  auto chunks_past_first = [&](int c) { return (uint32_t)max(c - 1, 0) / (uint32_t)kTokens; };
+  int next = 0, end = 0;  // the chunks past the first that this workgroup is dealt
+  int cnt = a.T, off = 0;
+  if (!DENSE) {
+    // (every load is issued before any is waited for: they are the first thing a workgroup waits for)
+    const int own = min(grp, E - 1);
+    cnt = a.cnt[own];
+    off = a.off[own];
+    auto two = [&](int b) {
+      const int c0 = a.cnt[min(b + l, E - 1)], c1 = a.cnt[min(b + 64 + l, E - 1)];
+      return (b + l < E ? chunks_past_first(c0) : 0u) + (b + 64 + l < E ? chunks_past_first(c1) : 0u);
+    };
+    uint32_t n = two(0);
+    for (int b = 128; b < E; b += 128) n += two(b);
+    if (grp >= E) cnt = 0;
+    if (__any(n > 0)) {
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) n += __shfl_xor(n, o, 64);
+      const int extra = __builtin_amdgcn_readfirstlane(n);
+      int none = 0, before = 0;  // experts without a pair; those of them before this workgroup's
+      for (int b = 0; b < E; b += 64) {
+        const unsigned long long m = __ballot(b + l < E && a.cnt[min(b + l, E - 1)] <= 0);
+        none += __builtin_popcountll(m);
+        before += __builtin_popcountll(grp >= b + 64 ? m : grp > b ? m & ((1ull << (grp - b)) - 1) : 0ull);
+      }
+      // the order: the groups past the experts, the experts without a pair, the others
+      const int past = a.dealt - E;
+      const int turn = grp >= E ? grp - E : cnt <= 0 ? past + before : past + none + grp - before;
+      const int each = extra / a.dealt, more = extra % a.dealt;
+      next = turn * each + min(turn, more);
+      end = next + each + (turn < more ? 1 : 0);
+    }
+    if (cnt <= 0 && next >= end) return;  // uniform over the workgroup
+  }
   const int lr = l & 15, lg = l >> 4;
   const int tid = threadIdx.x;
   const int GP = a.K >> 7;  // K steps (group pairs)
@@ -210,13 +251,16 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::
     else
       rbk[r] = kSegRB * (cb * WAVES + wave) + r;
   }
-  const uint8_t *wexp = a.w + (long long)e * a.w_estride;
+  const uint8_t *wexp, *wnib, *wscl;  // the expert's weights
   const long long tile_row = (long long)GP * qtile::kTileBytes;  // bytes of one row block's tiles
   // weight staging: nibble instruction r moves row block r's tile (lane l: its 16 B piece); the
   // scale instruction's lane l moves word l % 32 of row block l / 32's scale tile
-  const uint8_t *wnib = wexp + 16 * l;
-  const int rb_s = l >> 5 ? rbk[1] : rbk[0];
-  const uint8_t *wscl = wexp + rb_s * tile_row + (long long)GP * qtile::kNibbleBytes + 4 * (l & 31);
+  auto set_expert = [&](int e) {
+    wexp = a.w + (long long)e * a.w_estride;
+    wnib = wexp + 16 * l;
+    const int rb_s = l >> 5 ? rbk[1] : rbk[0];
+    wscl = wexp + rb_s * tile_row + (long long)GP * qtile::kNibbleBytes + 4 * (l & 31);
+  };
   const uint32_t wlds = lds0 + S::kWOff + wave * kSegWWave;  // + stage * kWStage
   const uint8_t *wmine = seg_lds + S::kWOff + wave * kSegWWave;
   auto load_w = [&](int p) {
@@ -255,11 +299,36 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::
   // fragment reads: lane (lr, lg) reads pieces 8 g + 2 lg and + 1 of row 16 t + lr
   const int frow = lr * 256;
 
-  const int cend = DENSE ? min(cnt, (grp + 1) * kTokens) : cnt;
-  const int cfirst = DENSE ? grp * kTokens : 0;
-  for (int c0 = cfirst; c0 < cend; c0 += kTokens) {
+  int c0 = DENSE ? grp * kTokens : 0;
+  set_expert(DENSE ? 0 : min(grp, E - 1));
+  for (bool own_chunk = DENSE || cnt > 0;; own_chunk = false) {
+    if (!DENSE && !own_chunk) {
+      if (next >= end) return;
+      const int item = next++;
+      uint32_t run = 0;
+      for (int b = 0;; b += 64) {
+        if (b >= E) return;  // (there are more than `item` of them: not reached)
+        const uint32_t v = b + l < E ? chunks_past_first(a.cnt[b + l]) : 0u;
+        uint32_t incl = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const uint32_t u = __shfl_up(incl, o, 64);
+          if (l >= o) incl += u;
+        }
+        const unsigned long long past = __ballot(run + incl > (uint32_t)item);
+        if (past) {
+          const int src = __builtin_ctzll(past), e = __builtin_amdgcn_readfirstlane(b + src);
+          c0 = (item - __builtin_amdgcn_readfirstlane(__shfl(run + incl - v, src, 64)) + 1) * kTokens;
+          cnt = a.cnt[e];
+          off = a.off[e];
+          set_expert(e);
+          break;
+        }
+        run += __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
+      }
+      __syncthreads();  // an earlier chunk's reads of the stages are done
+    }
     const int nt = min(kTokens, cnt - c0);
-    if (c0 != cfirst) __syncthreads();  // the previous chunk's reads of the stages are done
     const int last = GP - 1;
     // element offsets of this lane's pieces (x holds < 2^32 elements; rows past the segment re-read its
     // last row)
@@ -453,18 +522,19 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::
         }
         store_tile(t, c);
       }
-      continue;
-    }
+    } else {
 #pragma unroll
-    for (int t = 0; t < TTS; t++)
-      if (t < ntiles) store_tile(t, acc[t]);
+      for (int t = 0; t < TTS; t++)
+        if (t < ntiles) store_tile(t, acc[t]);
+    }
+    if (DENSE) return;
   }
 }
 
-// One launch of a shape: `cols` column blocks of its rows for each of a.groups groups (the kernels take
-// more LDS than the static limit: raise their dynamic limit once).
+// One launch of a shape: the column blocks of its rows for each of a.groups groups, P pairs in all (the kernels
+// take more LDS than the static limit: raise their dynamic limit once).
 template <bool SWIGLU, bool DENSE, class S>
-void seg_launch(SegArgs a, int rows, hipStream_t st) {
+void seg_launch(SegArgs a, int rows, hipStream_t st, int P = 0) {
   static const bool done = [] {
     (void)hipFuncSetAttribute((const void *)&seg_kernel<SWIGLU, DENSE, S>, hipFuncAttributeMaxDynamicSharedMemorySize,
                               S::kLds);
@@ -473,7 +543,12 @@ void seg_launch(SegArgs a, int rows, hipStream_t st) {
   (void)done;
   a.nx = rows / S::kRows;
   if (DENSE) a.groups = (a.T + S::kTokens - 1) / S::kTokens;
-  seg_kernel<SWIGLU, DENSE, S><<<seg_grid(a.nx, a.groups), S::kThreads, S::kLds, st>>>(a);
+  a.dealt = a.groups;
+  if (!DENSE) {  // as many groups as dealt chunks may need, where the experts' own leave room on an XCD's CUs
+    const int room = 8 * (jit::cu_count() / 8 * (S::WAVES == 4 ? 3 : 1) / a.nx) - a.groups;
+    a.dealt += std::max(0, std::min(room, P / S::kTokens));
+  }
+  seg_kernel<SWIGLU, DENSE, S><<<seg_grid(a.nx, a.dealt), S::kThreads, S::kLds, st>>>(a);
 }
 
 // The chunk length of expert segments: the smallest that holds the mean segment plus 2.5 of its
@@ -485,17 +560,17 @@ template <bool SWIGLU>
 void seg_experts(const SegArgs &a, int rows, int P, hipStream_t st) {
   const float mean = (float)P / (float)a.groups, need = mean + 2.5f * sqrtf(mean);
   if (need <= 16.0f)
-    seg_launch<SWIGLU, false, SegShape<1, 4, 2, 2, 4>>(a, rows, st);
+    seg_launch<SWIGLU, false, SegShape<1, 4, 2, 2, 4>>(a, rows, st, P);
   else if (need <= 32.0f)
-    seg_launch<SWIGLU, false, SegShape<2, 4, 2, 2, 3>>(a, rows, st);
+    seg_launch<SWIGLU, false, SegShape<2, 4, 2, 2, 3>>(a, rows, st, P);
   else if (need <= 48.0f)
-    seg_launch<SWIGLU, false, SegShape<3, 4, 1, 2, 3>>(a, rows, st);
+    seg_launch<SWIGLU, false, SegShape<3, 4, 1, 2, 3>>(a, rows, st, P);
   else if (need <= 64.0f)
-    seg_launch<SWIGLU, false, SegShape<4, 4, 1, 2, 3>>(a, rows, st);
+    seg_launch<SWIGLU, false, SegShape<4, 4, 1, 2, 3>>(a, rows, st, P);
   else if (need <= 96.0f)
-    seg_launch<SWIGLU, false, SegShape<6, 8, 1, 2>>(a, rows, st);
+    seg_launch<SWIGLU, false, SegShape<6, 8, 1, 2>>(a, rows, st, P);
   else
-    seg_launch<SWIGLU, false, SegShape<10, 8, 1, 2>>(a, rows, st);
+    seg_launch<SWIGLU, false, SegShape<10, 8, 1, 2>>(a, rows, st, P);
 }
 
 // The chunk length of a dense matrix (its token chunks spread over workgroups): the least estimated

@@ -269,3 +269,41 @@ def test_segment_gemm_takes_scales_of_any_size(mean):
     want = oracle.moe_down(x, ids, opk, *stack_np(QLinear(one.weight[None], one.scales[None], one.biases[None])), bf16w=True)
     y = ops.qmm(bf16_tensor(x, DEV), ops.prepack(one.to(DEV)), seg=True)
     assert assert_close_bf16(u16(y), want, what=f"wide dense {P} rows")["bit_equal"] > 0.9
+
+
+@pytest.mark.parametrize("E,K", [(12, 256), (70, 128), (200, 256)])
+@pytest.mark.parametrize("rows", [24, 150, 400, 1100])
+def test_segment_gemm_deals_the_chunks_of_hot_experts(E, K, rows):
+    """Experts of many chunks under a short mean segment, whose chunks past the first go to other workgroups: a
+    few hot experts among empty ones, one expert with every pair, and every expert in uneven numbers, with
+    fewer and more such chunks than workgroups.  Every row has the bits it has alone in a batch of its expert."""
+    N = 256
+    gu_h, dn_h = _stack(E, N, K, E + 1), _stack(E, N, K, E + 2)
+    gu, dn = ops.prepack(gu_h.to(DEV)), ops.prepack(dn_h.to(DEV))
+    x = bf16_tensor(normal_bf16((rows, K), seed=rows), DEV)
+    rng = np.random.default_rng(E + rows)
+    w = 1.0 / (1.0 + np.arange(E)) ** 1.3
+    for kind in ("hot", "one", "uneven"):
+        k = {"hot": 3, "one": 1, "uneven": 2}[kind]
+        if kind == "hot":
+            inds = np.tile(np.array([2, E - 1, E // 2], np.int32), (rows, 1))
+        elif kind == "one":
+            inds = np.full((rows, 1), E - 2, np.int32)
+        else:
+            inds = np.stack([rng.choice(E, k, replace=False, p=w / w.sum()) for _ in range(rows)]).astype(np.int32)
+        pk = ops.moe_pack(torch.from_numpy(inds).to(DEV), E)
+        h = ops.expert_gate_up(x, gu, pk, seg=True)
+        xs = x[pk.pair_row[:rows * k].long()].contiguous()
+        r = ops.expert_down(xs, dn, pk, seg=True)
+        cnt, off = pk.expert_cnt.cpu().numpy(), pk.expert_off.cpu().numpy()
+        for e in np.nonzero(cnt)[0][[0, -1]] if kind == "uneven" else np.nonzero(cnt)[0]:
+            pairs = slice(int(off[e]), int(off[e] + cnt[e]))
+            one = np.zeros((int(cnt[e]), 1), np.int32)  # the expert's rows as a whole batch
+            pk1 = ops.moe_pack(torch.from_numpy(one).to(DEV), 1)
+            part = [ops.prepack(QLinear(q.weight[e:e + 1], q.scales[e:e + 1], q.biases[e:e + 1]).to(DEV))
+                    for q in (gu_h, dn_h)]
+            assert torch.equal(h[pairs], ops.expert_gate_up(xs[pairs].contiguous(), part[0], pk1, seg=True)), (kind, e)
+            assert torch.equal(r[pairs], ops.expert_down(xs[pairs].contiguous(), part[1], pk1, seg=True)), (kind, e)
+        opk = oracle.moe_pack(inds.view(np.uint32), E)
+        want = oracle.moe_down(u16(xs), inds.view(np.uint32), opk, *stack_np(dn_h), bf16w=True)
+        assert assert_close_bf16(u16(r), want, what=f"{kind} down")["bit_equal"] > 0.9
