@@ -754,15 +754,31 @@ int dense_gpw(int K) {
 #ifndef JIT_DENSE_WALK_N
 #define JIT_DENSE_WALK_N 16384
 #endif
+// Whether a tall matrix walks its row tiles (qmm_walk_kernel): two row tiles of 32 rows a CU or more (N = 16,384,
+// K = 2048: 32 rows 13.0 -> 10.1 us, 64 rows 22 -> 15; below, workgroups of one or two tiles do not repay the walk),
+// and waves enough in its one or two workgroups a CU to cover the loads: a short K has few (K / 64 / GPW).
+// us, qmm_kernel / walk:
+//   K = 256 (2 waves) N = 151,936: 8 rows 7.9 / 11.7, 64 rows 29 / 36, 65 rows 36 / 41, 191 rows 0.71 of the time;
+//   K = 512 (4 waves): 8 rows 11.8 / 14.2, 17 rows 23.3 / 24.4, 32 rows 0.94; N = 20,480: 33 rows 6.7 / 7.6;
+//   K = 1024 (8 waves of 2 groups): 1 row N = 248,320 29.1 / 31.5, 16 rows N = 151,936 0.78, N = 16,384 5.2 / 5.6;
+//   K = 2048 (8 waves of 4): 1 row N = 16,384 5.7 / 6.8, N = 32,768 9.9 / 10.3, N = 40,960 0.95; 16 rows N =
+//   16,384 7.8 / 8.9; K = 1536 (6 waves): 1 row N = 18,432 0.86.
+bool walks(const QmmArgs &a, int gpw) {
+  const int waves = a.K / 64 / gpw;
+  if (a.N < JIT_DENSE_WALK_N) return false;
+  if (waves <= 2) return a.T > 96;
+  if (waves <= 4) return a.T > 56 || (a.T > 24 && a.N >= 24576);
+  if (a.T > 16) return true;
+  return a.N > JIT_DENSE_WALK_N && (a.T > 4 || (gpw == 4 && (waves < 8 || a.N >= 40960)));
+}
+
 template <bool PACKED, int GPW>
 int launch_dense_gpw(const QmmArgs &a, hipStream_t st, const char *what) {
   // (16-byte output stores: an output that is not 16-byte aligned keeps qmm_kernel's 2-byte ones)
   const bool aligned = ((uintptr_t)a.out & 15) == 0;
-  // a tall matrix: two row tiles of 32 rows a CU or more (N = 16,384: 32 rows 13.0 -> 10.1 us, 64 rows 22 ->
-  // 15; below, workgroups of one or two tiles do not repay the walk).  K slices of 6 or 8 groups a wave
-  // would not leave registers for the activations of 64 tokens.
+  // K slices of 6 or 8 groups a wave would not leave registers for the activations of 64 tokens
   if constexpr (PACKED && GPW <= 4) {
-    if (aligned && a.N >= JIT_DENSE_WALK_N) {
+    if (aligned && walks(a, GPW)) {
       if (a.T <= 16) return launch_walk<2, GPW, 1>(a, 2, st, what);
       if (a.T <= 32) return launch_walk<2, GPW, 2>(a, 1, st, what);
       return launch_walk<2, GPW, 4>(a, 1, st, what);

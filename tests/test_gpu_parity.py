@@ -530,10 +530,12 @@ def test_expert_and_combine_calls_reject_mismatched_packing():
 
 
 @pytest.mark.parametrize("N,K", [(16384, 2048), (16400, 2048), (20000, 512), (16400, 1024), (5120, 2048), (2048, 4096),
-                                 (144, 3072), (48, 256)])
+                                 (144, 3072), (48, 256), (18448, 256), (24592, 512), (16400, 768), (16400, 1536),
+                                 (40976, 2048)])
 def test_dense_projection_shapes_agree(N, K):
     """Each launch shape of the packed dense projection (tall matrices walk row tiles with the activations
-    of 16, 32 or 64 tokens in registers; past 64 tokens the others take 64-row workgroups) at the edges
+    of 16, 32 or 64 tokens in registers, by their rows, K and tokens; past 64 tokens the others take 64-row workgroups,
+    or 16-row ones while those about fit the CUs) at the edges
     of its token tiles and with a partial last row tile: every row's bits are those of the row alone
     in a matrix of fewer than 16,384 rows (the one-tile shape), and an output that is not 16-byte aligned
     gets the same bits."""
@@ -547,7 +549,7 @@ def test_dense_projection_shapes_agree(N, K):
     x = bf16_tensor(normal_bf16((130, K), seed=N), DEV)
     one = torch.cat([torch.cat([ops.qmm(x[t:t + 16].contiguous(), p, seg=False) for p in parts], 1)
                      for t in range(0, 130, 16)])
-    for T in (1, 15, 16, 17, 32, 33, 49, 64, 65, 96, 97, 130):
+    for T in (1, 4, 5, 15, 16, 17, 24, 25, 32, 33, 49, 64, 65, 96, 97, 130):
         assert torch.equal(ops.qmm(x[:T].contiguous(), pk, seg=False), one[:T]), T
     buf = torch.empty(130 * N + 1, dtype=torch.bfloat16, device=DEV)
     y = buf[1:].view(130, N)
