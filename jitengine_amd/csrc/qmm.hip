@@ -791,15 +791,21 @@ int launch_dense_gpw(const QmmArgs &a, hipStream_t st, const char *what) {
   if (tiles <= JIT_DENSE_ZMAX)
     return wide ? launch_qmm<2, GPW, false, PACKED, 1>(a, 1, st, what, tiles)
                 : launch_qmm<1, GPW, false, PACKED, 1>(a, 1, st, what, tiles);
-  // longer batches take 64-row workgroups: what bounds them is the activations, which each workgroup pulls
+  // Longer batches take 64-row workgroups: what bounds them is the activations, which each workgroup pulls
   // through L2 for all its rows.  Two token tiles a pass where the K slice is short (N = 5120, K = 2048: 100
   // rows 16.7 -> 13.9 us, 160 rows 24.4 -> 16.1; N = 128, 2,108 rows 15 -> 10), one where it is long (N = 2048,
   // K = 4096: 100 rows 19.4 -> 10.7 us, 160 rows 28.5 -> 19.1; two tiles 24.5 and 27.2).
-  if (aligned) {
-    constexpr int TT = GPW <= 4 ? 2 : 1;
-    return launch_qmm<4, GPW, false, PACKED, TT>(a, 1, st, what, (tiles + TT - 1) / TT);
-  }
+  // Not while the 16-row workgroups of two token tiles about fit the CUs: then a call takes as long as one workgroup,
+  // and four times the rows only make it longer.  us, 64 rows / 16 rows at K = 2048: N = 128, 100 to 1,024 rows 7.9 /
+  // 6.1, 1,500 rows 8.4 / 11.4; N = 1024, 129 rows 8.4 / 7.3, 161 rows 8.0 / 9.8; unpacked, which has more to do
+  // a word, N = 128, 700 rows 11.5 / 7.2, N = 2048, 81 rows 11.6 / 10.5, and with the shortest K slice up to twice
+  // the CUs (N = 256, K = 1024, 1,024 rows 8.6 / 7.8).  A packed long K slice gains at any size (0.5 to 0.92 of the
+  // time), an unpacked one past the CUs (K = 4096, N = 1024: 97 rows 16.6 / 11.9, 150 rows 0.82 of the time).
   const int passes = (tiles + 1) / 2;
+  constexpr int TT = GPW <= 4 ? 2 : 1;
+  constexpr int kFit = PACKED ? (GPW <= 4 ? 9 : 0) : GPW == 2 ? 16 : GPW == 4 ? 12 : 8;  // eighths of the CUs
+  if (aligned && (long long)a.N * a.T > kFit * 64LL * jit::cu_count())  // (16 x 32 outputs a workgroup)
+    return launch_qmm<4, GPW, false, PACKED, TT>(a, 1, st, what, (tiles + TT - 1) / TT);
   return wide ? launch_qmm<2, GPW, false, PACKED, 2>(a, 1, st, what, passes)
               : launch_qmm<1, GPW, false, PACKED, 2>(a, 1, st, what, passes);
 }

@@ -557,6 +557,23 @@ def test_dense_projection_shapes_agree(N, K):
     assert torch.equal(y, one)
 
 
+@pytest.mark.parametrize("N,K", [(16, 2048), (112, 1024), (400, 256), (1040, 2048), (272, 4096), (1024, 2560)])
+def test_narrow_projection_shapes_agree(N, K):
+    """Past 64 tokens a narrow matrix takes 16-row workgroups up to about as many as the CUs (by the layout and the
+    K slice) and 64-row ones from there: on both sides of that line, and with a partial 64-row tile, every row's
+    bits are those of a batch of 16, packed and not."""
+    from jitengine_amd.quant import random_quantized
+
+    q = random_quantized((N, K), N + K, device=DEV)
+    rows = 1400 if N <= 400 else 300
+    x = bf16_tensor(normal_bf16((rows, K), seed=N), DEV)
+    for lin in (q, ops.prepack(q)):
+        seg = False if lin is not q else None
+        one = torch.cat([ops.qmm(x[t:t + 16].contiguous(), lin, seg=seg) for t in range(0, rows, 16)])
+        for T in (65, 81, 100, 130, 161, 257, rows):
+            assert torch.equal(ops.qmm(x[:T].contiguous(), lin, seg=seg), one[:T]), (T, lin is q)
+
+
 @pytest.mark.parametrize("lens,H,Hkv", [
     ([1], 32, 4), ([1537], 32, 4), ([4096], 32, 4), ([1921, 383, 384, 385], 32, 4), ([1952, 2304, 2305], 32, 4),
     ([3000, 70], 64, 4), ([3071, 5], 8, 8), ([2000, 17], 16, 1), ([40000], 32, 4), ([200003], 16, 1)])
