@@ -175,10 +175,10 @@ def test_moe_block_prefill_switch():
     assert_close_bf16(u16(y), want, what="prefill experts")
 
 
-@pytest.mark.parametrize("T,N,K", [(512, 2048, 4096), (2108, 2048, 4096), (1200, 5120, 2048), (2108, 5120, 2048)])
+@pytest.mark.parametrize("T,N,K", [(512, 2048, 4096), (2108, 2048, 4096), (1200, 5120, 2048), (2108, 5120, 2048),
+                                   (300, 5120, 2048), (512, 5120, 2048), (1024, 5120, 2048)])
 def test_dense_segment_gemm_repeats_bit_for_bit(T, N, K):
-    """A dense batch sized to each token chunk the launch picks on 256 CUs (4, 6, 8 and 10 tiles: the
-    o_proj of a 512-row prompt chunk and of config 3's 2,108 rows, and qkv at 1,200 and 2,108 rows)
+    """A dense batch sized to each token chunk the launch picks on 256 CUs (2, 6, 10, 6, 3, 4 and 8 tiles)
     gives the same bits on every call.
     A regression test: the kernel's waits for its direct global->LDS loads count the loads issued
     after the awaited ones, and with a count fixed for 10-tile chunks the shorter chunks read a
@@ -197,13 +197,16 @@ def test_segment_gemm_chunk_lengths(mean, K):
     6 and 10 token tiles here) at its edges: segments of 0, 1, a tile, a tile + 1, a chunk, a chunk + 1
     and three chunks, over 1, 2, 5 and 16 K steps (fewer than the loads run ahead, and more).  The
     output of gate||up and of down equals the oracle's bf16-weight restatement as in the tests above."""
-    E, N = 12, 256
+    E, N = 24 if mean == 4 else 12, 256  # (the fixed segments alone are 114 pairs)
     tiles = {4: 1, 10: 2, 20: 3, 40: 4, 60: 6, 120: 10}[mean]
-    cnt = np.array([0, 1, 16, 17, 16 * tiles, 16 * tiles + 1, 48 * tiles - 1, 0, 0, 0, 0, 0])
+    cnt = np.zeros(E, np.int64)
+    cnt[:7] = [0, 1, 16, 17, 16 * tiles, 16 * tiles + 1, 48 * tiles - 1]
     rest = mean * E - int(cnt.sum())
     if rest > 0:
         cnt[7:11] = [rest // 4, rest // 4, rest // 4, rest - 3 * (rest // 4)]
     P = int(cnt.sum())
+    need = P / E + 2.5 * (P / E) ** 0.5
+    assert {1: 0, 2: 16, 3: 32, 4: 48, 6: 64, 10: 96}[tiles] < need <= {10: P}.get(tiles, 16 * tiles)  # (the rule's interval)
     inds = np.random.default_rng(mean + K).permutation(np.repeat(np.arange(E), cnt)).astype(np.int32).reshape(P, 1)
     gu_h, dn_h = _stack(E, N, K, mean + K), _stack(E, N, K, mean + K + 1)
     x = normal_bf16((P, K), seed=mean)
@@ -221,9 +224,9 @@ def test_segment_gemm_chunk_lengths(mean, K):
 
 
 @pytest.mark.parametrize("T,N,K", [(1, 256, 128), (40, 256, 256), (192, 5120, 2048), (300, 5120, 2048), (512, 5120, 2048),
-                                   (1024, 5120, 2048), (4000, 2048, 384)])
+                                   (1024, 5120, 2048), (4000, 2048, 384), (2108, 2048, 384), (1200, 5120, 384)])
 def test_dense_segment_gemm_shapes(T, N, K):
-    """The dense launch's chunk lengths (2, 3, 4, 6, 8 and 10 tiles by estimated time) against float64
+    """The dense launch's chunk lengths (by estimated time on 256 CUs 2, 2, 2, 3, 4, 8, 8, 6 and 10 tiles) against float64
     sums over the same bf16 weights: one bf16 rounding, and fp32 accumulation of K products."""
     from jitengine_amd.quant import dequantize4
 
