@@ -1042,7 +1042,7 @@ OP_KERNELS = {  # the kernels one op launches (rocprofv3 kernel names contain th
     "down": ["qmm_kernel<4, 4, false, true"],
     "gate_up_swiglu_seg": ["seg_kernel<true, false,"],  # (any token-chunk length)
     "down_seg": ["seg_kernel<false, false,"],
-    "qkv_proj_seg": ["seg_kernel<false, true, 10>"],  # (config 3's 2,108 rows: the 10-tile chunk; o_proj takes 5)
+    "qkv_proj_seg": ["seg_kernel<false, true,"],  # (at config 3's 2,108 rows o_proj is the same kernel: both counted)
     "prefill_attention": ["prefill_attn_kernel", "prefill_merge_kernel"],
 }
 
