@@ -2,18 +2,18 @@
 
 python bench.py [--gpus 1] [--steps K] [--warmup W] [--config 2] [--layers 48] [--no-graph] [--no-bs1]
 
-config 2 (the default; BASELINE.json configs[2], the workload the metric is quoted on): ragged
+config 2 (the default; the workload the metric is quoted on): ragged
 continuous-batch decode of 32 sequences over the paged KV pool through 48 layers of the 4-bit
 Qwen3-MoE-style block; a step decodes one token per sequence (value = tokens/s).  The step is
 captured once as a HIP graph and replayed (--no-graph times eager launches).  The metric's bs=1
 half -- config 4 on the same model -- is measured after it and reported in the line's "bs1" object
 (--no-bs1 leaves it out).
-config 4 (BASELINE.json configs[4]): single-sequence decode at 262,144 KV tokens through the 48
+config 4: single-sequence decode at 262,144 KV tokens through the 48
 layers (value = tokens/s).
-config 3 (BASELINE.json configs[3]): one mixed chunked-prefill + decode step of one block -- 4 x 512
+config 3: one mixed chunked-prefill + decode step of one block -- 4 x 512
 prefill tokens (causal attention over their contexts) + 60 decode rows, the MoE on the segment GEMM
 (value = rows/s; MFMA roofline of the dominant kernel).
-config 1 (BASELINE.json configs[1]): one standalone quantized-MoE call -- 64 tokens, top-8 of 128
+config 1: one standalone quantized-MoE call -- 64 tokens, top-8 of 128
 experts drawn from softmax of N(0,1) logits, gate/up [768 x 2048] and down [2048 x 768] per expert
 (4-bit g64, N(0, 0.02) weights); a step = packing + gate||up/SwiGLU + down + combine.
 Inputs are resident in HBM before timing; K steps are timed with HIP events after W warmups.
@@ -56,7 +56,7 @@ HOT_OPS = ("paged_attention", "gate_up_swiglu", "down")  # the ops that move the
 
 
 def hot_path_hbm(step_us: dict, alg_bytes: int) -> dict:
-    """A kernel-level diagnostic, not the north-star measure: a decode step's quantized-expert and
+    """A kernel-level diagnostic, not the step's measure: a decode step's quantized-expert and
     KV-pool bytes (alg_bytes) over the summed live time of only the ops that move them (step_us:
     microseconds per step by op), leaving out the rest of the step."""
     us = sum(step_us[n] for n in HOT_OPS if n in step_us)
@@ -65,11 +65,11 @@ def hot_path_hbm(step_us: dict, alg_bytes: int) -> dict:
             "alg_bytes": alg_bytes, "us_per_step": us, "GB_s": gbs, "frac": gbs / HBM_PEAK_GBS if gbs else None}
 
 
-NORTH_STAR_FRAC = 0.6  # BASELINE.json: >= 60% of HBM peak on the combined expert + KV-pool traffic
+NORTH_STAR_FRAC = 0.6  # >= 60% of HBM peak on the combined expert + KV-pool traffic
 
 
 def north_star(alg_bytes: int, ms_per_step: float, rows: int) -> dict:
-    """The north-star measure as BASELINE defines it: the step's quantized-expert and KV-pool bytes
+    """The step's quantized-expert and KV-pool bytes
     over the whole step's time (every launch of the step included), as a fraction of the 8 TB/s peak,
     and the tokens/s a step meeting the 60% target would give on these bytes."""
     gbs = alg_bytes / (ms_per_step * 1e-3) / 1e9
@@ -223,7 +223,7 @@ def bench_config1(steps: int, warmup: int, dev: str) -> dict:
 
 
 def bench_config3(steps: int, warmup: int, dev: str) -> dict:
-    """one mixed chunked-prefill + decode step of one decoder block -- 4
+    """Config 3: one mixed chunked-prefill + decode step of one decoder block -- 4
     prefill chunks of 512 tokens after prior contexts U{0..8192} plus 60 decode sequences with
     lengths log-uniform in [256, 16384], 2,108 rows in all (DecoderLayer.mixed: qkv, norms and
     RoPE with the KV append of every row, causal prefill attention and split-K decode attention,
@@ -382,8 +382,8 @@ def bench_config3(steps: int, warmup: int, dev: str) -> dict:
     }
 
 
-CONFIG4_KEYS = 262144  # one sequence decoding at 262,144 KV tokens
-CONFIG0_KEYS = 4096    # one block, batch 1, 4,096 context tokens in one page run
+CONFIG4_KEYS = 262144  # config 4: one sequence decoding at 262,144 KV tokens
+CONFIG0_KEYS = 4096    # config 0: one block, batch 1, 4,096 context tokens in one page run
 
 
 def decode_model(cfg, seed: int, dev: str):
@@ -408,9 +408,9 @@ def bench_decode(config: int, steps: int, warmup: int, dev: str, graph: bool, n_
     """A decode step of the 4-bit Qwen3-MoE-style model over the paged KV pool (16-token pages in a
     random permutation of the pool), one token per sequence through every layer (each row writes
     position L_b and attends to L_b + 1 keys).
-    config 2 (BASELINE configs[2]): 32 sequences with lengths log-uniform in [128, 32768], 48 layers
+    config 2: 32 sequences with lengths log-uniform in [128, 32768], 48 layers
     with independent seeded weights.
-    config 4 (BASELINE configs[4]): one sequence at 262,144 KV tokens (the step's own token is the
+    config 4: one sequence at 262,144 KV tokens (the step's own token is the
     262,144th key), 48 layers; `model` may pass in config 2's weights, which are as random as its own."""
     import oracle
     from jitengine_amd import ops

@@ -278,7 +278,7 @@ int jit_qmm_packed_combine_rmsnorm(const uint16_t *r, const int32_t *inv, const 
 
 /* The attention block between the qkv projection and attention
  * (Qwen3_5MoeAttention.step, Q36/model/attention.py:99-119, without the output
- * gate, which the BASELINE geometry does not have): qkv [B, (H + 2 Hkv) * 128]
+ * gate, which the Qwen3-MoE-style geometry does not have): qkv [B, (H + 2 Hkv) * 128]
  * (q heads, then k heads, then v heads); per head RMSNorm with q_norm_w /
  * k_norm_w [128]; RoPE with traditional = False on q and k (pairs (i, i + 64),
  * angle fp32(pos[b]) * inv_freq[i], inv_freq [64] fp32 = base^(-2i/128));

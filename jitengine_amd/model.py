@@ -1,4 +1,4 @@
-"""The decode step of the BASELINE geometry on the HIP kernels: decoder layers and decode_step.
+"""The decode step of the Qwen3-MoE-style geometry on the HIP kernels: decoder layers and decode_step.
 
 Mirrors the reference's batched decode call chain (Q36/model/model.py:504-517 `decode_step` ->
 `Qwen3_5MoeDecoderLayer.step` :77-80): input RMSNorm -> fused qkv projection -> q/k RMSNorm +

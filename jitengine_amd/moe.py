@@ -4,7 +4,7 @@ Mirrors the call sites of Qwen3_5MoeSparseMoeBlock (Q36/model/moe.py): the route
 (`_route_logits`, :296-302), the fused router top-k (`_route_top_k`, :304-315), token-to-expert
 packing (`_sort_pairs`, :151-159), gate||up + SwiGLU and down over the packed pairs (:191-193), and
 the slot-order weighted combine (:286) with the residual (`with_residual`, :119-123).  The
-BASELINE geometry has no shared expert, so there is no shared branch.
+Qwen3-MoE-style geometry has no shared expert, so there is no shared branch.
 """
 
 from __future__ import annotations

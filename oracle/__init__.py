@@ -325,7 +325,7 @@ def qk_norm_rope_append(qkv, H: int, Hkv: int, qn, kn, eps: float, inv_freq, pos
 
 
 def decoder_layer(x, layer: dict, pool, page_table, pos, cfg: dict, routing=None) -> dict:
-    """One decoder layer of the BASELINE geometry for rows x [B, D] (the reference's layer step,
+    """One decoder layer of the Qwen3-MoE-style geometry for rows x [B, D] (the reference's layer step,
     Q36/model/model.py:77-80 with Qwen3_5MoeAttention.step and the MoE block): input RMSNorm ->
     qkv -> q/k norm + RoPE + KV append -> attention over pos + 1 keys -> o_proj -> residual ->
     post-attention RMSNorm -> router -> experts -> combine + residual.  `layer` holds numpy

@@ -83,8 +83,8 @@ def bf16_ulp(v: np.ndarray) -> np.ndarray:
 
 def assert_close_bf16(got_u16: np.ndarray, want_u16: np.ndarray, max_abs: float = 2e-2, min_cos: float = 0.9995,
                       what: str = "", ulps: float = 2.0) -> dict:
-    """The north-star float tolerance on bf16 outputs: every element within max(2e-2, `ulps` bf16
-    ulps of the expected value) -- the absolute 2e-2 of the north star, widened to two ulps where
+    """The float tolerance on bf16 outputs: every element within max(2e-2, `ulps` bf16
+    ulps of the expected value) -- the absolute 2e-2 of the tolerance, widened to two ulps where
     values exceed |4| and one ulp alone is larger than 2e-2 -- and cosine >= 0.9995."""
     g = bf16_to_f32(got_u16).astype(np.float64)
     w = bf16_to_f32(want_u16).astype(np.float64)

@@ -1,7 +1,7 @@
 """The attention parity bar (tests.helpers.assert_attention_parity) can fail: mistakes a paged
 decode-attention kernel could make are planted in the CPU oracle's inputs -- one page id pointing
 at another sequence's page, a page dropped (its slot repeating the previous page), the last key
-left out -- and the bar must reject each result, at short and at BASELINE's 262,144-key context.
+left out -- and the bar must reject each result, at short and at the 262,144-key context.
 Outputs an fp32-accurate kernel would give pass it; one that rounds the probabilities to bf16
 before P.V does not (no CPU-only test runs a kernel: the planted results come from the oracle)."""
 
@@ -71,7 +71,7 @@ def test_accurate_results_pass_the_bar():
 
 def test_bf16_probabilities_fail_the_bar():
     """One bf16 P per key (each probability rounded by up to 2^-9) moves ~40% of the outputs by an
-    ulp: the floor rejects it where the north star's absolute 2e-2 would not."""
+    ulp: the floor rejects it where the tolerance's absolute 2e-2 would not."""
     lens = [5000, 40000]
     q, pool, table = _case(lens, seed=4)
     cr, exact, stock = _reference(q, pool, table, lens)
@@ -104,9 +104,9 @@ def test_planted_mistakes_fail_the_bar(b):
 
 
 def test_planted_mistakes_fail_the_bar_at_262144_keys():
-    """BASELINE config 4's context: one 16-key page of 262,144 moves the outputs by about an ulp,
+    """Config 4's context: one 16-key page of 262,144 moves the outputs by about an ulp,
     under the 2e-2 absolute tolerance and the cosine, but not under this bar.  (8 q heads over one
-    kv head -- BASELINE's GQA group -- keep the CPU pool at 134 MB.)"""
+    kv head -- the model's GQA group -- keep the CPU pool at 134 MB.)"""
     lens = [262144, 1000]
     q, pool, table = _case(lens, seed=6, H=8, Hkv=1)
     cr, exact, stock = _reference(q, pool, table, lens)
@@ -114,6 +114,6 @@ def test_planted_mistakes_fail_the_bar_at_262144_keys():
     for name, t, ln in _mutations(table, lens, 0):
         bad = oracle.paged_decode_attn(q, pool, t, ln, SCALE)
         g, w = bf16_to_f32(bad[0]).astype(np.float64), exact[0]
-        assert np.abs(g - w).max() < 2e-2  # the north star's absolute bound misses it
+        assert np.abs(g - w).max() < 2e-2  # the tolerance's absolute bound misses it
         with pytest.raises(AssertionError, match="sequence 0"):
             assert_attention_parity(bad, exact, stock, what=name)

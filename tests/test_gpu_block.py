@@ -101,7 +101,7 @@ def _stages_on_gpu_inputs(cfg, lens, table, pool_after, w, dbg, what):
       criterion, one ulp + 2^-14 of the row, >= 98% correctly rounded) on the GPU's q over the pool
       the GPU's append left, through the layer's plan, page table and pos + 1 lengths;
     * router logits: the reference's criterion for quantized projections and >= 95% bit-equal;
-    * gate||up + SwiGLU (h) and down (r): the north-star tolerance (h at 4 ulps, as its SwiGLU
+    * gate||up + SwiGLU (h) and down (r): the float tolerance (h at 4 ulps, as its SwiGLU
       may flip with one ulp of g or u) and >= 95% bit-equal, under the GPU's routing;
     * the closing combine: y = bf16(h + combine(r, scores)) bit for bit."""
     lens1 = np.asarray(lens, np.int64) + 1
@@ -158,7 +158,7 @@ def _layer_vs_oracle(cfg, lens, table, pool, x, w, what, max_flips):
 
 
 def test_decoder_layer_config0():
-    """BASELINE configs[0] on the GPU: one Qwen3-MoE-style block (128 experts, top-8) at batch 1,
+    """One Qwen3-MoE-style block (128 experts, top-8) at batch 1,
     decoding at position 4,096 over a 4,096-token context in pages 0..255 in order (the new key
     goes to page 256), against the oracle's block."""
     cfg = MoEConfig(layers=1)
@@ -172,7 +172,7 @@ def test_decoder_layer_config0():
 
 
 def test_decoder_layer_config2_rows():
-    """BASELINE configs[2]'s step on one layer at full geometry: the bench's 32 ragged rows (lengths
+    """The ragged decode step (config 2 of bench.py) on one layer at full geometry: the bench's 32 ragged rows (lengths
     log-uniform in [128, 32768], pages a random permutation) through a 128-expert block -- the
     decode expert GEMVs in their real regime (~2 rows per distinct expert) -- against the oracle."""
     cfg = MoEConfig(layers=1)

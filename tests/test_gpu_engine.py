@@ -2,7 +2,7 @@
 engine and the checkpoint loader on MI355X.
 
 Kernel parity: embedding and argmax bit-exact against the oracle, page copies bit-exact, logits
-within the north-star tolerance.  Engine: generation is a function of each request alone --
+within the float tolerance.  Engine: generation is a function of each request alone --
 bit-identical tokens whether a request runs alone or batched with staggered others, whether its
 prompt's KV is computed or restored from the prefix store (shared pages, one copied), and when a
 small pool defers admission.  The engine tests keep every step under 64 rows, where every op takes

@@ -1,7 +1,7 @@
 """HIP path vs the CPU oracle on the same seeded inputs (MI355X only).
 
 Integer outputs (expert ids, packing tables, KV bytes) must be bit-exact; bf16 outputs must meet
-the north-star tolerance (max-abs <= 2e-2, cosine >= 0.9995) and, for the quantized projections,
+the float tolerance (max-abs <= 2e-2, cosine >= 0.9995) and, for the quantized projections,
 the reference's own criterion (FN/kernels/selfcheck.py:313-331): the kernel's largest error against
 the float64 result is at most 8x that of the reference's fp32 arithmetic (restated in
 oracle.qmv_mlx_f32, rounded to bf16 as the reference returns it) plus 4 fp32 ulps of the scale."""
@@ -420,7 +420,7 @@ def _attn_bar(got, q, pool, table, lens, what, scale=128 ** -0.5):
     """The attention bar (tests.helpers.assert_attention_parity): the reference's 8x-stock criterion
     against oracle.sdpa_mlx_f32, every element within one ulp + 2^-14 of its row of the float64
     result, and per sequence >= 98% of the outputs equal to the correctly rounded result; plus the
-    north star's max-abs / cosine tolerance."""
+    max-abs / cosine tolerance."""
     want, exact = oracle.paged_decode_attn(q, pool, table, lens, scale, exact=True)
     stock, _ = oracle.sdpa_mlx_f32(q, pool, table, lens, scale)
     st = assert_attention_parity(got, exact, stock, what=what)
@@ -437,7 +437,7 @@ def test_paged_attention_parity():
 
 @pytest.mark.parametrize("L", [262144, 200003])
 def test_paged_attention_long_context(L):
-    """BASELINE config 4's shape: one sequence of 262,144 keys in permuted 16-token pages
+    """Config 4's shape: one sequence of 262,144 keys in permuted 16-token pages
     (128 chunks of 2048 keys split over 4 waves per kv head, merged in chunk order); and a
     length just past the 1536-key rule (121 chunks of 1664, the last one partial)."""
     q, pool, table = _pool([L], seed=23)

@@ -2,11 +2,11 @@
 
 The oracle states the causal mask as what it is: chunk token t at position ctx + t attends the
 first ctx + t + 1 keys of its sequence, i.e. the float64 decode attention of that token over
-ctx + t + 1 keys (oracle.paged_prefill_attn).  The bar is the north-star float tolerance; the
+ctx + t + 1 keys (oracle.paged_prefill_attn).  The bar is the float tolerance; the
 invariants below are bit-exact.  The float bar is tests.helpers.assert_attention_parity without its
 stock criterion (MLX's full-attention kernel is not restated): every element within one bf16 ulp +
 2^-14 of its row of the float64 result and >= 98% of each row's outputs correctly rounded, which a
-dropped or misplaced page fails (tests/test_attention_bar.py); plus the north star's tolerance."""
+dropped or misplaced page fails (tests/test_attention_bar.py); plus the float tolerance."""
 
 from __future__ import annotations
 
@@ -146,7 +146,7 @@ def test_prefill_page_permutation_and_stale_slots():
 
 
 def test_prefill_config3_chunks():
-    """BASELINE config 3's prefill half: 4 chunks of 512 tokens after contexts up to 8,192."""
+    """Config 3's prefill half: 4 chunks of 512 tokens after contexts up to 8,192."""
     rng = np.random.default_rng(0x4A450030)
     ctx = rng.integers(0, 8193, 4)
     chunks = [(i, int(c), 512) for i, c in enumerate(ctx)]

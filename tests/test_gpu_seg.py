@@ -2,7 +2,7 @@
 
 Its arithmetic is the reference's prefill tile GEMM (Q36/kernels/gather_qmm_prefill.py): weights
 dequantized to bf16, bf16 products accumulated in fp32.  The oracle restates it with float64 sums
-over the same bf16 weights (oracle.moe_gate_up / moe_down with bf16w), so the bar is the north-star
+over the same bf16 weights (oracle.moe_gate_up / moe_down with bf16w), so the bar is the
 float tolerance; the integer tables are shared with the decode path (jit_moe_pack)."""
 
 from __future__ import annotations
@@ -76,7 +76,7 @@ def _pairs_of(inds_flat, order, pair_row, sel):
 
 
 def test_segment_gemm_config3_geometry():
-    """BASELINE configs[3]'s MoE half at full size: 2,108 rows (four 512-token prefill chunks and 60
+    """The mixed step's MoE half (config 3 of bench.py) at full size: 2,108 rows (four 512-token prefill chunks and 60
     decode rows) routed top-8 over 128 experts -- 16,864 pairs, ~132 per expert, 160-row token
     chunks, every expert's column blocks on the XCD of its expert -- through the segment GEMMs,
     against the oracle's bf16-weight restatement on every pair of 16 experts (the largest segment
