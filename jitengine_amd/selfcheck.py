@@ -6,7 +6,7 @@ Q36/engine/engine.py:355-375).  This build has no other compute path to fall bac
 that disagrees raises SelfCheckError instead.  Each case is tiny and compares the HIP kernel with a
 plain torch fp32 computation of the same op on the same device (integer outputs exactly, bf16
 outputs within the float tolerance: max-abs <= 2e-2 or 2 bf16 ulps, cosine >= 0.9995).  The
-torch computations are the checker only; nothing here feeds a result back into a step.
+torch computations only check; nothing here feeds a result back into a step.
 
 Opt in with Engine(..., selfcheck=True) or JITENGINE_SELFCHECK=1 in the environment.
 """

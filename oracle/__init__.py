@@ -1,7 +1,7 @@
 """CPU oracle for the ragged MoE decode step -- TEST INFRASTRUCTURE ONLY.
 
 Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg import this package, and
-only as the checker; the product path (jitengine_amd) never imports it.  The arithmetic lives in
+only to check results; the product path (jitengine_amd) never imports it.  The arithmetic lives in
 jit_oracle.c (a C restatement of the reference's algorithm, each function citing the reference
 lines it follows); this module wraps it with numpy.  bf16 arrays are numpy uint16 bit patterns.
 
